@@ -70,7 +70,35 @@ LRH_DN inline float unkey(uint32_t k) {
 LRH_DN inline float expScale(uint32_t e) { return fromBits(e << 23); }
 LRH_DN inline float decodeQ(float org, uint32_t q, float s) { return org + (float)q * s; }
 
-// outward-rounded 8-bit child bounds, the rule of the host builder's quantize
+// exponent byte of one axis of a quantized node over [o, hi]: the smallest
+// power of two whose 255 steps from o reach hi
+LRH_DN inline int axisExp(float o, float hi) {
+	const float ext = hi - o;
+	int e2 = -126;
+	if (ext > 0.f) frexpf(ext / 255.f, &e2);
+	int e = e2 + 127;
+	if (e < 1) e = 1;
+	while (e < 254 && decodeQ(o, 255, expScale((uint32_t)e)) < hi) ++e;
+	return e;
+}
+
+// a child's bounds on one axis as steps of s from o, rounded outward (the
+// rule of the host builder's quantize)
+LRH_DN inline uint8_t axisLo(float lo, float o, float s) {
+	long q = (long)floorf((lo - o) / s);
+	if (q < 0) q = 0;
+	if (q > 255) q = 255;
+	while (q > 0 && decodeQ(o, (uint32_t)q, s) > lo) --q;
+	return (uint8_t)q;
+}
+LRH_DN inline uint8_t axisHi(float hi, float o, float s) {
+	long q = (long)ceilf((hi - o) / s);
+	if (q < 0) q = 0;
+	if (q > 255) q = 255;
+	while (q < 255 && decodeQ(o, (uint32_t)q, s) < hi) ++q;
+	return (uint8_t)q;
+}
+
 // W-wide quantized node (lrh_node4q, lrh_node8q): the host builder's
 // outward rounding
 template <int W, class Node>
@@ -92,31 +120,13 @@ LRH_DN inline void quantizeNodeW(const GBox *cb, int n, const uint32_t *child, N
 	for (int k = 0; k < 3; ++k) {
 		const float o = pb.lo[k];
 		q.org[k] = o;
-		const float ext = pb.hi[k] - o;
-		int e2 = -126;
-		if (ext > 0.f) frexpf(ext / 255.f, &e2);
-		int e = e2 + 127;
-		if (e < 1) e = 1;
-		while (e < 254 && decodeQ(o, 255, expScale((uint32_t)e)) < pb.hi[k]) ++e;
+		const int e = axisExp(o, pb.hi[k]);
 		const float s = expScale((uint32_t)e);
 		*ex[k] = (uint8_t)e;
 		for (int c = 0; c < W; ++c) {
-			if (c >= n) {
-				qlo[k][c] = 255;  // empty slot: inverted box
-				qhi[k][c] = 0;
-				continue;
-			}
-			const float lo = cb[c].lo[k], hi = cb[c].hi[k];
-			long ql = (long)floorf((lo - o) / s);
-			if (ql < 0) ql = 0;
-			if (ql > 255) ql = 255;
-			while (ql > 0 && decodeQ(o, (uint32_t)ql, s) > lo) --ql;
-			long qh = (long)ceilf((hi - o) / s);
-			if (qh < 0) qh = 0;
-			if (qh > 255) qh = 255;
-			while (qh < 255 && decodeQ(o, (uint32_t)qh, s) < hi) ++qh;
-			qlo[k][c] = (uint8_t)ql;
-			qhi[k][c] = (uint8_t)qh;
+			// empty slot: inverted box
+			qlo[k][c] = c < n ? axisLo(cb[c].lo[k], o, s) : 255;
+			qhi[k][c] = c < n ? axisHi(cb[c].hi[k], o, s) : 0;
 		}
 	}
 	q.nchild = (uint8_t)n;
@@ -148,6 +158,69 @@ LRH_DN inline void floatNode(const GBox *cb, int n, const uint32_t child[4], lrh
 	}
 	*out = f;
 }
+
+#if defined(__HIPCC__)
+// The same node written by W neighbouring lanes of a wave, lane c (0..W-1)
+// with child c: one lane per child instead of one thread per node, whose
+// children's roundings (a division and a few compares each, six per child)
+// would run one after another.  All W lanes call it together; lane c < n has
+// the child's box and reference, the others pass any box and
+// LRH_CHILD_EMPTY.  Returns the union of the boxes to all of them: min and
+// max are exact, so its order does not show in the bytes, and a NaN bound (a
+// triangle of NaN vertices, which no ray meets) is left out of it.
+template <int W, class Node>
+__device__ inline GBox quantizeNodeLanes(const GBox &b, int c, int n, uint32_t child, Node *out) {
+	GBox u = b;
+	for (int k = 0; k < 3; ++k) {
+		if (c >= n) {
+			u.lo[k] = INFINITY;
+			u.hi[k] = -INFINITY;
+		}
+		for (int o = W / 2; o > 0; o >>= 1) {
+			u.lo[k] = fminf(__shfl_xor(u.lo[k], o), u.lo[k]);
+			u.hi[k] = fmaxf(__shfl_xor(u.hi[k], o), u.hi[k]);
+		}
+	}
+	uint8_t *const qlo[3] = {out->qlo_x, out->qlo_y, out->qlo_z};
+	uint8_t *const qhi[3] = {out->qhi_x, out->qhi_y, out->qhi_z};
+	for (int k = 0; k < 3; ++k) {
+		const float o = u.lo[k];
+		const int e = axisExp(o, u.hi[k]);
+		const float s = expScale((uint32_t)e);
+		qlo[k][c] = c < n ? axisLo(b.lo[k], o, s) : 255;
+		qhi[k][c] = c < n ? axisHi(b.hi[k], o, s) : 0;
+		if (c == 0) {
+			out->org[k] = o;
+			(&out->ex)[k] = (uint8_t)e;
+		}
+	}
+	out->child[c] = child;
+	constexpr int kPads = (int)(sizeof(out->pad) / 4);
+	if (c < kPads) out->pad[c] = 0;
+	if (c == 0) out->nchild = (uint8_t)n;
+	return u;
+}
+
+// the fp32 node (lrh_node4f) by four lanes, likewise
+__device__ inline GBox floatNodeLanes(const GBox &b, int c, int n, uint32_t child, lrh_node4f *out) {
+	GBox u = b;
+	for (int k = 0; k < 3; ++k)
+		if (c >= n) {
+			u.lo[k] = INFINITY;
+			u.hi[k] = -INFINITY;
+		}
+	out->lo_x[c] = u.lo[0]; out->lo_y[c] = u.lo[1]; out->lo_z[c] = u.lo[2];
+	out->hi_x[c] = u.hi[0]; out->hi_y[c] = u.hi[1]; out->hi_z[c] = u.hi[2];
+	out->child[c] = child;
+	out->pad[c] = 0;
+	for (int k = 0; k < 3; ++k)
+		for (int o = 2; o > 0; o >>= 1) {
+			u.lo[k] = fminf(__shfl_xor(u.lo[k], o), u.lo[k]);
+			u.hi[k] = fmaxf(__shfl_xor(u.hi[k], o), u.hi[k]);
+		}
+	return u;
+}
+#endif
 
 }  // namespace lrhdev
 

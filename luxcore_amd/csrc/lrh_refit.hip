@@ -8,8 +8,9 @@
  *   1. motion objects' world boxes: MotionSystem::Bound(box, true)
  *      (src/luxrays/core/geometry/motionsystem.cpp:75-87, 356-365), i.e. the
  *      union over every segment of 1,025 samples of Sample(t).Inverse() * box,
- *      one thread per (object, segment, sample), combined with exact atomic
- *      min/max on ordered float keys, then expanded by MachineEpsilon::E
+ *      one thread per (object, segment, sample), combined with exact min/max
+ *      on ordered float keys (across the wave, then by atomics), then
+ *      expanded by MachineEpsilon::E
  *      (mbvhaccel.cpp:192-193); rounded as the host computes them (this file
  *      builds with -ffp-contract=off and correctly rounded division);
  *   2. the root nodes bottom-up, one launch per level, deepest first: each
@@ -20,6 +21,8 @@
  * Instance and plain objects' boxes are cheap and come from the host.
  */
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "lrh_devnode.h"
 #include "lrh_layout.h"
@@ -122,37 +125,75 @@ __global__ void k_clear(uint32_t *p) {
 	if (threadIdx.x == 0 && blockIdx.x == 0) *p = 0u;
 }
 
-// one thread per (motion object, segment, sample)
-__global__ void k_motionBounds(const LrhRefitMotion *mo, uint32_t nMo, const uint32_t *sampleBase,
+// One thread per (motion object, segment, sample).  The samples of an object
+// are consecutive threads, so a wave holds one object's (two, where it
+// straddles) and reduces the boxes by lane exchanges before it goes to
+// memory: six atomics per wave and object instead of six per sample, all of
+// an object's on the same six words (1,000 objects, 200 moving: 1.85 ms ->
+// 0.07 ms, now the matrix inverses).  A segment whose samples are all the same
+// matrix (not active, or of no duration) is evaluated at its first sample
+// only.
+__global__ __launch_bounds__(256) void k_motionBounds(const LrhRefitMotion *mo, uint32_t nMo, const uint32_t *sampleBase,
 		const lrh_motion *motions, const lrh_motion_seg *segs, const float *meshBoxes, uint32_t *keys,
 		uint32_t *error) {
 	const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
-	if (tid >= sampleBase[nMo]) return;
-	uint32_t lo = 0, hi = nMo;  // motion object m with sampleBase[m] <= tid < sampleBase[m + 1]
-	while (hi - lo > 1) {
-		const uint32_t mid = (lo + hi) >> 1;
-		if (sampleBase[mid] <= tid) lo = mid; else hi = mid;
+	uint32_t m = nMo;  // no object: past the last sample, or a repeated one
+	uint32_t mn[3] = {0xffffffffu, 0xffffffffu, 0xffffffffu}, mx[3] = {0u, 0u, 0u};
+	if (tid < sampleBase[nMo]) {
+		uint32_t lo = 0, hi = nMo;  // motion object with sampleBase[lo] <= tid < sampleBase[lo + 1]
+		while (hi - lo > 1) {
+			const uint32_t mid = (lo + hi) >> 1;
+			if (sampleBase[mid] <= tid) lo = mid; else hi = mid;
+		}
+		const uint32_t local = tid - sampleBase[lo];
+		const uint32_t seg = local / kSamples, i = local % kSamples;
+		const lrh_motion &md = motions[mo[lo].motion];
+		const lrh_motion_seg &g = segs[md.firstSeg + seg];
+		const bool constant = !(g.flags & LRH_MF_ACTIVE) || g.startTime == g.endTime;
+		if (!constant || i == 0) {
+			m = lo;
+			const float t = lrhLerp((float)i / 1024.f, g.startTime, g.endTime);
+			float M[16], inv[16];
+			lrhSegSample(g, t, M);
+			if (!invert4d(M, inv)) {
+				atomicOr(error, 1u);
+				m = nMo;
+			} else {
+				const float *mb = meshBoxes + 6 * (size_t)mo[lo].mesh;
+				GBox ib;
+				for (int k = 0; k < 3; ++k) { ib.lo[k] = mb[k]; ib.hi[k] = mb[3 + k]; }
+				const GBox b = transformBoxD(inv, ib);
+				for (int k = 0; k < 3; ++k) {
+					mn[k] = fkey(b.lo[k]);
+					mx[k] = fkey(b.hi[k]);
+				}
+			}
+		}
 	}
-	const uint32_t m = lo;
-	const uint32_t local = tid - sampleBase[m];
-	const uint32_t seg = local / kSamples, i = local % kSamples;
-	const lrh_motion &md = motions[mo[m].motion];
-	const lrh_motion_seg &g = segs[md.firstSeg + seg];
-	const float t = lrhLerp((float)i / 1024.f, g.startTime, g.endTime);
-	float M[16], inv[16];
-	lrhSegSample(g, t, M);
-	if (!invert4d(M, inv)) {
-		atomicOr(error, 1u);
-		return;
-	}
-	const float *mb = meshBoxes + 6 * (size_t)mo[m].mesh;
-	GBox ib;
-	for (int k = 0; k < 3; ++k) { ib.lo[k] = mb[k]; ib.hi[k] = mb[3 + k]; }
-	const GBox b = transformBoxD(inv, ib);
-	uint32_t *kk = keys + 6 * (size_t)m;
-	for (int k = 0; k < 3; ++k) {
-		atomicMin(&kk[k], fkey(b.lo[k]));
-		atomicMax(&kk[3 + k], fkey(b.hi[k]));
+	// per object of the wave: the boxes of its lanes reduced, six lanes write
+	uint64_t todo = __ballot(m < nMo);
+	while (todo) {
+		const uint32_t obj = (uint32_t)__builtin_amdgcn_readlane((int)m, __ffsll((long long)todo) - 1);
+		const bool mine = m == obj;
+		todo &= ~__ballot(mine);
+		uint32_t a[6];
+		for (int k = 0; k < 3; ++k) {
+			a[k] = mine ? mn[k] : 0xffffffffu;
+			a[3 + k] = mine ? mx[k] : 0u;
+		}
+		for (int o = 32; o > 0; o >>= 1)
+			for (int k = 0; k < 3; ++k) {
+				const uint32_t x = (uint32_t)__shfl_xor((int)a[k], o), y = (uint32_t)__shfl_xor((int)a[3 + k], o);
+				a[k] = x < a[k] ? x : a[k];
+				a[3 + k] = y > a[3 + k] ? y : a[3 + k];
+			}
+		if (__lane_id() == 0) {
+			uint32_t *kk = keys + 6 * (size_t)obj;
+			for (int k = 0; k < 3; ++k) {
+				atomicMin(&kk[k], a[k]);
+				atomicMax(&kk[3 + k], a[3 + k]);
+			}
+		}
 	}
 }
 
@@ -181,61 +222,49 @@ __device__ GBox loadBox(const float *p) {
 	return b;
 }
 
-// one root node per thread; its children are leaf slots or nodes of a deeper level
-__global__ void k_refitLevel(const uint32_t *levelNodes, uint32_t count, uint32_t layout, void *nodes,
+// W lanes per root node, one child each (its children are leaf slots or nodes
+// of a deeper level): with a thread per node and its eight children one after
+// another in scratch a level of some hundred nodes took 27 us, so 6 us.
+template <int W, class Node>
+__global__ __launch_bounds__(256) void k_refitLevel(const uint32_t *levelNodes, uint32_t count, Node *nodes,
 		const float *slotBoxes, float *nodeBoxes) {
-	const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
+	const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+	const uint32_t e = t / W;
+	const int c = (int)(t % W);
 	if (e >= count) return;
 	const uint32_t idx = levelNodes[e];
-	uint32_t child[8];
-	for (int c = 0; c < 8; ++c) child[c] = LRH_CHILD_EMPTY;
-	int n = 0, width = 4;
-	if (layout == 0) {
-		const lrh_node4q *q = reinterpret_cast<const lrh_node4q *>(nodes) + idx;
-		n = q->nchild;
-		for (int c = 0; c < 4; ++c) child[c] = q->child[c];
-	} else if (layout == 2) {
-		const lrh_node8q *q = reinterpret_cast<const lrh_node8q *>(nodes) + idx;
-		n = q->nchild;
-		width = 8;
-		for (int c = 0; c < 8; ++c) child[c] = q->child[c];
-	} else {
-		const lrh_node4f *f = reinterpret_cast<const lrh_node4f *>(nodes) + idx;
-		for (int c = 0; c < 4; ++c) {
-			child[c] = f->child[c];
-			if (child[c] != LRH_CHILD_EMPTY) n = c + 1;
-		}
+	Node *node = nodes + idx;
+	const uint32_t child = node->child[c];
+	// children fill the first slots
+	int n = child != LRH_CHILD_EMPTY ? c + 1 : 0;
+	for (int o = W / 2; o > 0; o >>= 1) {
+		const int x = __shfl_xor(n, o);
+		n = x > n ? x : n;
 	}
-	if (n > width) n = width;
-	GBox cb[8];
-	GBox u;
-	for (int k = 0; k < 3; ++k) { u.lo[k] = INFINITY; u.hi[k] = -INFINITY; }
-	for (int c = 0; c < n; ++c) {
-		const uint32_t r = child[c];
-		if (r & LRH_CHILD_LEAF) {
-			const uint32_t start = r & LRH_LEAF_START_MASK;
-			const uint32_t cnt = ((r >> LRH_LEAF_START_BITS) & 7u) + 1u;
-			GBox b = loadBox(slotBoxes + 6 * (size_t)start);
+	GBox b;
+	for (int k = 0; k < 3; ++k) { b.lo[k] = INFINITY; b.hi[k] = -INFINITY; }
+	if (child != LRH_CHILD_EMPTY) {
+		if (child & LRH_CHILD_LEAF) {
+			const uint32_t start = child & LRH_LEAF_START_MASK;
+			const uint32_t cnt = ((child >> LRH_LEAF_START_BITS) & 7u) + 1u;
+			b = loadBox(slotBoxes + 6 * (size_t)start);
 			for (uint32_t j = 1; j < cnt; ++j) {
 				const GBox o = loadBox(slotBoxes + 6 * (size_t)(start + j));
 				for (int k = 0; k < 3; ++k) { b.lo[k] = minT(b.lo[k], o.lo[k]); b.hi[k] = maxT(b.hi[k], o.hi[k]); }
 			}
-			cb[c] = b;
-		} else {
-			cb[c] = loadBox(nodeBoxes + 6 * (size_t)r);
-		}
-		for (int k = 0; k < 3; ++k) { u.lo[k] = minT(u.lo[k], cb[c].lo[k]); u.hi[k] = maxT(u.hi[k], cb[c].hi[k]); }
+		} else
+			b = loadBox(nodeBoxes + 6 * (size_t)child);
 	}
-	for (int k = 0; k < 3; ++k) {
-		nodeBoxes[6 * (size_t)idx + k] = u.lo[k];
-		nodeBoxes[6 * (size_t)idx + 3 + k] = u.hi[k];
-	}
-	if (layout == 0)
-		quantizeNode(cb, n, child, reinterpret_cast<lrh_node4q *>(nodes) + idx);
-	else if (layout == 2)
-		quantizeNode8(cb, n, child, reinterpret_cast<lrh_node8q *>(nodes) + idx);
+	GBox u;
+	if constexpr (std::is_same<Node, lrh_node4f>::value)
+		u = floatNodeLanes(b, c, n, child, node);
 	else
-		floatNode(cb, n, child, reinterpret_cast<lrh_node4f *>(nodes) + idx);
+		u = quantizeNodeLanes<W>(b, c, n, child, node);
+	if (c == 0)
+		for (int k = 0; k < 3; ++k) {
+			nodeBoxes[6 * (size_t)idx + k] = u.lo[k];
+			nodeBoxes[6 * (size_t)idx + 3 + k] = u.hi[k];
+		}
 }
 
 inline unsigned grid(size_t n, unsigned b) { return (unsigned)((n + b - 1) / b); }
@@ -257,9 +286,16 @@ hipError_t lrhLaunchRefitMotion(const LrhRefitArgs &a, hipStream_t st) {
 hipError_t lrhLaunchRefitLevels(const LrhRefitArgs &a, hipStream_t st) {
 	for (uint32_t l = 0; l < a.nLevels; ++l) {
 		const uint32_t b = a.levelStart[l], c = a.levelStart[l + 1] - b;
-		if (c)
-			hipLaunchKernelGGL(k_refitLevel, dim3(grid(c, 256)), dim3(256), 0, st, a.levelNodes + b, c, a.layout,
-					a.nodes, a.slotBoxes, a.nodeBoxes);
+		if (!c) continue;
+		if (a.layout == 2)
+			hipLaunchKernelGGL((k_refitLevel<8, lrh_node8q>), dim3(grid(8 * (size_t)c, 256)), dim3(256), 0, st,
+					a.levelNodes + b, c, (lrh_node8q *)a.nodes, a.slotBoxes, a.nodeBoxes);
+		else if (a.layout == 1)
+			hipLaunchKernelGGL((k_refitLevel<4, lrh_node4f>), dim3(grid(4 * (size_t)c, 256)), dim3(256), 0, st,
+					a.levelNodes + b, c, (lrh_node4f *)a.nodes, a.slotBoxes, a.nodeBoxes);
+		else
+			hipLaunchKernelGGL((k_refitLevel<4, lrh_node4q>), dim3(grid(4 * (size_t)c, 256)), dim3(256), 0, st,
+					a.levelNodes + b, c, (lrh_node4q *)a.nodes, a.slotBoxes, a.nodeBoxes);
 	}
 	return hipGetLastError();
 }

@@ -164,3 +164,17 @@ def test_refit_motion_bound_closed_form(gpu_device, probe):
     assert _bound_err(box[0] + e, box[1] - e, expected(1024)) <= BOUND_TOL + 1e-6
     assert _bound_err(box[0] + e, box[1] - e, expected(1023)) > 2 * BOUND_TOL
     dsc.close()
+
+
+@pytest.mark.parametrize("layout", [0, 1, 2])
+@pytest.mark.parametrize("n_inst", [1, 2, 9, 70, 300])
+def test_refit_in_place_rewrites_the_built_nodes(gpu_device, layout, n_inst):
+    """A refit with the objects the scene was built from: every root node, a
+    lane per child, comes out with the bytes the host builder wrote."""
+    sc = scenes.instanced_scene(n_inst=n_inst, motion_frac=0.4, freq=3, extent=30.0, seed=5)
+    s = gpu_device.scene_mbvh(sc, layout=layout)
+    before, _ = s.download()
+    s.refit(sc)
+    after, _ = s.download()
+    assert np.array_equal(before, after)
+    s.close()
