@@ -320,27 +320,35 @@ def _mesh_structs(meshes):
     return arr, keep
 
 
+# LrhObject as numpy fills it, all objects at once (setting the fields of a
+# thousand ctypes structures one by one takes 2 ms, several times the edit)
+_OBJECT_DTYPE = np.dtype({"names": [f for f, _ in LrhObject._fields_],
+                          "formats": ["<u4", "<u4", "<u8", "<u8", "<u4", "<u8", "<u8"],
+                          "offsets": [getattr(LrhObject, f).offset for f, _ in LrhObject._fields_],
+                          "itemsize": ctypes.sizeof(LrhObject)})
+
+
 def _object_structs(scene):
     """LrhObject array from an InstancedScene (kind 1: obj_mat local->world;
     kind 2: keys global->local)."""
     n = len(scene.obj_mesh)
-    arr = (LrhObject * max(1, n))()
-    keep = []
     mats = np.ascontiguousarray(scene.obj_mat, dtype=np.float32).reshape(-1, 16)
     kt = np.ascontiguousarray(scene.key_times, dtype=np.float32)
     km = np.ascontiguousarray(scene.key_mats, dtype=np.float32).reshape(-1, 16)
-    keep += [mats, kt, km]
-    for o in range(n):
-        arr[o].mesh = int(scene.obj_mesh[o])
-        arr[o].kind = int(scene.obj_kind[o])
-        if arr[o].kind == 1:
-            arr[o].m = ctypes.cast(mats.ctypes.data + 64 * o, ctypes.POINTER(ctypes.c_float))
-        elif arr[o].kind == 2:
-            k0, k1 = int(scene.key_off[o]), int(scene.key_off[o + 1])
-            arr[o].nKeys = k1 - k0
-            arr[o].keyTimes = ctypes.cast(kt.ctypes.data + 4 * k0, ctypes.POINTER(ctypes.c_float))
-            arr[o].keyMats = ctypes.cast(km.ctypes.data + 64 * k0, ctypes.POINTER(ctypes.c_float))
-    return arr, keep
+    a = np.zeros(max(1, n), _OBJECT_DTYPE)
+    if n:
+        kind = np.asarray(scene.obj_kind[:n]).astype(np.int64)
+        a["mesh"][:n] = np.asarray(scene.obj_mesh).astype(np.int64)
+        a["kind"][:n] = kind
+        o = np.nonzero(kind == 1)[0]
+        a["m"][o] = mats.ctypes.data + 64 * o.astype(np.uint64)
+        o = np.nonzero(kind == 2)[0]
+        if o.size:
+            off = np.asarray(scene.key_off).astype(np.uint64)
+            a["nKeys"][o] = off[o + 1] - off[o]
+            a["keyTimes"][o] = kt.ctypes.data + np.uint64(4) * off[o]
+            a["keyMats"][o] = km.ctypes.data + np.uint64(64) * off[o]
+    return (LrhObject * max(1, n)).from_buffer(a), [a, mats, kt, km]
 
 
 def _build_opts(layout=0, max_leaf=4, threads=0, trav_cost=1.0, builder=BUILD_HOST_SAH, split_budget=0.0):
