@@ -1267,7 +1267,11 @@ LaunchShape chooseShape(lrh_device *dev, unsigned layout, bool two, bool any, bo
 	// idle lanes do too: 4,194,304 rays over moving instances 1,838 / 1,660 /
 	// 1,534 / 1,358 us.
 	L.refill = (o && o->refillThreshold) ? std::min(64u, o->refillThreshold) : two ? 48 : 16;
-	L.leafTris = (o && o->leafTris) ? o->leafTris : 8u;
+	// Two triangles of a leaf per pass: a wave waits for its longest leaf
+	// otherwise (8 / 2 / 1, bounce rays over 26.2M triangles 603 / 569 / 574 us,
+	// 3M rays among spheres 684 / 618 / 617; a soup, whose rays test 24
+	// triangles each, 863 / 875 / 896).  Two-level scenes test whole leaves.
+	L.leafTris = (o && o->leafTris) ? o->leafTris : 2u;
 	if (L.leafTris > 8) throw Error(LRH_EINVAL, "leafTris must be 0..8");
 	L.ldsBytes = (size_t)L.lds * L.block * sizeof(uint2) + extraLds;
 	if (L.ldsBytes > 65536) throw Error(LRH_ERANGE, "LDS stack, node cache and item table exceed 64 KiB per block");
@@ -1385,6 +1389,7 @@ struct BatchTable {
 	std::vector<uint32_t> starts;
 	unsigned layout = 0;
 	bool two = false;
+	bool any = false;  // some items are any-hit queries
 	unsigned maxDepth = 0;
 	uint64_t total = 0;
 	// the distinct scenes of the batch with their generation at creation
@@ -1426,6 +1431,7 @@ BatchTable makeTable(lrh_device *dev, const lrh_batch_item *items, unsigned n) {
 		if (j == 0) T.layout = s->layout;
 		else if (s->layout != T.layout) throw Error(LRH_EINVAL, "all scenes of a batch must share the node layout");
 		T.two = T.two || s->twoLevel;
+		T.any = T.any || it.query == LRH_QUERY_ANY;
 		T.maxDepth = std::max(T.maxDepth, s->maxDepth);
 		bool seen = false;
 		for (const auto &sg : T.sceneGen) seen = seen || sg.scene == s;
@@ -1554,7 +1560,7 @@ int lrh_batch_create(lrh_device *dev, const lrh_batch_item *items, unsigned int 
 		b->dev = dev;
 		b->T = makeTable(dev, items, nItems);
 		const size_t extra = ((nItems + 1) * sizeof(uint32_t) + 15) & ~(size_t)15;
-		b->L = chooseShape(dev, b->T.layout, b->T.two, false, true, (unsigned)std::max<uint64_t>(b->T.total, 1),
+		b->L = chooseShape(dev, b->T.layout, b->T.two, b->T.any, true, (unsigned)std::max<uint64_t>(b->T.total, 1),
 				b->T.maxDepth, extra, opts);
 		const unsigned nLanes = b->L.blocks * b->L.block;
 		b->descs.alloc(dev, b->T.descs.size() * sizeof(LrhBatchDesc));
@@ -1593,7 +1599,7 @@ int lrh_batch_launch(lrh_batch *b, void *stream) {
 		if (b->T.total == 0) return;
 		checkBatchScenes(b);
 		hipStream_t st = stream ? (hipStream_t)stream : b->dev->stream;
-		HIPCHK(lrhLaunchTrace(b->T.layout, b->T.two, false, false, true, dim3(b->L.blocks), dim3(b->L.block),
+		HIPCHK(lrhLaunchTrace(b->T.layout, b->T.two, b->T.any, false, true, dim3(b->L.blocks), dim3(b->L.block),
 				b->L.ldsBytes, st, b->P));
 		b->dev->rays += b->T.total;
 	});
@@ -1610,7 +1616,7 @@ int lrh_batch_capture(lrh_batch *b, void *stream) {
 		HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
 		hipError_t le = hipSuccess;
 		if (b->T.total)
-			le = lrhLaunchTrace(b->T.layout, b->T.two, false, false, true, dim3(b->L.blocks), dim3(b->L.block),
+			le = lrhLaunchTrace(b->T.layout, b->T.two, b->T.any, false, true, dim3(b->L.blocks), dim3(b->L.block),
 					b->L.ldsBytes, st, b->P);
 		const hipError_t ce = hipStreamEndCapture(st, &b->graph);
 		HIPCHK(le);
@@ -1658,7 +1664,7 @@ int lrh_trace_batch(lrh_device *dev, const lrh_batch_item *items, unsigned int n
 		BatchTable T = makeTable(dev, items, nItems);
 		if (T.total == 0) return;
 		const size_t extra = ((nItems + 1) * sizeof(uint32_t) + 15) & ~(size_t)15;
-		const LaunchShape L = chooseShape(dev, T.layout, T.two, false, true, (unsigned)T.total, T.maxDepth, extra, opts);
+		const LaunchShape L = chooseShape(dev, T.layout, T.two, T.any, true, (unsigned)T.total, T.maxDepth, extra, opts);
 		const unsigned nLanes = L.blocks * L.block;
 		lrh_device::Workspace &w = workspace(dev, st, (size_t)nLanes * L.spillDepth * sizeof(uint2));
 		{
@@ -1695,7 +1701,7 @@ int lrh_trace_batch(lrh_device *dev, const lrh_batch_item *items, unsigned int n
 		P.items = dDesc;
 		P.itemStart = dStart;
 		P.nItems = nItems;
-		HIPCHK(lrhLaunchTrace(T.layout, T.two, false, false, true, dim3(L.blocks), dim3(L.block), L.ldsBytes, st, P));
+		HIPCHK(lrhLaunchTrace(T.layout, T.two, T.any, false, true, dim3(L.blocks), dim3(L.block), L.ldsBytes, st, P));
 		dev->rays += T.total;
 	});
 }

@@ -38,10 +38,16 @@ namespace {
 DEVI float asf(uint32_t u) { return __uint_as_float(u); }
 DEVI uint32_t asu(float f) { return __float_as_uint(f); }
 
+// Reciprocal of a direction component for the box tests: a zero component
+// becomes +-1e-20 so slab products stay finite.  The hardware reciprocal is
+// within 1 ulp, far inside the widening of the intervals, and the triangle
+// test does not use it; a correctly rounded division takes ten instructions
+// more, for every ray and, in two-level scenes, on entering and on leaving
+// an object (moving instances 1,365 -> 1,320 us).  It flushes results
+// below the normal range, so huge components are divided.
 DEVI float safeRcp(float d) {
-	// a zero component becomes +-1e-20 so slab products stay finite
 	const float dd = fabsf(d) < 1e-20f ? copysignf(1e-20f, d) : d;
-	return 1.0f / dd;
+	return __builtin_amdgcn_rcpf(dd);
 }
 
 DEVI float byteF(uint32_t w, int c) {
@@ -59,6 +65,11 @@ DEVI void setupRay(LocalRay &r) {
 	r.ix = safeRcp(r.dx);
 	r.iy = safeRcp(r.dy);
 	r.iz = safeRcp(r.dz);
+	if (fmaxf(fmaxf(fabsf(r.dx), fabsf(r.dy)), fabsf(r.dz)) > 1e30f) {
+		if (fabsf(r.dx) > 1e30f) r.ix = 1.0f / r.dx;
+		if (fabsf(r.dy) > 1e30f) r.iy = 1.0f / r.dy;
+		if (fabsf(r.dz) > 1e30f) r.iz = 1.0f / r.dz;
+	}
 	r.nx = -r.ox * r.ix;
 	r.ny = -r.oy * r.iy;
 	r.nz = -r.oz * r.iz;
@@ -114,12 +125,14 @@ __device__ __forceinline__ void motionSample(const lrh_motion *mot, const lrh_mo
 }
 
 // ---- node tests: up to 4 children -> (entry distance, child ref) ----
-// conservative widening of the slab interval by 2^-20 of |t| on each side
-// (entry t - |t| eps, exit t + |t| eps: wider for either sign of t, which a
-// plain scale by 1 -/+ eps is not for negative t, i.e. negative mint)
-constexpr float kWiden = 1.0f / 1048576.0f;
-DEVI float widenLo(float t) { return fmaf(-fabsf(t), kWiden, t); }
-DEVI float widenHi(float t) { return fmaf(fabsf(t), kWiden, t); }
+// The slab interval is widened conservatively on its far side only, by 2^-19
+// of |t| and with the current hit's distance in it: what a hit at t needs is
+// entry <= exit with both off by up to 2^-20 of |t|, and the same of entry
+// and best, so one widening of min(exit, best) serves where one on each side
+// was two instructions per child.  Adding a multiple of |t| is wider for
+// either sign of t, which a scale by 1 + eps is not (negative mint).
+constexpr float kWiden = 1.0f / 524288.0f;
+DEVI float widen(float t) { return fmaf(fabsf(t), kWiden, t); }
 
 DEVI void testNodeQ(const lrh_node4q *__restrict__ nodes, uint32_t idx, const LocalRay &r, float mint, float best,
 		float t[4], uint32_t c[4]) {
@@ -138,9 +151,7 @@ DEVI void testNodeQ(const lrh_node4q *__restrict__ nodes, uint32_t idx, const Lo
 		const float tnx = fmaf(byteF(nX, k), Ax, Bx), tfx = fmaf(byteF(fX, k), Ax, Bx);
 		const float tny = fmaf(byteF(nY, k), Ay, By), tfy = fmaf(byteF(fY, k), Ay, By);
 		const float tnz = fmaf(byteF(nZ, k), Az, Bz), tfz = fmaf(byteF(fZ, k), Az, Bz);
-		const float tn = widenLo(fmaxf(fmaxf(tnx, tny), tnz));
-		const float tf = widenHi(fminf(fminf(tfx, tfy), tfz));
-		const float a = fmaxf(tn, mint), b = fminf(tf, best);
+		const float a = fmaxf(fmaxf(fmaxf(tnx, tny), tnz), mint), b = widen(fminf(fminf(fminf(tfx, tfy), tfz), best));
 		// empty slots hold inverted boxes; one that still passes (a far node
 		// whose inverted extent is below the widening) is dropped when its
 		// LRH_CHILD_EMPTY reference is taken or popped
@@ -170,9 +181,7 @@ DEVI void testNode8Q(const lrh_node8q *__restrict__ nodes, uint32_t idx, const L
 		const float tnx = fmaf(byteF(nX[w], b), Ax, Bx), tfx = fmaf(byteF(fX[w], b), Ax, Bx);
 		const float tny = fmaf(byteF(nY[w], b), Ay, By), tfy = fmaf(byteF(fY[w], b), Ay, By);
 		const float tnz = fmaf(byteF(nZ[w], b), Az, Bz), tfz = fmaf(byteF(fZ[w], b), Az, Bz);
-		const float tn = widenLo(fmaxf(fmaxf(tnx, tny), tnz));
-		const float tf = widenHi(fminf(fminf(tfx, tfy), tfz));
-		const float a = fmaxf(tn, mint), bb = fminf(tf, best);
+		const float a = fmaxf(fmaxf(fmaxf(tnx, tny), tnz), mint), bb = widen(fminf(fminf(fminf(tfx, tfy), tfz), best));
 		t[k] = (a <= bb) ? a : INFINITY;
 	}
 }
@@ -192,11 +201,27 @@ DEVI void testNodeF(const lrh_node4f *__restrict__ nodes, uint32_t idx, const Lo
 		const float tnx = fmaf(sx ? LX[k] : HX[k], r.ix, r.nx), tfx = fmaf(sx ? HX[k] : LX[k], r.ix, r.nx);
 		const float tny = fmaf(sy ? LY[k] : HY[k], r.iy, r.ny), tfy = fmaf(sy ? HY[k] : LY[k], r.iy, r.ny);
 		const float tnz = fmaf(sz ? LZ[k] : HZ[k], r.iz, r.nz), tfz = fmaf(sz ? HZ[k] : LZ[k], r.iz, r.nz);
-		const float tn = widenLo(fmaxf(fmaxf(tnx, tny), tnz));
-		const float tf = widenHi(fminf(fminf(tfx, tfy), tfz));
-		const float a = fmaxf(tn, mint), b = fminf(tf, best);
+		const float a = fmaxf(fmaxf(fmaxf(tnx, tny), tnz), mint), b = widen(fminf(fminf(fminf(tfx, tfy), tfz), best));
 		t[k] = (a <= b) ? a : INFINITY;  // empty slots: lo = +inf, hi = -inf
 	}
+}
+
+// Children as (entry distance, reference) in one double: the distance's bits
+// are its high word, so doubles order as the distances do (INFINITY's bits are
+// those of a finite double, and no distance is a NaN), and a comparator is one
+// v_min_f64 and one v_max_f64, each issued in 4 cycles like any fp32 minimum,
+// where comparing and exchanging two registers takes one compare and four
+// selects of 4 cycles each.  Equal distances order by reference, not by the
+// network, which a closest hit does not see.
+DEVI double key64(float t, uint32_t c) { return __hiloint2double((int)asu(t), (int)c); }
+DEVI float keyT(double k) { return asf((uint32_t)__double2hiint(k)); }
+DEVI uint32_t keyC(double k) { return (uint32_t)__double2loint(k); }
+DEVI void kswap(double &a, double &b) {
+	double lo, hi;
+	asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
+	asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+	a = lo;
+	b = hi;
 }
 
 DEVI void cswap(float &ta, uint32_t &ca, float &tb, uint32_t &cb) {
@@ -206,11 +231,56 @@ DEVI void cswap(float &ta, uint32_t &ca, float &tb, uint32_t &cb) {
 	ta = t0; tb = t1; ca = c0; cb = c1;
 }
 
+// sorting networks: 5 comparators for four entries, 19 for eight
+DEVI void sort4(float t[4], uint32_t c[4]) {
+	cswap(t[0], c[0], t[1], c[1]);
+	cswap(t[2], c[2], t[3], c[3]);
+	cswap(t[0], c[0], t[2], c[2]);
+	cswap(t[1], c[1], t[3], c[3]);
+	cswap(t[1], c[1], t[2], c[2]);
+}
+DEVI void sort4Closest(float t[4], uint32_t c[4]) {
+	double k[4];
+#pragma unroll
+	for (int i = 0; i < 4; ++i) k[i] = key64(t[i], c[i]);
+	kswap(k[0], k[1]);
+	kswap(k[2], k[3]);
+	kswap(k[0], k[2]);
+	kswap(k[1], k[3]);
+	kswap(k[1], k[2]);
+#pragma unroll
+	for (int i = 0; i < 4; ++i) { t[i] = keyT(k[i]); c[i] = keyC(k[i]); }
+}
+DEVI void sort8(float t[8], uint32_t c[8]) {
+	cswap(t[0], c[0], t[2], c[2]); cswap(t[1], c[1], t[3], c[3]);
+	cswap(t[4], c[4], t[6], c[6]); cswap(t[5], c[5], t[7], c[7]);
+	cswap(t[0], c[0], t[4], c[4]); cswap(t[1], c[1], t[5], c[5]);
+	cswap(t[2], c[2], t[6], c[6]); cswap(t[3], c[3], t[7], c[7]);
+	cswap(t[0], c[0], t[1], c[1]); cswap(t[2], c[2], t[3], c[3]);
+	cswap(t[4], c[4], t[5], c[5]); cswap(t[6], c[6], t[7], c[7]);
+	cswap(t[2], c[2], t[4], c[4]); cswap(t[3], c[3], t[5], c[5]);
+	cswap(t[1], c[1], t[4], c[4]); cswap(t[3], c[3], t[6], c[6]);
+	cswap(t[1], c[1], t[2], c[2]); cswap(t[3], c[3], t[4], c[4]);
+	cswap(t[5], c[5], t[6], c[6]);
+}
+DEVI void sort8Closest(float t[8], uint32_t c[8]) {
+	double k[8];
+#pragma unroll
+	for (int i = 0; i < 8; ++i) k[i] = key64(t[i], c[i]);
+	kswap(k[0], k[2]); kswap(k[1], k[3]); kswap(k[4], k[6]); kswap(k[5], k[7]);
+	kswap(k[0], k[4]); kswap(k[1], k[5]); kswap(k[2], k[6]); kswap(k[3], k[7]);
+	kswap(k[0], k[1]); kswap(k[2], k[3]); kswap(k[4], k[5]); kswap(k[6], k[7]);
+	kswap(k[2], k[4]); kswap(k[3], k[5]); kswap(k[1], k[4]); kswap(k[3], k[6]);
+	kswap(k[1], k[2]); kswap(k[3], k[4]); kswap(k[5], k[6]);
+#pragma unroll
+	for (int i = 0; i < 8; ++i) { t[i] = keyT(k[i]); c[i] = keyC(k[i]); }
+}
+
 // ---- stack: top ldsDepth entries in LDS (ring), the rest spilled ----
 struct Stack {
 	uint2 *lds;
 	uint2 *spill;
-	uint32_t stride;    // blockDim (LDS) / nLanes (spill)
+	uint32_t shift;     // log2 of blockDim
 	uint32_t lane;      // threadIdx / global lane
 	uint32_t gstride;
 	uint32_t glane;
@@ -221,7 +291,7 @@ struct Stack {
 };
 
 DEVI bool push(Stack &s, uint32_t ref, float t, uint32_t *err) {
-	uint2 *e = &s.lds[(s.sp & s.mask) * s.stride + s.lane];
+	uint2 *e = &s.lds[((s.sp & s.mask) << s.shift) + s.lane];
 	if (s.sp >= s.depth) {
 		const uint32_t k = s.sp - s.depth;
 		if (k >= s.spillDepth) {
@@ -237,7 +307,7 @@ DEVI bool push(Stack &s, uint32_t ref, float t, uint32_t *err) {
 
 DEVI uint2 pop(Stack &s) {
 	--s.sp;
-	uint2 *e = &s.lds[(s.sp & s.mask) * s.stride + s.lane];
+	uint2 *e = &s.lds[((s.sp & s.mask) << s.shift) + s.lane];
 	const uint2 v = *e;
 	if (s.sp >= s.depth) *e = s.spill[(size_t)(s.sp - s.depth) * s.gstride + s.glane];
 	return v;
@@ -319,6 +389,12 @@ DEVI Tickets takeTickets(TicketPool &pool, uint32_t *counter, uint32_t n, uint32
 }
 
 constexpr uint32_t kNoRay = 0xffffffffu;
+// Stack entries a lane pops in one pass: a lane whose entries all lie behind
+// its hit goes on popping in the next pass instead of holding up the wave
+// (no limit / 1 / 2 / 3: bounce rays over 26.2M triangles 600 / 603 / 603 /
+// 600 us, over 2.1M 174 / 165 / 168 / 168, a soup 871 / 895 / 863 / 863, moving
+// instances 1,292 / 1,311 / 1,238 / 1,244).
+constexpr uint32_t kMaxPops = 2;
 constexpr uint32_t kMaxSteps = 1u << 24;  // per-ray guard against corrupt trees
 
 }  // namespace
@@ -346,7 +422,7 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 	Stack st;
 	st.lds = ldsStack;
 	st.spill = P.spill;
-	st.stride = blockDim.x;
+	st.shift = 31u - (uint32_t)__clz((int)blockDim.x);
 	st.lane = threadIdx.x;
 	st.gstride = P.nLanes;
 	st.glane = blockIdx.x * blockDim.x + threadIdx.x;
@@ -378,7 +454,7 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 	v.times = P.times;
 	v.hits = P.hits;
 	v.root = P.root;
-	v.flags = (ANY ? LRH_ITEM_ANY : 0u) | (TWO ? LRH_ITEM_TWO : 0u);
+	v.flags = (ANY && !BATCH ? LRH_ITEM_ANY : 0u) | (TWO ? LRH_ITEM_TWO : 0u);
 
 	uint32_t rid = kNoRay;  // ray index within its buffer
 	LocalRay r;
@@ -498,9 +574,9 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 		// ---- node phase: one node test per lane and pass ----
 		bool done = false, tested = false;
 		if (rid != kNoRay) {
-			for (;;) {
+			for (uint32_t pops = 0;;) {
 				if (cur == LRH_CHILD_EMPTY) {
-					if (st.sp == 0) break;
+					if (st.sp == 0 || pops++ == kMaxPops) break;
 					const uint2 e = pop(st);
 					cur = e.x;
 					curT = asf(e.y);
@@ -511,7 +587,7 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 						setupRay(r);
 						inInst = false;
 						cur = LRH_CHILD_EMPTY;
-					} else if (!(curT < best)) {
+					} else if (!(curT <= widen(best))) {
 						cur = LRH_CHILD_EMPTY;  // entry not before the current hit
 					}
 					if (cur == LRH_CHILD_EMPTY) continue;
@@ -530,17 +606,9 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 					float t8[8];
 					uint32_t c8[8];
 					testNode8Q(reinterpret_cast<const lrh_node8q *>(v.nodes), cur, r, mint, best, t8, c8);
-					// 19-comparator sorting network for eight entries
-					cswap(t8[0], c8[0], t8[2], c8[2]); cswap(t8[1], c8[1], t8[3], c8[3]);
-					cswap(t8[4], c8[4], t8[6], c8[6]); cswap(t8[5], c8[5], t8[7], c8[7]);
-					cswap(t8[0], c8[0], t8[4], c8[4]); cswap(t8[1], c8[1], t8[5], c8[5]);
-					cswap(t8[2], c8[2], t8[6], c8[6]); cswap(t8[3], c8[3], t8[7], c8[7]);
-					cswap(t8[0], c8[0], t8[1], c8[1]); cswap(t8[2], c8[2], t8[3], c8[3]);
-					cswap(t8[4], c8[4], t8[5], c8[5]); cswap(t8[6], c8[6], t8[7], c8[7]);
-					cswap(t8[2], c8[2], t8[4], c8[4]); cswap(t8[3], c8[3], t8[5], c8[5]);
-					cswap(t8[1], c8[1], t8[4], c8[4]); cswap(t8[3], c8[3], t8[6], c8[6]);
-					cswap(t8[1], c8[1], t8[2], c8[2]); cswap(t8[3], c8[3], t8[4], c8[4]);
-					cswap(t8[5], c8[5], t8[6], c8[6]);
+					// an any-hit ray reports the first blocker it meets: its order is kept to the network's
+					if (ANY) sort8(t8, c8);
+					else sort8Closest(t8, c8);
 					bool ok = true;
 					// sorted: the lanes that push entry k also push k-1..1; a
 					// position no lane of the wave reaches is skipped as a whole
@@ -562,11 +630,8 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 					testNodeQ(reinterpret_cast<const lrh_node4q *>(v.nodes), cur, r, mint, best, t4, c4);
 				else
 					testNodeF(reinterpret_cast<const lrh_node4f *>(v.nodes), cur, r, mint, best, t4, c4);
-				cswap(t4[0], c4[0], t4[1], c4[1]);
-				cswap(t4[2], c4[2], t4[3], c4[3]);
-				cswap(t4[0], c4[0], t4[2], c4[2]);
-				cswap(t4[1], c4[1], t4[3], c4[3]);
-				cswap(t4[1], c4[1], t4[2], c4[2]);
+				if (ANY) sort4(t4, c4);
+				else sort4Closest(t4, c4);
 				bool ok = true;
 				if (t4[3] != INFINITY) ok = ok && push(st, c4[3], t4[3], P.error);
 				if (t4[2] != INFINITY) ok = ok && push(st, c4[2], t4[2], P.error);
@@ -590,7 +655,7 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 		}
 		if (atLeaf) {
 			const bool two = TWO && (v.flags & LRH_ITEM_TWO);
-			const bool anyq = (BATCH || ANY) && (v.flags & LRH_ITEM_ANY);
+			const bool anyq = ANY && (v.flags & LRH_ITEM_ANY);
 			const uint32_t start = cur & LRH_LEAF_START_MASK;
 			uint32_t cnt = ((cur >> LRH_LEAF_START_BITS) & 7u) + 1u;
 			cur = LRH_CHILD_EMPTY;
@@ -734,8 +799,9 @@ __global__ __launch_bounds__(256) void lrh_trace2_kernel(LrhTraceParams P) {
 
 // batched traces over 8-wide nodes: at 7 waves per SIMD the per-lane item
 // view and the eight-entry sort spill; built for 6
+template <bool ANY>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void lrh_trace8b_kernel(LrhTraceParams P) {
-	traceBody<2, false, false, false, true>(P);
+	traceBody<2, false, ANY, false, true>(P);
 }
 
 // two-level traces over 8-wide nodes: the compiler's choice is 105 VGPRs
@@ -774,7 +840,10 @@ static const void *kernelPtr(int layout, bool two, bool any, bool count, bool ba
 			{(const void *)&lrh_trace28_kernel<false, false>, (const void *)&lrh_trace2_kernel<2, false, true, false>},
 			{(const void *)&lrh_trace28_kernel<true, false>, (const void *)&lrh_trace2_kernel<2, true, true, false>}};
 	if (layout == 2) {
-		if (batch) return two ? (const void *)&lrh_trace28_kernel<false, true> : (const void *)&lrh_trace8b_kernel;
+		static const void *batched8[2][2] = {
+				{(const void *)&lrh_trace8b_kernel<false>, (const void *)&lrh_trace8b_kernel<true>},
+				{(const void *)&lrh_trace28_kernel<false, true>, (const void *)&lrh_trace28_kernel<true, true>}};
+		if (batch) return batched8[two ? 1 : 0][any ? 1 : 0];
 		return two ? wide8Two[any ? 1 : 0][count ? 1 : 0] : wide8[any ? 1 : 0][count ? 1 : 0];
 	}
 	static const void *plain[2][2][2][2] = {
@@ -786,10 +855,13 @@ static const void *kernelPtr(int layout, bool two, bool any, bool count, bool ba
 		  {LRH_K(1, false, true, false, false), LRH_K(1, false, true, true, false)}},
 		 {{LRH_K(1, true, false, false, false), LRH_K(1, true, false, true, false)},
 		  {LRH_K(1, true, true, false, false), LRH_K(1, true, true, true, false)}}}};
-	// batched: the query is per item, so ANY is unused; COUNT is not offered
-	static const void *batched[2][2] = {{LRH_K(0, false, false, false, true), LRH_K(0, true, false, false, true)},
-			{LRH_K(1, false, false, false, true), LRH_K(1, true, false, false, true)}};
-	if (batch) return batched[layout ? 1 : 0][two ? 1 : 0];
+	// batched: the query is per item, `any` says that some of the batch's are any-hit; COUNT is not offered
+	static const void *batched[2][2][2] = {
+		{{LRH_K(0, false, false, false, true), LRH_K(0, false, true, false, true)},
+		 {LRH_K(0, true, false, false, true), LRH_K(0, true, true, false, true)}},
+		{{LRH_K(1, false, false, false, true), LRH_K(1, false, true, false, true)},
+		 {LRH_K(1, true, false, false, true), LRH_K(1, true, true, false, true)}}};
+	if (batch) return batched[layout ? 1 : 0][two ? 1 : 0][any ? 1 : 0];
 	return plain[layout ? 1 : 0][two ? 1 : 0][any ? 1 : 0][count ? 1 : 0];
 }
 
