@@ -1238,8 +1238,9 @@ int lrh_scene_download(lrh_scene *s, void *nodes, size_t nodeBytes, void *prims,
 namespace {
 
 struct LaunchShape {
-	unsigned block, lds, blocks, refill, spillDepth, leafTris;
+	unsigned block, lds, blocks, refill, spillDepth, leafTris, waveRays;
 	size_t ldsBytes;
+	bool drain;
 };
 
 unsigned pow2floor(unsigned v) {
@@ -1252,21 +1253,28 @@ unsigned pow2floor(unsigned v) {
 // from the occupancy of the kernel variant, and the spill depth the tree
 // depth needs (3 pushes per level plus the object sentinel)
 LaunchShape chooseShape(lrh_device *dev, unsigned layout, bool two, bool any, bool batch, unsigned count,
-		unsigned maxDepth, size_t extraLds, const lrh_trace_opts *o) {
+		unsigned maxDepth, size_t extraLds, const lrh_trace_opts *o, bool counting = false) {
 	LaunchShape L;
-	L.block = (o && o->blockSize) ? o->blockSize : 256;
+	// A small launch starts in the drain, which shares a ray among as many
+	// lanes as a node has children, 16 (4-wide nodes) or 8 rays to a wave: up to
+	// 4 or 6 such waves per SIMD (bounce rays, by lane and shared: 4,096 over
+	// 4-wide nodes 85 and 64 us, 60,000 118 and 102, over 8-wide ones 71 and 47,
+	// 40,000 98 and 75, 60,000 113 and 114).  Up to one wave per SIMD they go
+	// out in blocks of one wave, over all CUs.
+	const uint64_t simds = 4ull * (unsigned)dev->cuCount;
+	const unsigned drainRays = layout == 2 ? 8u : 16u;
+	const bool sparse = !batch && !counting && count <= drainRays * simds * (layout == 2 ? 6u : 4u);
+	// Two-level traces with the drain run four waves per SIMD instead of five
+	// or six: worth it up to four rays a lane (8-wide nodes, without and with it:
+	// 262,144 rays 213 and 182 us, 700,000 336 and 320, 1,500,000 548 and 550;
+	// 4-wide ones at 1,500,000 579 and 605).
+	L.drain = !two || batch || count <= simds * 1024u;
+	L.waveRays = sparse ? drainRays : 64u;
+	L.block = (o && o->blockSize) ? o->blockSize : sparse && count <= drainRays * simds ? 64 : 256;
 	if (L.block != 64 && L.block != 128 && L.block != 256) throw Error(LRH_EINVAL, "blockSize must be 64, 128 or 256");
 	L.lds = (o && o->ldsStack) ? o->ldsStack : 8;
 	if (L.lds < 4 || L.lds > 64 || pow2floor(L.lds) != L.lds)
 		throw Error(LRH_EINVAL, "ldsStack must be a power of two in 4..64");
-	// A refill costs a wave one LDS atomic and the wait for its rays, so waves
-	// are topped up early.  Measured on 2,073,600 rays, threshold 8 / 16 / 24 /
-	// 48: bounce rays over 26.2M triangles 670 / 640 / 622 / 624 us, camera rays
-	// 440 / 451 / 458 / 473 us (neighbouring rays end together: an early refill
-	// mixes them).  A two-level pass costs twice as much (object entries), so
-	// idle lanes do too: 4,194,304 rays over moving instances 1,838 / 1,660 /
-	// 1,534 / 1,358 us.
-	L.refill = (o && o->refillThreshold) ? std::min(64u, o->refillThreshold) : two ? 48 : 16;
 	// Two triangles of a leaf per pass: a wave waits for its longest leaf
 	// otherwise (8 / 2 / 1, bounce rays over 26.2M triangles 603 / 569 / 574 us,
 	// 3M rays among spheres 684 / 618 / 617; a soup, whose rays test 24
@@ -1280,12 +1288,12 @@ LaunchShape chooseShape(lrh_device *dev, unsigned layout, bool two, bool any, bo
 	int perCU = (o && o->blocksPerCU) ? (int)o->blocksPerCU : 0;
 	if (!perCU) {
 		const uint64_t key = ((uint64_t)layout << 40) | ((uint64_t)two << 39) | ((uint64_t)any << 38) |
-				((uint64_t)batch << 37) | ((uint64_t)L.ldsBytes << 8) | (L.block >> 6);
+				((uint64_t)batch << 37) | ((uint64_t)L.drain << 36) | ((uint64_t)L.ldsBytes << 8) | (L.block >> 6);
 		std::lock_guard<std::mutex> g(dev->mu);
 		auto it = dev->occ.find(key);
 		if (it == dev->occ.end()) {
 			int nb = 0;
-			HIPCHK(lrhOccupancy(layout, two, any, batch, L.block, L.ldsBytes, &nb));
+			HIPCHK(lrhOccupancy(layout, two, any, batch, L.drain, L.block, L.ldsBytes, &nb));
 			dev->occ[key] = nb > 0 ? nb : 1;
 			perCU = nb > 0 ? nb : 1;
 		} else
@@ -1293,8 +1301,22 @@ LaunchShape chooseShape(lrh_device *dev, unsigned layout, bool two, bool any, bo
 		perCU = std::max(1, (int)(((unsigned)perCU * pct + 50u) / 100u));
 	}
 	const unsigned persistent = (unsigned)perCU * (unsigned)dev->cuCount;
-	const unsigned need = (unsigned)(((uint64_t)count + L.block - 1) / L.block);
+	const unsigned blockRays = L.block / 64u * L.waveRays;
+	const unsigned need = (unsigned)(((uint64_t)count + blockRays - 1) / blockRays);
+	if (sparse && need > persistent) L.waveRays = 64u;  // (a small grid was asked for)
 	L.blocks = std::max(1u, std::min(persistent, need));
+	// A refill costs a wave one LDS atomic and the wait for its rays, so waves
+	// are topped up early, and the earlier the more rays there are to come for
+	// a lane: towards the end the rays that start last decide.  Measured at
+	// thresholds 8 / 16 / 24 / 40: 700,001 bounce rays (1.5 per lane) 211 / 212 /
+	// 220 / 225 us, 2,073,600 (4.5) 544 / 505 / 497 / 503, camera rays (4.5) 391 /
+	// 393 / 397 / 393, 3,000,001 among spheres (6.5) 637 / 579 / 572 / 554, a batch
+	// of 3.9M (12) 1,061 / 982 / 941 / 900.  A two-level pass costs twice as much
+	// (object entries), so idle lanes do too: 4,194,304 rays over moving
+	// instances at 8 / 16 / 24 / 48 1,627 / 1,475 / 1,373 / 1,238.
+	const uint64_t perLane = count / ((uint64_t)L.blocks * L.block);
+	L.refill = (o && o->refillThreshold) ? std::min(64u, o->refillThreshold)
+			: two ? 48 : perLane >= 6 ? 40 : perLane >= 3 ? 24 : 16;
 	// a visit pushes at most width - 1 entries
 	const unsigned worst = (layout == 2 ? 7u : 3u) * (maxDepth + 2u) + 4u;
 	L.spillDepth = worst > L.lds ? worst - L.lds : 1u;
@@ -1354,7 +1376,8 @@ int traceImpl(lrh_scene *s, const void *rays, void *hits, unsigned int count, un
 		dev->activate();
 		hipStream_t st = stream ? (hipStream_t)stream : dev->stream;
 		const bool any = query == LRH_QUERY_ANY;
-		const LaunchShape L = chooseShape(dev, s->layout, s->twoLevel, any, false, count, s->maxDepth, 0, opts);
+		const LaunchShape L = chooseShape(dev, s->layout, s->twoLevel, any, false, count, s->maxDepth, 0, opts,
+				statsOut != nullptr);
 		const unsigned nLanes = L.blocks * L.block;
 		lrh_device::Workspace &w = workspace(dev, st, (size_t)nLanes * L.spillDepth * sizeof(uint2));
 		LrhTraceParams P;
@@ -1367,13 +1390,14 @@ int traceImpl(lrh_scene *s, const void *rays, void *hits, unsigned int count, un
 		P.spill = w.spill;
 		P.spillDepth = L.spillDepth;
 		P.nLanes = nLanes;
+		P.waveRays = L.waveRays;
 		P.ldsDepth = L.lds;
 		P.refill = L.refill;
 		P.leafTris = L.leafTris;
 		P.error = dev->dError;
 		P.stats = w.stats;
 		if (statsOut) HIPCHK(hipMemsetAsync(w.stats, 0, LRH_TRACE_STATS * sizeof(unsigned long long), st));
-		HIPCHK(lrhLaunchTrace(s->layout, s->twoLevel, any, statsOut != nullptr, false, dim3(L.blocks), dim3(L.block),
+		HIPCHK(lrhLaunchTrace(s->layout, s->twoLevel, any, statsOut != nullptr, false, L.drain, dim3(L.blocks), dim3(L.block),
 				L.ldsBytes, st, P));
 		dev->rays += count;
 		if (statsOut) {
@@ -1539,12 +1563,13 @@ int lrh_trace_noalloc(lrh_scene *s, const void *rays, void *hits, unsigned int c
 		P.spill = spill;
 		P.spillDepth = L.spillDepth;
 		P.nLanes = L.blocks * L.block;
+		P.waveRays = L.waveRays;
 		P.ldsDepth = L.lds;
 		P.refill = L.refill;
 		P.leafTris = L.leafTris;
 		P.error = dev->dError;
 		P.stats = nullptr;
-		HIPCHK(lrhLaunchTrace(s->layout, s->twoLevel, any, false, false, dim3(L.blocks), dim3(L.block), L.ldsBytes, st,
+		HIPCHK(lrhLaunchTrace(s->layout, s->twoLevel, any, false, false, L.drain, dim3(L.blocks), dim3(L.block), L.ldsBytes, st,
 				P));
 		dev->rays += count;
 	});
@@ -1579,6 +1604,7 @@ int lrh_batch_create(lrh_device *dev, const lrh_batch_item *items, unsigned int 
 		P.spill = (uint2 *)b->spill.p;
 		P.spillDepth = b->L.spillDepth;
 		P.nLanes = nLanes;
+		P.waveRays = b->L.waveRays;
 		P.ldsDepth = b->L.lds;
 		P.refill = b->L.refill;
 		P.leafTris = b->L.leafTris;
@@ -1599,7 +1625,7 @@ int lrh_batch_launch(lrh_batch *b, void *stream) {
 		if (b->T.total == 0) return;
 		checkBatchScenes(b);
 		hipStream_t st = stream ? (hipStream_t)stream : b->dev->stream;
-		HIPCHK(lrhLaunchTrace(b->T.layout, b->T.two, b->T.any, false, true, dim3(b->L.blocks), dim3(b->L.block),
+		HIPCHK(lrhLaunchTrace(b->T.layout, b->T.two, b->T.any, false, true, true, dim3(b->L.blocks), dim3(b->L.block),
 				b->L.ldsBytes, st, b->P));
 		b->dev->rays += b->T.total;
 	});
@@ -1616,7 +1642,7 @@ int lrh_batch_capture(lrh_batch *b, void *stream) {
 		HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
 		hipError_t le = hipSuccess;
 		if (b->T.total)
-			le = lrhLaunchTrace(b->T.layout, b->T.two, b->T.any, false, true, dim3(b->L.blocks), dim3(b->L.block),
+			le = lrhLaunchTrace(b->T.layout, b->T.two, b->T.any, false, true, true, dim3(b->L.blocks), dim3(b->L.block),
 					b->L.ldsBytes, st, b->P);
 		const hipError_t ce = hipStreamEndCapture(st, &b->graph);
 		HIPCHK(le);
@@ -1693,6 +1719,7 @@ int lrh_trace_batch(lrh_device *dev, const lrh_batch_item *items, unsigned int n
 		P.spill = w.spill;
 		P.spillDepth = L.spillDepth;
 		P.nLanes = nLanes;
+		P.waveRays = L.waveRays;
 		P.ldsDepth = L.lds;
 		P.refill = L.refill;
 		P.leafTris = L.leafTris;
@@ -1701,7 +1728,7 @@ int lrh_trace_batch(lrh_device *dev, const lrh_batch_item *items, unsigned int n
 		P.items = dDesc;
 		P.itemStart = dStart;
 		P.nItems = nItems;
-		HIPCHK(lrhLaunchTrace(T.layout, T.two, T.any, false, true, dim3(L.blocks), dim3(L.block), L.ldsBytes, st, P));
+		HIPCHK(lrhLaunchTrace(T.layout, T.two, T.any, false, true, true, dim3(L.blocks), dim3(L.block), L.ldsBytes, st, P));
 		dev->rays += T.total;
 	});
 }

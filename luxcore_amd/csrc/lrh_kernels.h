@@ -43,6 +43,7 @@ struct LrhTraceParams {
 	uint2 *spill;                   /* spill stack: spillDepth entries x nLanes */
 	uint32_t spillDepth;
 	uint32_t nLanes;
+	uint32_t waveRays;              /* rays each wave starts with (at most 64), lane k the k-th of them */
 	uint32_t ldsDepth;              /* power of two */
 	uint32_t refill;                /* refill a wave when fewer lanes than this are live */
 	uint32_t leafTris;              /* triangles a lane tests per pass (1..8); the rest of a leaf waits a pass */
@@ -54,9 +55,10 @@ struct LrhTraceParams {
 };
 
 hipError_t lrhLaunchReset(uint32_t *p, uint32_t n, hipStream_t s);
-hipError_t lrhOccupancy(int layout, bool two, bool any, bool batch, int block, size_t lds,
+hipError_t lrhOccupancy(int layout, bool two, bool any, bool batch, bool drain, int block, size_t lds,
 		int *blocksPerCU);
-hipError_t lrhLaunchTrace(int layout, bool two, bool any, bool count, bool batch, dim3 grid, dim3 block,
+/* `drain` chooses between the two builds of a two-level trace (count, batch: ignored) */
+hipError_t lrhLaunchTrace(int layout, bool two, bool any, bool count, bool batch, bool drain, dim3 grid, dim3 block,
 		size_t lds, hipStream_t s, const LrhTraceParams &P);
 
 #endif

@@ -231,6 +231,34 @@ DEVI void cswap(float &ta, uint32_t &ca, float &tb, uint32_t &cb) {
 	ta = t0; tb = t1; ca = c0; cb = c1;
 }
 
+// Triangle::Intersect on one record, rounded as written: true if the ray
+// hits it at mint <= t < best
+DEVI bool testTri(const lrh_tri *__restrict__ rec, const LocalRay &r, float mint, float best, float &t, float &b1,
+		float &b2, uint32_t &triIndex, uint32_t &meshIndex) {
+	const uint4 *tp = reinterpret_cast<const uint4 *>(rec);
+	const uint4 a = tp[0], b = tp[1], c = tp[2];
+	const float p0x = asf(a.x), p0y = asf(a.y), p0z = asf(a.z);
+	const float e1x = asf(a.w), e1y = asf(b.x), e1z = asf(b.y);
+	const float e2x = asf(b.z), e2y = asf(b.w), e2z = asf(c.x);
+	const float s1x = (r.dy * e2z) - (r.dz * e2y);
+	const float s1y = (r.dz * e2x) - (r.dx * e2z);
+	const float s1z = (r.dx * e2y) - (r.dy * e2x);
+	const float div = s1x * e1x + s1y * e1y + s1z * e1z;
+	const float inv = 1.f / div;
+	const float ddx = r.ox - p0x, ddy = r.oy - p0y, ddz = r.oz - p0z;
+	b1 = (ddx * s1x + ddy * s1y + ddz * s1z) * inv;
+	const float s2x = (ddy * e1z) - (ddz * e1y);
+	const float s2y = (ddz * e1x) - (ddx * e1z);
+	const float s2z = (ddx * e1y) - (ddy * e1x);
+	b2 = (r.dx * s2x + r.dy * s2y + r.dz * s2z) * inv;
+	const float b0 = 1.f - b1 - b2;
+	t = (e2x * s2x + e2y * s2y + e2z * s2z) * inv;
+	triIndex = c.y;
+	meshIndex = c.z;
+	return (div != 0.f) && !(b1 < 0.f) && !(b2 < 0.f) && !(b0 < 0.f) &&
+			!(t < mint) && (t < best);
+}
+
 // sorting networks: 5 comparators for four entries, 19 for eight
 DEVI void sort4(float t[4], uint32_t c[4]) {
 	cswap(t[0], c[0], t[1], c[1]);
@@ -283,7 +311,7 @@ struct Stack {
 	uint32_t shift;     // log2 of blockDim
 	uint32_t lane;      // threadIdx / global lane
 	uint32_t gstride;
-	uint32_t glane;
+	uint32_t glane0;    // of thread 0: the spill column is glane0 + lane
 	uint32_t mask;      // ldsDepth - 1
 	uint32_t depth;     // ldsDepth
 	uint32_t spillDepth;
@@ -298,7 +326,7 @@ DEVI bool push(Stack &s, uint32_t ref, float t, uint32_t *err) {
 			atomicOr(err, 1u);
 			return false;
 		}
-		s.spill[(size_t)k * s.gstride + s.glane] = *e;
+		s.spill[(size_t)k * s.gstride + s.glane0 + s.lane] = *e;
 	}
 	*e = make_uint2(ref, asu(t));
 	++s.sp;
@@ -309,7 +337,7 @@ DEVI uint2 pop(Stack &s) {
 	--s.sp;
 	uint2 *e = &s.lds[((s.sp & s.mask) << s.shift) + s.lane];
 	const uint2 v = *e;
-	if (s.sp >= s.depth) *e = s.spill[(size_t)(s.sp - s.depth) * s.gstride + s.glane];
+	if (s.sp >= s.depth) *e = s.spill[(size_t)(s.sp - s.depth) * s.gstride + s.glane0 + s.lane];
 	return v;
 }
 
@@ -415,7 +443,307 @@ struct SceneView {
 	uint32_t flags;  // LRH_ITEM_ANY | LRH_ITEM_TWO
 };
 
-template <int LAYOUT, bool TWO, bool ANY, bool COUNT, bool BATCH>
+// ---- the drain: once no tickets are left and a wave holds at most 64 / W
+// rays, W lanes take each of them, a lane per child of a node and per
+// triangle of a leaf (W = the width of the nodes) ----
+// At the end of a launch every wave waits for its longest ray with the
+// other lanes idle, and its passes cost as much for one ray as for 64.  Shared
+// by W lanes a pass takes about a fifth of the vector instructions, with the
+// same order of visits and the same arithmetic, so the same hits.
+template <int CTRL>
+DEVI uint32_t dpp(uint32_t x) {
+	return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, true);
+}
+constexpr int kXor1 = 0xb1, kXor2 = 0x4e, kXor3 = 0x1b, kHalfMirror = 0x141;  // quad_perm, row_half_mirror
+
+// how many of the group's W keys are below this lane's
+template <int W>
+DEVI uint32_t groupRank(int key) {
+	const uint32_t k = (uint32_t)key;
+	uint32_t n = ((int)dpp<kXor1>(k) < key) + ((int)dpp<kXor2>(k) < key) + ((int)dpp<kXor3>(k) < key);
+	if (W == 8) {
+		const uint32_t m = dpp<kHalfMirror>(k);
+		n += ((int)m < key) + ((int)dpp<kXor1>(m) < key) + ((int)dpp<kXor2>(m) < key) + ((int)dpp<kXor3>(m) < key);
+	}
+	return n;
+}
+
+// One layer of a sorting network across the lanes of a group: the lanes of
+// `part` exchange with their partner (its entry: ot, oc), those of `low`
+// keep the nearer entry; equal ones stay, as in cswap.
+template <uint32_t PART, uint32_t LOW>
+DEVI void layer(uint32_t lane, float &t, uint32_t &ref, float ot, uint32_t oc) {
+	const bool low = (LOW >> lane) & 1u, part = (PART >> lane) & 1u;
+	const bool s = part && (low ? ot < t : t < ot);
+	t = s ? ot : t;
+	ref = s ? oc : ref;
+}
+
+// sort4 / sort8 across the lanes of a group, lane k with entry k: any-hit rays
+// report the first blocker they meet, so equal distances must come out in
+// the network's order here too
+template <int W>
+DEVI void groupSort(uint32_t lane, float &t, uint32_t &ref) {
+	auto T = [&t](auto f) { return asf(f(asu(t))); };
+	auto x1 = [](uint32_t x) { return dpp<kXor1>(x); };
+	auto x2 = [](uint32_t x) { return dpp<kXor2>(x); };
+	auto x3 = [](uint32_t x) { return dpp<kXor3>(x); };
+	if (W == 4) {
+		layer<0xf, 0x5>(lane, t, ref, T(x1), x1(ref));
+		layer<0xf, 0x3>(lane, t, ref, T(x2), x2(ref));
+		layer<0x6, 0x2>(lane, t, ref, T(x3), x3(ref));
+		return;
+	}
+	auto x7 = [](uint32_t x) { return dpp<kHalfMirror>(x); };
+	auto x4 = [](uint32_t x) { return dpp<kXor3>(dpp<kHalfMirror>(x)); };
+	auto x5 = [](uint32_t x) { return dpp<kXor2>(dpp<kHalfMirror>(x)); };
+	auto x6 = [](uint32_t x) { return dpp<kXor1>(dpp<kHalfMirror>(x)); };
+	layer<0xff, 0x33>(lane, t, ref, T(x2), x2(ref));
+	layer<0xff, 0x0f>(lane, t, ref, T(x4), x4(ref));
+	layer<0xff, 0x55>(lane, t, ref, T(x1), x1(ref));
+	layer<0x3c, 0x0c>(lane, t, ref, T(x6), x6(ref));  // (2,4) (3,5)
+	layer<0x5a, 0x0a>(lane, t, ref, T(x5), x5(ref));  // (1,4) (3,6)
+	const bool mid = lane == 3 || lane == 4;          // (1,2) (3,4) (5,6)
+	const float t3 = T(x3), t7 = T(x7);
+	const uint32_t r3 = x3(ref), r7 = x7(ref);
+	layer<0x7e, 0x2a>(lane, t, ref, mid ? t7 : t3, mid ? r7 : r3);
+}
+
+// the group's smallest float, to all its lanes
+template <int W>
+DEVI float groupMin(float x) {
+	x = fminf(x, asf(dpp<kXor1>(asu(x))));
+	x = fminf(x, asf(dpp<kXor2>(asu(x))));
+	if (W == 8) x = fminf(x, asf(dpp<kHalfMirror>(asu(x))));
+	return x;
+}
+
+DEVI void waveFence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
+// Pushes the entries of the lanes with `has` set, lane's own at place `i` of
+// the ray's stack (places sp .. top-1, one lane each): the top `depth`
+// places live in the LDS ring, what they displace and what lies below them
+// goes to the spill array.
+DEVI void drainPush(const Stack &s, bool has, uint32_t i, uint32_t top, uint32_t ref, float t, uint32_t *err) {
+	if (!has) return;
+	const uint2 entry = make_uint2(ref, asu(t));
+	if (i + s.depth < top) {
+		if (i < s.spillDepth) s.spill[(size_t)i * s.gstride + s.glane0 + s.lane] = entry;
+		else atomicOr(err, 1u);
+		return;
+	}
+	uint2 *e = &s.lds[((i & s.mask) << s.shift) + s.lane];
+	int old = (int)i - (int)s.depth;
+	if (old >= (int)s.sp) old -= (int)s.depth;
+	if (old >= 0) {
+		if ((uint32_t)old < s.spillDepth) s.spill[(size_t)old * s.gstride + s.glane0 + s.lane] = *e;
+		else atomicOr(err, 1u);
+	}
+	*e = entry;
+}
+
+// pops the top entry, for all lanes of the group (lane 0 refills the ring)
+DEVI uint2 drainPop(Stack &s, bool leader) {
+	--s.sp;
+	uint2 *e = &s.lds[((s.sp & s.mask) << s.shift) + s.lane];
+	const uint2 v = *e;
+	if (s.sp >= s.depth && leader) *e = s.spill[(size_t)(s.sp - s.depth) * s.gstride + s.glane0 + s.lane];
+	return v;
+}
+
+template <int LAYOUT, bool TWO, bool ANY, bool BATCH>
+DEVI void drain(const LrhTraceParams &P, Stack &st, SceneView &v, LocalRay &r, float wo[3], float wd[3], float mint,
+		float best, float time, float hb1, float hb2, uint32_t hTri, uint32_t hMesh, uint32_t cur, float curT,
+		uint32_t obj, bool inInst, uint32_t rid) {
+	constexpr uint32_t W = LAYOUT == 2 ? 8u : 4u;
+	const uint32_t lane = __lane_id();
+	const uint32_t c = lane & (W - 1u), group = lane / W;
+	// group g takes the g-th live ray: its registers from the lane that held
+	// it, its stack where it is
+	uint64_t live = __ballot(rid != kNoRay);
+	const uint32_t nLive = (uint32_t)__popcll(live);
+	uint32_t src = lane;
+	for (uint32_t g = 0; g < nLive; ++g) {
+		const uint32_t l = (uint32_t)__ffsll((long long)live) - 1u;
+		live &= live - 1u;
+		if (group == g) src = l;
+	}
+	auto shu = [src](uint32_t x) { return (uint32_t)__shfl((int)x, (int)src); };
+	auto shf = [&](float x) { return asf(shu(asu(x))); };
+	auto shp = [&](auto *x) {
+		const uint64_t a = (uint64_t)x;
+		return (decltype(x))(((uint64_t)shu((uint32_t)(a >> 32)) << 32) | shu((uint32_t)a));
+	};
+	r.ox = shf(r.ox); r.oy = shf(r.oy); r.oz = shf(r.oz);
+	r.dx = shf(r.dx); r.dy = shf(r.dy); r.dz = shf(r.dz);
+	r.ix = shf(r.ix); r.iy = shf(r.iy); r.iz = shf(r.iz);
+	r.nx = shf(r.nx); r.ny = shf(r.ny); r.nz = shf(r.nz);
+	mint = shf(mint); best = shf(best); hb1 = shf(hb1); hb2 = shf(hb2); curT = shf(curT);
+	hTri = shu(hTri); hMesh = shu(hMesh); cur = shu(cur);
+	if (TWO) {
+		for (int k = 0; k < 3; ++k) { wo[k] = shf(wo[k]); wd[k] = shf(wd[k]); }
+		time = shf(time);
+		obj = shu(obj);
+		inInst = shu(inInst ? 1u : 0u) != 0u;
+	}
+	if (BATCH) {
+		v.nodes = shp(v.nodes);
+		v.tris = shp(v.tris);
+		v.hits = shp(v.hits);
+		v.flags = shu(v.flags);
+		if (TWO) {
+			v.insts = shp(v.insts);
+			v.xforms = shp(v.xforms);
+			v.motions = shp(v.motions);
+			v.segs = shp(v.segs);
+			v.times = shp(v.times);
+		}
+	}
+	st.sp = shu(st.sp);
+	st.lane = (st.lane & ~63u) + src;
+	const uint32_t taken = shu(rid);  // (every exchange with all lanes active)
+	rid = group < nLive ? taken : kNoRay;
+	const bool two = TWO && (v.flags & LRH_ITEM_TWO);
+	const bool anyq = ANY && (v.flags & LRH_ITEM_ANY);
+	const bool leader = c == 0;
+	waveFence();
+	for (uint32_t steps = 0; __ballot(rid != kNoRay); ++steps) {
+		if (rid == kNoRay) continue;
+		bool done = false;
+		while (cur == LRH_CHILD_EMPTY && st.sp) {
+			const uint2 e = drainPop(st, leader);
+			waveFence();
+			cur = e.x;
+			curT = asf(e.y);
+			if (TWO && cur == LRH_SENTINEL) {
+				r.ox = wo[0]; r.oy = wo[1]; r.oz = wo[2];
+				r.dx = wd[0]; r.dy = wd[1]; r.dz = wd[2];
+				setupRay(r);
+				inInst = false;
+				cur = LRH_CHILD_EMPTY;
+			} else if (!(curT <= widen(best)))
+				cur = LRH_CHILD_EMPTY;
+		}
+		if (cur != LRH_CHILD_EMPTY && !(cur & LRH_CHILD_LEAF)) {
+			float tnx, tfx, tny, tfy, tnz, tfz;
+			uint32_t child;
+			if (LAYOUT == 1) {
+				const char *nb = reinterpret_cast<const char *>(reinterpret_cast<const lrh_node4f *>(v.nodes) + cur) + 4 * c;
+				const uint32_t x = r.ix >= 0.f ? 0u : 16u, y = r.iy >= 0.f ? 32u : 48u, z = r.iz >= 0.f ? 64u : 80u;
+				auto f = [nb](uint32_t off) { return *reinterpret_cast<const float *>(nb + off); };
+				tnx = fmaf(f(x), r.ix, r.nx); tfx = fmaf(f(x ^ 16u), r.ix, r.nx);
+				tny = fmaf(f(y), r.iy, r.ny); tfy = fmaf(f(y ^ 16u), r.iy, r.ny);
+				tnz = fmaf(f(z), r.iz, r.nz); tfz = fmaf(f(z ^ 16u), r.iz, r.nz);
+				child = *reinterpret_cast<const uint32_t *>(nb + 96);
+			} else {
+				// the bounds' words of this child: lo and hi of an axis are `far` bytes apart
+				constexpr uint32_t far = W, axis = 2 * W;
+				const char *nb = reinterpret_cast<const char *>(v.nodes) + (size_t)cur * (LAYOUT == 2 ? 128u : 64u);
+				const uint4 q0 = *reinterpret_cast<const uint4 *>(nb);
+				const uint32_t o = 16u + (c & 4u);
+				const uint32_t x = o ^ (r.ix >= 0.f ? 0u : far), y = (o + axis) ^ (r.iy >= 0.f ? 0u : far),
+						z = (o + 2 * axis) ^ (r.iz >= 0.f ? 0u : far);
+				auto u = [nb](uint32_t off) { return *reinterpret_cast<const uint32_t *>(nb + off); };
+				const uint32_t wnx = u(x), wfx = u(x ^ far), wny = u(y), wfy = u(y ^ far), wnz = u(z), wfz = u(z ^ far);
+				child = u((LAYOUT == 2 ? 64u : 40u) + 4u * c);
+				const uint32_t sh = 8u * (c & 3u);
+				auto q = [sh](uint32_t w) { return (float)((w >> sh) & 0xffu); };
+				const float sx = asf((q0.w & 0xffu) << 23), sy = asf(((q0.w >> 8) & 0xffu) << 23),
+						sz = asf(((q0.w >> 16) & 0xffu) << 23);
+				const float Ax = sx * r.ix, Ay = sy * r.iy, Az = sz * r.iz;
+				const float Bx = fmaf(asf(q0.x), r.ix, r.nx), By = fmaf(asf(q0.y), r.iy, r.ny),
+						Bz = fmaf(asf(q0.z), r.iz, r.nz);
+				tnx = fmaf(q(wnx), Ax, Bx); tfx = fmaf(q(wfx), Ax, Bx);
+				tny = fmaf(q(wny), Ay, By); tfy = fmaf(q(wfy), Ay, By);
+				tnz = fmaf(q(wnz), Az, Bz); tfz = fmaf(q(wfz), Az, Bz);
+			}
+			const float a = fmaxf(fmaxf(fmaxf(tnx, tny), tnz), mint), b = widen(fminf(fminf(fminf(tfx, tfy), tfz), best));
+			// (INFINITY is a miss, as in the tests by lane: a hit's key lies below every miss's)
+			const bool hit = a <= b && a < INFINITY && child != LRH_CHILD_EMPTY;
+			const uint32_t n = (uint32_t)__popc((uint32_t)(__ballot(hit) >> (lane & ~(W - 1u))) & ((1u << W) - 1u));
+			if (ANY) {
+				float t = hit ? a : INFINITY;
+				groupSort<W>(c, t, child);
+				drainPush(st, c < n, st.sp + (n - 1u - c), st.sp + n, child, t, P.error);
+			} else {
+				const uint32_t rank = groupRank<W>((int)(hit ? (asu(a) & ~7u) | c : 0x7f800000u | c));
+				drainPush(st, hit, st.sp + (n - 1u - rank), st.sp + n, child, a, P.error);
+			}
+			if (__ballot(st.sp + n > st.depth)) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // spilled entries written by other lanes
+			st.sp += n;
+			waveFence();
+			cur = LRH_CHILD_EMPTY;
+			if (n) {
+				const uint2 e = drainPop(st, leader);
+				waveFence();
+				cur = e.x;
+				curT = asf(e.y);
+			}
+			if (steps > kMaxSteps) {
+				if (leader) atomicOr(P.error, 2u);
+				done = true;
+			}
+		}
+		if (!done && cur != LRH_CHILD_EMPTY && (cur & LRH_CHILD_LEAF)) {
+			const uint32_t start = cur & LRH_LEAF_START_MASK, cnt = ((cur >> LRH_LEAF_START_BITS) & 7u) + 1u;
+			cur = LRH_CHILD_EMPTY;
+			if (two && !inInst) {
+				const lrh_inst in = v.insts[start];
+				if (in.kind == 1u) {
+					xfRay(v.xforms + 16 * (size_t)in.index, wo, wd, r);
+				} else if (in.kind == 2u) {
+					float M[16];
+					motionSample(v.motions + in.index, v.segs, v.times, time, M);
+					xfRay(M, wo, wd, r);
+				}
+				obj = in.object;
+				inInst = true;
+				drainPush(st, leader, st.sp, st.sp + 1u, LRH_SENTINEL, -INFINITY, P.error);
+				if (st.sp >= st.depth) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+				++st.sp;
+				waveFence();
+				cur = in.root;
+				curT = -INFINITY;
+			} else {
+				for (uint32_t k = 0; k < cnt && !done; k += W) {
+					float t = 0.f, b1 = 0.f, b2 = 0.f;
+					uint32_t triIndex = 0, meshIndex = 0;
+					const bool ok = k + c < cnt &&
+							testTri(v.tris + start + k + c, r, mint, best, t, b1, b2, triIndex, meshIndex);
+					const uint64_t oks = __ballot(ok);
+					const uint32_t mine = (uint32_t)(oks >> (lane & ~(W - 1u))) & ((1u << W) - 1u);
+					if (mine) {
+						// the record the sequential test would keep: the nearest, of equal ones
+						// the first; an any-hit ray's first
+						const float tm = groupMin<W>(ok ? t : INFINITY);
+						const uint32_t first = (uint32_t)(__ballot(ok && (anyq || t == tm)) >> (lane & ~(W - 1u))) &
+								((1u << W) - 1u);
+						const int w = (int)((lane & ~(W - 1u)) + (uint32_t)__ffs((int)first) - 1u);
+						best = __shfl(t, w);
+						hb1 = __shfl(b1, w);
+						hb2 = __shfl(b2, w);
+						hTri = (uint32_t)__shfl((int)triIndex, w);
+						hMesh = two ? obj : (uint32_t)__shfl((int)meshIndex, w);
+						done = anyq;
+					}
+				}
+			}
+		}
+		if (done || (cur == LRH_CHILD_EMPTY && st.sp == 0)) {
+			if (leader) {
+				lrh_hit_rec *h = v.hits + rid;
+				h->t = best;
+				h->b1 = hb1;
+				h->b2 = hb2;
+				h->meshIndex = hMesh;
+				h->triangleIndex = hTri;
+			}
+			rid = kNoRay;
+		}
+	}
+}
+
+template <int LAYOUT, bool TWO, bool ANY, bool COUNT, bool BATCH, bool DRAIN>
 __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 	extern __shared__ uint2 ldsStack[];  // [ldsDepth][blockDim] stack; batched: then item starts
 	const uint32_t lane = __lane_id();
@@ -425,7 +753,7 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 	st.shift = 31u - (uint32_t)__clz((int)blockDim.x);
 	st.lane = threadIdx.x;
 	st.gstride = P.nLanes;
-	st.glane = blockIdx.x * blockDim.x + threadIdx.x;
+	st.glane0 = blockIdx.x * blockDim.x;
 	st.mask = P.ldsDepth - 1;
 	st.depth = P.ldsDepth;
 	st.spillDepth = P.spillDepth;
@@ -442,7 +770,8 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 		pool.fetching = 0;
 	}
 	__syncthreads();
-	const uint32_t nStatic = gridDim.x * blockDim.x;  // tickets handed out by lane, without a counter
+	// tickets handed out by lane, without a counter: `waveRays` to each wave
+	const uint32_t nStatic = gridDim.x * (blockDim.x >> 6) * P.waveRays;
 
 	SceneView v;
 	v.nodes = P.nodes;
@@ -464,6 +793,8 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 	float curT = 0.f;
 	bool inInst = false;
 	bool first = true, exhausted = nStatic >= P.nRays;
+	// rays a wave hands to the drain (without one it goes on ray by lane)
+	constexpr uint32_t kDrainRays = !DRAIN ? 0u : LAYOUT == 2 ? 8u : 16u;
 	// COUNT variant only: per lane node tests / primitive tests / rays; per
 	// wave passes, live lanes summed over passes, passes with a node test,
 	// passes with a leaf test, refills
@@ -480,7 +811,7 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 		uint32_t ticket = P.nRays;  // none
 		if (first) {
 			first = false;
-			ticket = st.glane;
+			if (lane < P.waveRays) ticket = ((st.glane0 + st.lane) >> 6) * P.waveRays + lane;
 		} else if (!exhausted) {
 			const uint64_t idle = __ballot(rid == kNoRay);
 			const uint32_t nIdle = (uint32_t)__popcll(idle);
@@ -558,13 +889,21 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 				if (COUNT) ++cRay;
 			}
 		}
-		if (!__ballot(rid != kNoRay)) {
+		const uint64_t liveNow = __ballot(rid != kNoRay);
+		if (!liveNow) {
 			if (exhausted) break;
 			continue;
 		}
+		if constexpr (DRAIN) {
+			if (exhausted && (uint32_t)__popcll(liveNow) <= kDrainRays) {
+				drain<LAYOUT, TWO, ANY, BATCH>(P, st, v, r, wo, wd, mint, best, time, hb1, hb2, hTri, hMesh, cur, curT, obj,
+						inInst, rid);
+				break;
+			}
+		}
 		// passes until fewer than `refill` lanes are live (after the last
-		// ticket: until the wave is empty)
-		const uint32_t minLive = exhausted ? 1u : P.refill;
+		// ticket: until the drain takes the rest)
+		const uint32_t minLive = exhausted ? kDrainRays + 1u : P.refill;
 		do {
 		if (COUNT) {
 			++cPass;
@@ -691,33 +1030,14 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 					done = true;
 			} else {
 				for (uint32_t k = 0; k < cnt; ++k) {
-					const uint4 *tp = reinterpret_cast<const uint4 *>(v.tris + start + k);
-					const uint4 a = tp[0], b = tp[1], c = tp[2];
-					// Triangle::Intersect, rounded as written
-					const float p0x = asf(a.x), p0y = asf(a.y), p0z = asf(a.z);
-					const float e1x = asf(a.w), e1y = asf(b.x), e1z = asf(b.y);
-					const float e2x = asf(b.z), e2y = asf(b.w), e2z = asf(c.x);
-					const float s1x = (r.dy * e2z) - (r.dz * e2y);
-					const float s1y = (r.dz * e2x) - (r.dx * e2z);
-					const float s1z = (r.dx * e2y) - (r.dy * e2x);
-					const float div = s1x * e1x + s1y * e1y + s1z * e1z;
-					const float inv = 1.f / div;
-					const float ddx = r.ox - p0x, ddy = r.oy - p0y, ddz = r.oz - p0z;
-					const float b1 = (ddx * s1x + ddy * s1y + ddz * s1z) * inv;
-					const float s2x = (ddy * e1z) - (ddz * e1y);
-					const float s2y = (ddz * e1x) - (ddx * e1z);
-					const float s2z = (ddx * e1y) - (ddy * e1x);
-					const float b2 = (r.dx * s2x + r.dy * s2y + r.dz * s2z) * inv;
-					const float b0 = 1.f - b1 - b2;
-					const float t = (e2x * s2x + e2y * s2y + e2z * s2z) * inv;
-					const bool ok = (div != 0.f) && !(b1 < 0.f) && !(b2 < 0.f) && !(b0 < 0.f) &&
-							!(t < mint) && (t < best);
-					if (ok) {
+					float t, b1, b2;
+					uint32_t triIndex, meshIndex;
+					if (testTri(v.tris + start + k, r, mint, best, t, b1, b2, triIndex, meshIndex)) {
 						best = t;
 						hb1 = b1;
 						hb2 = b2;
-						hTri = c.y;
-						hMesh = two ? obj : c.z;
+						hTri = triIndex;
+						hMesh = two ? obj : meshIndex;
 						if (anyq) {
 							done = true;
 							break;
@@ -779,44 +1099,46 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 	}
 }
 
-// Single-level traces are built for 7 waves per SIMD (at most 72 VGPRs, no
-// spills), measured 1-3% faster than the 6 the compiler picks on its own.
-// Two-level traces over 64-byte nodes are built for 6 waves (80 VGPRs, 8
-// spilled): the motion sample is inlined and reads its motion record and
-// the hot part of its segment with all loads in flight at once; measured on
-// moving instances, 6 waves are 3% faster than 5 (90 VGPRs, no spills);
-// the other two-level variants (fp32 nodes, batched, counting) keep the
-// compiler's choice, which does not spill.
+// Single-level traces are built for 7 waves per SIMD (at most 72 VGPRs),
+// batched ones over 8-wide nodes (per-lane item view) for 5: at 6 the loop
+// spills (a batch of 3.9M rays 1,032 us, at 5 983 us).
 template <int LAYOUT, bool ANY, bool COUNT, bool BATCH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void lrh_trace_kernel(LrhTraceParams P) {
-	traceBody<LAYOUT, false, ANY, COUNT, BATCH>(P);
+	traceBody<LAYOUT, false, ANY, COUNT, BATCH, !COUNT>(P);
 }
 
+template <bool ANY>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void lrh_trace8b_kernel(LrhTraceParams P) {
+	traceBody<2, false, ANY, false, true, true>(P);
+}
+
+// Two-level traces inline the motion sample, which reads its motion record
+// and the hot part of its segment with all loads in flight at once.  Over
+// 64-byte nodes they are built for 6 waves per SIMD (80 VGPRs, 8 spilled: 3%
+// faster than 5 and 90 on moving instances), over 8-wide nodes for 5 (94
+// VGPRs; at 6 it spills 10), batched 8-wide ones for 4 (at 5 it spills 37).
+// With the drain, which holds a second motion sample, the loop spills; so
+// a launch that the drain is a small part of goes without.
 template <int LAYOUT, bool ANY, bool COUNT, bool BATCH>
 __global__ __launch_bounds__(256) void lrh_trace2_kernel(LrhTraceParams P) {
-	traceBody<LAYOUT, true, ANY, COUNT, BATCH>(P);
+	traceBody<LAYOUT, true, ANY, COUNT, BATCH, false>(P);
 }
 
-// batched traces over 8-wide nodes: at 7 waves per SIMD the per-lane item
-// view and the eight-entry sort spill; built for 6
-template <bool ANY>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void lrh_trace8b_kernel(LrhTraceParams P) {
-	traceBody<2, false, ANY, false, true>(P);
-}
-
-// two-level traces over 8-wide nodes: the compiler's choice is 105 VGPRs
-// (4 waves per SIMD); built for 5 (94 VGPRs, no spills; at 6 it spills 10),
-// the batched form (per-lane item view) for 4 (at 5 it spills 37)
 template <bool ANY, bool BATCH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BATCH ? 4 : 5))) void lrh_trace28_kernel(
 		LrhTraceParams P) {
-	traceBody<2, true, ANY, false, BATCH>(P);
+	traceBody<2, true, ANY, false, BATCH, false>(P);
 }
 
-template <bool ANY, bool COUNT>
+template <bool ANY>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void lrh_trace2q_kernel(LrhTraceParams P) {
-	traceBody<0, true, ANY, COUNT, false>(P);
-}  // (the counting variants keep lrh_trace2_kernel: at 80 VGPRs they would spill)
+	traceBody<0, true, ANY, false, false, false>(P);
+}
+
+template <int LAYOUT, bool ANY>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void lrh_trace2_drain_kernel(LrhTraceParams P) {
+	traceBody<LAYOUT, true, ANY, false, false, true>(P);
+}
 
 __global__ void lrh_reset_kernel(uint32_t *p, uint32_t n) {
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -828,41 +1150,34 @@ __global__ void lrh_reset_kernel(uint32_t *p, uint32_t n) {
 // ---------------------------------------------------------------------------
 typedef void (*KernelFn)(LrhTraceParams);
 
-#define LRH_K(L, T, A, C, B)                                                                  \
-	((T) ? ((L) == 0 && !(B) && !(C) ? (const void *)&lrh_trace2q_kernel<A, false>            \
-	                         : (const void *)&lrh_trace2_kernel<L, A, C, B>)                  \
-	     : (const void *)&lrh_trace_kernel<L, A, C, B>)
-static const void *kernelPtr(int layout, bool two, bool any, bool count, bool batch) {
-	// 8-wide nodes
-	static const void *wide8[2][2] = {{LRH_K(2, false, false, false, false), LRH_K(2, false, false, true, false)},
-			{LRH_K(2, false, true, false, false), LRH_K(2, false, true, true, false)}};
-	static const void *wide8Two[2][2] = {
-			{(const void *)&lrh_trace28_kernel<false, false>, (const void *)&lrh_trace2_kernel<2, false, true, false>},
-			{(const void *)&lrh_trace28_kernel<true, false>, (const void *)&lrh_trace2_kernel<2, true, true, false>}};
-	if (layout == 2) {
-		static const void *batched8[2][2] = {
-				{(const void *)&lrh_trace8b_kernel<false>, (const void *)&lrh_trace8b_kernel<true>},
-				{(const void *)&lrh_trace28_kernel<false, true>, (const void *)&lrh_trace28_kernel<true, true>}};
-		if (batch) return batched8[two ? 1 : 0][any ? 1 : 0];
-		return two ? wide8Two[any ? 1 : 0][count ? 1 : 0] : wide8[any ? 1 : 0][count ? 1 : 0];
+template <int L, bool A>
+static const void *kernelOf(bool two, bool count, bool batch, bool drain) {
+	if (batch) {
+		if (L == 2)
+			return two ? (const void *)&lrh_trace28_kernel<A, true> : (const void *)&lrh_trace8b_kernel<A>;
+		return two ? (const void *)&lrh_trace2_kernel<L == 2 ? 0 : L, A, false, true>
+				: (const void *)&lrh_trace_kernel<L == 2 ? 0 : L, A, false, true>;
 	}
-	static const void *plain[2][2][2][2] = {
-		{{{LRH_K(0, false, false, false, false), LRH_K(0, false, false, true, false)},
-		  {LRH_K(0, false, true, false, false), LRH_K(0, false, true, true, false)}},
-		 {{LRH_K(0, true, false, false, false), LRH_K(0, true, false, true, false)},
-		  {LRH_K(0, true, true, false, false), LRH_K(0, true, true, true, false)}}},
-		{{{LRH_K(1, false, false, false, false), LRH_K(1, false, false, true, false)},
-		  {LRH_K(1, false, true, false, false), LRH_K(1, false, true, true, false)}},
-		 {{LRH_K(1, true, false, false, false), LRH_K(1, true, false, true, false)},
-		  {LRH_K(1, true, true, false, false), LRH_K(1, true, true, true, false)}}}};
-	// batched: the query is per item, `any` says that some of the batch's are any-hit; COUNT is not offered
-	static const void *batched[2][2][2] = {
-		{{LRH_K(0, false, false, false, true), LRH_K(0, false, true, false, true)},
-		 {LRH_K(0, true, false, false, true), LRH_K(0, true, true, false, true)}},
-		{{LRH_K(1, false, false, false, true), LRH_K(1, false, true, false, true)},
-		 {LRH_K(1, true, false, false, true), LRH_K(1, true, true, false, true)}}};
-	if (batch) return batched[layout ? 1 : 0][two ? 1 : 0][any ? 1 : 0];
-	return plain[layout ? 1 : 0][two ? 1 : 0][any ? 1 : 0][count ? 1 : 0];
+	if (!two) return count ? (const void *)&lrh_trace_kernel<L, A, true, false> : (const void *)&lrh_trace_kernel<L, A, false, false>;
+	if (count) return (const void *)&lrh_trace2_kernel<L, A, true, false>;
+	if (drain) return (const void *)&lrh_trace2_drain_kernel<L, A>;
+	if (L == 0) return (const void *)&lrh_trace2q_kernel<A>;
+	if (L == 2) return (const void *)&lrh_trace28_kernel<A, false>;
+	return (const void *)&lrh_trace2_kernel<1, A, false, false>;
+}
+
+// `any` of a batch: some of its items are any-hit queries.  The counting
+// variants are not offered for batches and have no drain.
+static const void *kernelPtr(int layout, bool two, bool any, bool count, bool batch, bool drain) {
+	switch (layout * 2 + (any ? 1 : 0)) {
+	case 0: return kernelOf<0, false>(two, count, batch, drain);
+	case 1: return kernelOf<0, true>(two, count, batch, drain);
+	case 2: return kernelOf<1, false>(two, count, batch, drain);
+	case 3: return kernelOf<1, true>(two, count, batch, drain);
+	case 4: return kernelOf<2, false>(two, count, batch, drain);
+	case 5: return kernelOf<2, true>(two, count, batch, drain);
+	default: return nullptr;
+	}
 }
 
 hipError_t lrhLaunchReset(uint32_t *p, uint32_t n, hipStream_t s) {
@@ -870,17 +1185,17 @@ hipError_t lrhLaunchReset(uint32_t *p, uint32_t n, hipStream_t s) {
 	return hipGetLastError();
 }
 
-hipError_t lrhOccupancy(int layout, bool two, bool any, bool batch, int block, size_t lds,
+hipError_t lrhOccupancy(int layout, bool two, bool any, bool batch, bool drain, int block, size_t lds,
 		int *blocksPerCU) {
-	const void *k = kernelPtr(layout, two, any, false, batch);
+	const void *k = kernelPtr(layout, two, any, false, batch, drain);
 	if (!k) return hipErrorInvalidDeviceFunction;
 	return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocksPerCU, k, block, lds);
 }
 
-hipError_t lrhLaunchTrace(int layout, bool two, bool any, bool count, bool batch, dim3 grid, dim3 block,
+hipError_t lrhLaunchTrace(int layout, bool two, bool any, bool count, bool batch, bool drain, dim3 grid, dim3 block,
 		size_t lds, hipStream_t s, const LrhTraceParams &P) {
 	void *args[] = {(void *)&P};
-	const void *k = kernelPtr(layout, two, any, count, batch);
+	const void *k = kernelPtr(layout, two, any, count, batch, drain);
 	if (!k) return hipErrorInvalidDeviceFunction;
 	return hipLaunchKernel(k, grid, block, args, lds, s);
 }
