@@ -79,8 +79,8 @@ double now() {
 
 }  // namespace
 
-// Scratch memory of lrh_trace_noalloc: the ray-ticket counter (first 256
-// bytes) and the spill stack, in one statically sized array that every GPU
+// Scratch memory of lrh_trace_noalloc: the ray-ticket counters (first 2 KiB)
+// and the spill stack, in one statically sized array that every GPU
 // the library runs on holds from the loading of this code object until the
 // process ends.  In host code `scratch` is only the host-side stand-in of the
 // array; its device address on each GPU comes from hipGetSymbolAddress,
@@ -88,7 +88,8 @@ double now() {
 static __device__ __align__(256) unsigned char scratch[LRH_NOALLOC_SCRATCH_BYTES];
 
 namespace {
-constexpr size_t kScratchCounterBytes = 256;
+constexpr size_t kScratchCounterBytes = 2048;
+static_assert(LRH_COUNTER_WORDS * sizeof(uint32_t) <= kScratchCounterBytes, "counters precede the spill stack");
 constexpr int kMaxOrdinals = 64;
 std::mutex g_scratchMu;
 void *g_scratchPtr[kMaxOrdinals] = {};
@@ -126,7 +127,7 @@ struct lrh_device {
 	// per-stream trace workspace: ray-ticket counter + spill stack, so that
 	// traces issued on different streams never share scratch memory
 	struct Workspace {
-		uint32_t *counter = nullptr;      // [0] tickets, [1] finished blocks
+		uint32_t *counter = nullptr;      // LRH_COUNTER_WORDS
 		unsigned long long *stats = nullptr;
 		uint2 *spill = nullptr;
 		size_t spillBytes = 0;
@@ -673,7 +674,7 @@ int lrh_device_close(lrh_device *dev) {
 	for (lrh_scene *s : live) delete s;
 	for (auto &w : dev->ws) {
 		dev->devFree(w.second.spill, w.second.spillBytes);
-		dev->devFree(w.second.counter, 2 * sizeof(uint32_t));
+		dev->devFree(w.second.counter, LRH_COUNTER_WORDS * sizeof(uint32_t));
 		dev->devFree(w.second.stats, LRH_TRACE_STATS * sizeof(unsigned long long));
 		dev->devFree(w.second.table, w.second.tableBytes);
 	}
@@ -1306,17 +1307,14 @@ LaunchShape chooseShape(lrh_device *dev, unsigned layout, bool two, bool any, bo
 	if (sparse && need > persistent) L.waveRays = 64u;  // (a small grid was asked for)
 	L.blocks = std::max(1u, std::min(persistent, need));
 	// A refill costs a wave one LDS atomic and the wait for its rays, so waves
-	// are topped up early, and the earlier the more rays there are to come for
-	// a lane: towards the end the rays that start last decide.  Measured at
-	// thresholds 8 / 16 / 24 / 40: 700,001 bounce rays (1.5 per lane) 211 / 212 /
-	// 220 / 225 us, 2,073,600 (4.5) 544 / 505 / 497 / 503, camera rays (4.5) 391 /
-	// 393 / 397 / 393, 3,000,001 among spheres (6.5) 637 / 579 / 572 / 554, a batch
-	// of 3.9M (12) 1,061 / 982 / 941 / 900.  A two-level pass costs twice as much
-	// (object entries), so idle lanes do too: 4,194,304 rays over moving
-	// instances at 8 / 16 / 24 / 48 1,627 / 1,475 / 1,373 / 1,238.
-	const uint64_t perLane = count / ((uint64_t)L.blocks * L.block);
-	L.refill = (o && o->refillThreshold) ? std::min(64u, o->refillThreshold)
-			: two ? 48 : perLane >= 6 ? 40 : perLane >= 3 ? 24 : 16;
+	// are topped up early.  Measured at thresholds 8 / 16 / 40 / 56: bounce rays
+	// over 26.2M triangles 553 / 502 / 494 / 516 us, 700,001 over 2.1M 190 / 176 /
+	// 172 / 176, camera rays 366 / 354 / 354 / 357 (8-wide nodes 341 / 339 / 350 /
+	// 363), 3M among spheres 636 / 576 / 545 / 551, a batch of 3.9M 1,050 / 974 /
+	// 895 / 885.  A two-level pass costs twice as much (object entries), so idle
+	// lanes do too: 4,194,304 rays over moving instances at 8 / 16 / 40 / 48 1,630 /
+	// 1,473 / 1,250 / 1,242.
+	L.refill = (o && o->refillThreshold) ? std::min(64u, o->refillThreshold) : two ? 48 : 40;
 	// a visit pushes at most width - 1 entries
 	const unsigned worst = (layout == 2 ? 7u : 3u) * (maxDepth + 2u) + 4u;
 	L.spillDepth = worst > L.lds ? worst - L.lds : 1u;
@@ -1327,9 +1325,9 @@ lrh_device::Workspace &workspace(lrh_device *dev, hipStream_t st, size_t spillBy
 	std::lock_guard<std::mutex> g(dev->mu);
 	lrh_device::Workspace &w = dev->ws[st];
 	if (!w.counter) {
-		w.counter = (uint32_t *)dev->devAlloc(2 * sizeof(uint32_t));
+		w.counter = (uint32_t *)dev->devAlloc(LRH_COUNTER_WORDS * sizeof(uint32_t));
 		w.stats = (unsigned long long *)dev->devAlloc(LRH_TRACE_STATS * sizeof(unsigned long long));
-		HIPCHK(hipMemsetAsync(w.counter, 0, 2 * sizeof(uint32_t), st));
+		HIPCHK(hipMemsetAsync(w.counter, 0, LRH_COUNTER_WORDS * sizeof(uint32_t), st));
 	}
 	if (w.spillBytes < spillBytes) {
 		// the previous spill array may still be read by work queued on st
@@ -1552,7 +1550,7 @@ int lrh_trace_noalloc(lrh_scene *s, const void *rays, void *hits, unsigned int c
 		uint2 *spill = reinterpret_cast<uint2 *>(static_cast<unsigned char *>(dev->scratch) + kScratchCounterBytes);
 		// the ticket counters start at zero whatever the last call left (a fill
 		// kernel, not a memset node, so the call may be graph-captured)
-		HIPCHK(lrhLaunchReset(counter, 2, st));
+		HIPCHK(lrhLaunchReset(counter, LRH_COUNTER_WORDS, st));
 		LrhTraceParams P;
 		std::memset(&P, 0, sizeof(P));
 		fillSceneParams(P, s);
@@ -1590,11 +1588,11 @@ int lrh_batch_create(lrh_device *dev, const lrh_batch_item *items, unsigned int 
 		const unsigned nLanes = b->L.blocks * b->L.block;
 		b->descs.alloc(dev, b->T.descs.size() * sizeof(LrhBatchDesc));
 		b->starts.alloc(dev, b->T.starts.size() * sizeof(uint32_t));
-		b->counter.alloc(dev, 2 * sizeof(uint32_t));
+		b->counter.alloc(dev, LRH_COUNTER_WORDS * sizeof(uint32_t));
 		b->spill.alloc(dev, (size_t)nLanes * b->L.spillDepth * sizeof(uint2));
 		b->descs.upload(b->T.descs.data(), b->descs.bytes, dev->stream);
 		b->starts.upload(b->T.starts.data(), b->starts.bytes, dev->stream);
-		HIPCHK(hipMemsetAsync(b->counter.p, 0, 2 * sizeof(uint32_t), dev->stream));
+		HIPCHK(hipMemsetAsync(b->counter.p, 0, LRH_COUNTER_WORDS * sizeof(uint32_t), dev->stream));
 		HIPCHK(hipStreamSynchronize(dev->stream));
 		LrhTraceParams &P = b->P;
 		std::memset(&P, 0, sizeof(P));

@@ -10,6 +10,13 @@
 #define LRH_ITEM_ANY 1u
 #define LRH_ITEM_TWO 2u
 
+/* Counters of a launch, each on a 128-byte line of its own: ray tickets of
+ * each group of blocks, finished blocks of each group.  Blocks are dealt to
+ * the XCDs in turn, and to the groups alike. */
+#define LRH_COUNTER_STRIDE 32u
+#define LRH_GROUPS 8u
+#define LRH_COUNTER_WORDS (2u * LRH_GROUPS * LRH_COUNTER_STRIDE)
+
 /* One ray buffer of a batched launch, as the kernel reads it (96 bytes). */
 struct LrhBatchDesc {
 	const void *nodes;
@@ -39,7 +46,7 @@ struct LrhTraceParams {
 	lrh_hit_rec *hits;
 	uint32_t nRays;
 	uint32_t root;                  /* child reference of the (root) tree */
-	uint32_t *counter;              /* [0] ray tickets, [1] finished blocks; the last block rewinds both */
+	uint32_t *counter;              /* LRH_COUNTER_WORDS, zero between launches (the last blocks rewind them) */
 	uint2 *spill;                   /* spill stack: spillDepth entries x nLanes */
 	uint32_t spillDepth;
 	uint32_t nLanes;

@@ -342,22 +342,40 @@ DEVI uint2 pop(Stack &s) {
 }
 
 // ---- ray tickets ----
-// A launch hands out its first gridDim * blockDim rays by lane and the rest
-// through a counter in memory.  Atomics on one address from all eight XCDs
-// take 11.4 ns each (measured, whatever the number of waves), so a wave does
-// not go to the counter for each of its refills: a block takes a chunk and
-// its waves divide it through this pool in LDS (2,073,600 rays, one atomic
-// per refill and for every first ray -> this: camera rays 662 -> 425 us,
-// bounce rays over 26.2M triangles 716 -> 630 us).
+// A launch hands out its first rays by lane (waveRays to each wave) and the
+// rest through counters in memory.  Atomics on one address from all eight
+// XCDs take 11.4 ns each, whatever the number of waves, and when all waves
+// come at once, for their second ray or to learn that there is none, the last
+// waits 80 us; on eight addresses they take 1.9 ns.  So the blocks form eight
+// groups (blockIdx modulo eight, as they are dealt to the XCDs), each with a
+// counter of its own and every eighth unit of 256 rays, and a block's waves
+// go there for a chunk that they divide through a pool in LDS.
+// (2,073,600 rays, one counter and an atomic for each refill -> a pool -> and
+// eight counters: camera rays 662 -> 395 -> 368 us; 500,001 shadow rays 300 ->
+// 188 -> 140; 921,600 in a room 219 -> 145, a sixth of them live 200 -> 123.)
+constexpr uint32_t kUnit = 256u;
 struct TicketPool {
 	unsigned long long range;  // low half: next ticket, high half: end of the chunk
-	uint32_t fetching;         // a wave of the block is replacing the chunk
+	uint32_t fetching;         // 1: a wave of the block is replacing the chunk; 2: the counter is past the group's last
 };
 
 struct Tickets {
 	uint32_t b0, n0, b1, n1;  // n0 tickets from b0, then n1 from b1
 	bool exhausted;           // nothing is left in the counter (or, for this wave, in the pool)
 };
+
+// tickets of group g beyond the `first` rays handed out by lane (the last
+// unit may run past the launch's rays)
+DEVI uint32_t groupTickets(uint32_t g, uint32_t groups, uint32_t first, uint32_t nRays) {
+	if (first >= nRays) return 0u;
+	const uint32_t units = (nRays - first + kUnit - 1u) / kUnit;
+	return units > g ? (units - g + groups - 1u) / groups * kUnit : 0u;
+}
+
+// the ray of ticket x of group g
+DEVI uint32_t rayOf(uint32_t x, uint32_t g, uint32_t groups, uint32_t first) {
+	return first + ((x / kUnit) * groups + g) * kUnit + x % kUnit;
+}
 
 // takes up to n tickets from the pool: the first one in `base`
 DEVI uint32_t poolTake(TicketPool &pool, uint32_t n, uint32_t &base, uint32_t &end) {
@@ -375,36 +393,40 @@ DEVI uint32_t poolTake(TicketPool &pool, uint32_t n, uint32_t &base, uint32_t &e
 // while holding it, so no ticket is lost; nobody waits for it.  The chunk is
 // a share of what was left at the block's last visit, so that the launch
 // ends evenly: large reservations to the end cost 13%.  A wave stops asking
-// once the counter is past the last ray; a chunk it has not seen belongs to
-// the wave that took it, which asks again.
-DEVI Tickets takeTickets(TicketPool &pool, uint32_t *counter, uint32_t n, uint32_t nStatic, uint32_t nRays, uint32_t leader) {
+// once the counter is past the group's last ticket, and its block's other
+// waves with it; a chunk that a wave has not seen then belongs to the wave
+// that took it, which asks again.
+DEVI Tickets takeTickets(TicketPool &pool, uint32_t *counter, uint32_t n, uint32_t total, uint32_t blocks,
+		uint32_t leader) {
 	uint32_t b0 = 0, n0 = 0, b1 = 0, n1 = 0, over = 0;
 	if (__lane_id() == leader) {
 		uint32_t end;
 		n0 = poolTake(pool, n, b0, end);
-		uint32_t rest = n - n0;
+		const uint32_t rest = n - n0;
 		if (rest) {
-			uint32_t chunk = 0;
-			bool mine = __hip_atomic_exchange(&pool.fetching, 1u, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) == 0u;
+			uint32_t chunk = 0, held = 0u;
+			__hip_atomic_compare_exchange_strong(&pool.fetching, &held, 1u, __ATOMIC_ACQUIRE, __ATOMIC_RELAXED,
+					__HIP_MEMORY_SCOPE_WORKGROUP);
+			const bool mine = held == 0u;
+			over = held == 2u ? 1u : 0u;
 			if (mine) {
 				// another wave may have put a chunk there meanwhile
 				n1 = poolTake(pool, rest, b1, end);
-				const uint32_t left = nRays - (end > nStatic ? (end < nRays ? end : nRays) : nStatic);
-				chunk = left / gridDim.x;
+				chunk = (total - (end < total ? end : total)) / blocks;
 				chunk = chunk < 256u ? chunk : 256u;
 				if (chunk < 16u) chunk = 0;
 			}
-			if (n1 == 0) {
-				b1 = nStatic + atomicAdd(counter, rest + chunk);
+			if (n1 == 0 && !over) {
+				b1 = atomicAdd(counter, rest + chunk);
 				n1 = rest;
-				over = b1 + rest >= nRays ? 1u : 0u;
+				over = b1 + rest >= total ? 1u : 0u;
 				if (mine && chunk) {
-					const uint32_t a = b1 + rest, e = a + chunk < nRays ? a + chunk : nRays;
+					const uint32_t a = b1 + rest, e = a + chunk < total ? a + chunk : total;
 					__hip_atomic_store(&pool.range, ((unsigned long long)e << 32) | a, __ATOMIC_RELAXED,
 							__HIP_MEMORY_SCOPE_WORKGROUP);
 				}
 			}
-			if (mine) __hip_atomic_store(&pool.fetching, 0u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+			if (mine) __hip_atomic_store(&pool.fetching, over ? 2u : 0u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
 		}
 	}
 	Tickets t;
@@ -792,7 +814,12 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 	uint32_t hTri = LRH_NULL_INDEX, hMesh = LRH_NULL_INDEX, cur = LRH_CHILD_EMPTY, obj = 0, steps = 0;
 	float curT = 0.f;
 	bool inInst = false;
-	bool first = true, exhausted = nStatic >= P.nRays;
+	// (a grid of fewer blocks than groups is one group)
+	const uint32_t tGroups = gridDim.x < LRH_GROUPS ? 1u : LRH_GROUPS;
+	const uint32_t tGroup = blockIdx.x % tGroups, tBlocks = (gridDim.x - tGroup + tGroups - 1u) / tGroups;
+	const uint32_t tTotal = groupTickets(tGroup, tGroups, nStatic, P.nRays);
+	uint32_t *const tCounter = P.counter + tGroup * LRH_COUNTER_STRIDE;
+	bool first = true, exhausted = tTotal == 0;
 	// rays a wave hands to the drain (without one it goes on ray by lane)
 	constexpr uint32_t kDrainRays = !DRAIN ? 0u : LAYOUT == 2 ? 8u : 16u;
 	// COUNT variant only: per lane node tests / primitive tests / rays; per
@@ -817,11 +844,11 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 			const uint32_t nIdle = (uint32_t)__popcll(idle);
 			if (64u - nIdle < P.refill) {
 				if (COUNT) ++cRefill;
-				const Tickets tk = takeTickets(pool, P.counter, nIdle, nStatic, P.nRays, (uint32_t)__ffsll((long long)idle) - 1u);
+				const Tickets tk = takeTickets(pool, tCounter, nIdle, tTotal, tBlocks, (uint32_t)__ffsll((long long)idle) - 1u);
 				exhausted = tk.exhausted;
 				const uint32_t rank = (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
 				if (rid == kNoRay && rank < tk.n0 + tk.n1)
-					ticket = rank < tk.n0 ? tk.b0 + rank : tk.b1 + (rank - tk.n0);
+					ticket = rayOf(rank < tk.n0 ? tk.b0 + rank : tk.b1 + (rank - tk.n0), tGroup, tGroups, nStatic);
 			}
 		}
 		if (ticket < P.nRays) {
@@ -1085,16 +1112,16 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 			}
 		}
 	}
-	// the last block to finish rewinds the ticket counter for the next launch
-	// (a launch that never used it has nothing to rewind; every block's own
-	// additions to it have returned before its barrier)
-	if (nStatic >= P.nRays) return;
+	// the last block of a group to finish rewinds its counters for the next
+	// launch (a group that never used them has nothing to rewind; every block's
+	// own additions have returned before its barrier)
+	if (tTotal == 0) return;
 	__syncthreads();
 	if (threadIdx.x == 0) {
-		const uint32_t d = atomicAdd(P.counter + 1, 1u);
-		if (d == gridDim.x - 1) {
-			atomicExch(P.counter + 0, 0u);
-			atomicExch(P.counter + 1, 0u);
+		uint32_t *done = tCounter + LRH_GROUPS * LRH_COUNTER_STRIDE;
+		if (atomicAdd(done, 1u) == tBlocks - 1u) {
+			atomicExch(tCounter, 0u);
+			atomicExch(done, 0u);
 		}
 	}
 }

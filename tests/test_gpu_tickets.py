@@ -1,5 +1,6 @@
 """Ray tickets of a persistent launch: the first grid's worth by lane, the rest
-through each block's pool and the launch counter.  Every ray is traced exactly
+in units of 256 dealt to eight groups of blocks, each with a counter, and
+through each block's pool.  Every ray is traced exactly
 once whatever the count, grid and refill threshold: hits equal those of small
 traces that never use the counter, bit for bit, on repeated launches."""
 import numpy as np
@@ -30,9 +31,9 @@ def workload(gpu_device):
 
 
 # one block per CU = cu_count * block lanes; offsets from it in rays: the
-# remainders of waves, of blocks and of the pool's chunks (16 to 256 per block)
+# remainders of waves, of blocks, of units and of rounds of units
 @pytest.mark.parametrize("block", [64, 256])
-@pytest.mark.parametrize("offset", [-1, 0, 1, 63, 64, 65, 4095, 4096, 4097, 65537, 200001])
+@pytest.mark.parametrize("offset", [-1, 0, 1, 63, 64, 65, 255, 256, 257, 2047, 2048, 2049, 65537, 200001])
 @pytest.mark.parametrize("refill", [1, 16, 64])
 def test_every_ray_once(workload, block, offset, refill):
     dev, sc, rays, init, want = workload
