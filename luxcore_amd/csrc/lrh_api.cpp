@@ -196,8 +196,29 @@ struct lrh_device {
 		buildPool.emplace(bytes, p);
 		pooledBytes += bytes;
 	}
+	// pinned words for a build's readbacks, one block per build under way
+	std::vector<void *> pinPool;
+	void *pinTake() {
+		{
+			std::lock_guard<std::mutex> g(poolMu);
+			if (!pinPool.empty()) {
+				void *p = pinPool.back();
+				pinPool.pop_back();
+				return p;
+			}
+		}
+		void *p = nullptr;
+		HIPCHK(hipHostMalloc(&p, LRH_BUILD_PINNED, hipHostMallocDefault));
+		return p;
+	}
+	void pinGive(void *p) {
+		std::lock_guard<std::mutex> g(poolMu);
+		pinPool.push_back(p);
+	}
 	void drainPool() {
 		std::lock_guard<std::mutex> g(poolMu);
+		for (void *p : pinPool) (void)hipHostFree(p);
+		pinPool.clear();
 		for (auto &b : buildPool) devFree(b.second, b.first);
 		buildPool.clear();
 		pooledBytes = 0;
@@ -837,6 +858,8 @@ namespace {
 
 void *gbAlloc(void *ctx, size_t bytes) { return static_cast<lrh_device *>(ctx)->buildAlloc(bytes); }
 void gbRelease(void *ctx, void *p, size_t bytes) { static_cast<lrh_device *>(ctx)->buildRelease(p, bytes); }
+void *gbPinned(void *ctx) { return static_cast<lrh_device *>(ctx)->pinTake(); }
+void gbUnpin(void *ctx, void *p) { static_cast<lrh_device *>(ctx)->pinGive(p); }
 
 // single-level scene built on the device (LRH_BUILD_DEVICE_LBVH / _PLOC):
 // vertices and triangles are uploaded mesh by mesh, the tree and the records
@@ -891,7 +914,7 @@ void deviceBuild(lrh_scene *s, const lrh_mesh *meshes, unsigned nMeshes, unsigne
 	in.layout = s->layout;
 	in.method = builder == LRH_BUILD_DEVICE_PLOC ? 1u : 0u;
 	in.travCost = s->params.travCost;
-	LrhGpuAlloc a{gbAlloc, gbRelease, dev};
+	LrhGpuAlloc a{gbAlloc, gbRelease, gbPinned, gbUnpin, dev};
 	LrhGpuBuildOut out;
 	try {
 		lrhGpuBuildBVH(in, a, dev->stream, &out);

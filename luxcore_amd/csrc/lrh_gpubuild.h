@@ -13,9 +13,13 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#define LRH_BUILD_PINNED 4096
+
 struct LrhGpuAlloc {
 	void *(*alloc)(void *ctx, size_t bytes);  // throws on failure
 	void (*release)(void *ctx, void *p, size_t bytes);
+	void *(*pinned)(void *ctx);  // LRH_BUILD_PINNED bytes of pinned host memory for one build; throws on failure
+	void (*unpin)(void *ctx, void *p);
 	void *ctx;
 };
 

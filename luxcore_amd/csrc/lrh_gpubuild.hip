@@ -5,19 +5,20 @@
  *   1. leaf boxes and the bounds of their centres;
  *   2. 63-bit Morton codes over a cube of cells, sorted with the triangle id
  *      as value by a stable LSD radix sort (8-bit digits: per-tile digit
- *      counts, one exclusive scan of the [digit][tile] table, a scatter that
- *      ranks equal digits in index order with wave ballots, stages the tile
- *      in LDS in sorted order and writes each digit's run coalesced), then
- *      checked to be in order;
+ *      counts, an exclusive scan of each digit's row of the [digit][tile]
+ *      table, a scatter that ranks equal digits in index order with wave
+ *      ballots, stages the tile in LDS in sorted order and writes each digit's
+ *      run coalesced), then checked to be in order;
  *   3. a binary tree over the sorted leaves: the radix tree (LBVH) or
  *      agglomerative clustering in rounds of mutual nearest neighbours
  *      within 16 places (PLOC), brought into the radix tree's form;
- *   4. boxes bottom-up -- LBVH: one launch per depth (depths by pointer
- *      jumping, nodes ordered by depth); PLOC: one launch per round -- and
- *      surface-area costs, which decide whether a node of at most maxLeaf
- *      triangles becomes one leaf;
+ *   4. boxes bottom-up -- LBVH: nodes ordered by the length of their common
+ *      prefix, a launch per length (runs of short ones in one block); PLOC: as
+ *      the clusters merge -- and surface-area costs, which decide whether a
+ *      node of at most maxLeaf triangles becomes one leaf;
  *   5. breadth-first collapse into 4- or 8-wide nodes, child slots from an
- *      exclusive scan, so the node order is deterministic;
+ *      exclusive scan, so the node order is deterministic; level sizes stay on
+ *      the device, the host looks at them once per few levels;
  *   6. triangle records in leaf order, bit for bit the host records.
  * Every kernel runs a bounded amount of work: no block waits on another
  * (the sort and the scans are sequences of kernels, not decoupled
@@ -27,9 +28,11 @@
  */
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "lrh_devnode.h"
@@ -139,41 +142,47 @@ __global__ __launch_bounds__(kSortBlock) void k_sortCount(const uint64_t *keys, 
 // order, so consecutive threads write consecutive addresses of one digit's
 // run (its global start from the scanned [digit][tile] table). ----
 __global__ __launch_bounds__(kSortBlock) void k_sortScatter(const uint64_t *keysIn, const uint32_t *valsIn, uint32_t n,
-		uint32_t shift, uint32_t nTiles, const uint32_t *offsets, uint64_t *keysOut, uint32_t *valsOut, uint32_t *err) {
+		uint32_t shift, uint32_t nTiles, const uint32_t *offsets, const uint32_t *totals, uint64_t *keysOut,
+		uint32_t *valsOut, uint32_t *err) {
 	constexpr uint32_t kWaves = kSortBlock / 64;
 	__shared__ uint32_t run[256];
 	__shared__ uint32_t wcnt[kWaves][256];
 	__shared__ uint32_t off[256];    // global start of each digit's run for this tile
 	__shared__ uint32_t start[256];  // each digit's start within the tile
+	__shared__ uint32_t base[256];   // each digit's start in the whole output
 	__shared__ uint64_t sKey[kSortTile];
 	__shared__ uint32_t sVal[kSortTile];
 	const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
-	const uint64_t base = (uint64_t)blockIdx.x * kSortTile;
-	const uint32_t tileN = (uint32_t)((n - base) < kSortTile ? (n - base) : kSortTile);
+	const uint64_t tile0 = (uint64_t)blockIdx.x * kSortTile;
+	const uint32_t tileN = (uint32_t)((n - tile0) < kSortTile ? (n - tile0) : kSortTile);
 	// the tile's digit counts, scanned to starts
 	run[tid] = 0;
 	for (uint32_t w = 0; w < kWaves; ++w) wcnt[w][tid] = 0;
 	off[tid] = offsets[(size_t)tid * nTiles + blockIdx.x];
+	const uint32_t total = totals[tid];
+	base[tid] = total;
 	__syncthreads();
-	for (uint32_t j = tid; j < tileN; j += kSortBlock) atomicAdd(&run[digitOf(keysIn[base + j], shift)], 1u);
+	for (uint32_t j = tid; j < tileN; j += kSortBlock) atomicAdd(&run[digitOf(keysIn[tile0 + j], shift)], 1u);
 	__syncthreads();
 	start[tid] = run[tid];
 	__syncthreads();
-	for (uint32_t o = 1; o < 256; o <<= 1) {  // inclusive scan (Hillis-Steele)
-		const uint32_t add = tid >= o ? start[tid - o] : 0u;
+	for (uint32_t o = 1; o < 256; o <<= 1) {  // inclusive scans (Hillis-Steele)
+		const uint32_t add = tid >= o ? start[tid - o] : 0u, add2 = tid >= o ? base[tid - o] : 0u;
 		__syncthreads();
 		start[tid] += add;
+		base[tid] += add2;
 		__syncthreads();
 	}
 	start[tid] -= run[tid];  // exclusive
+	off[tid] += base[tid] - total;
 	run[tid] = 0;
 	__syncthreads();
 	const uint64_t lanesBelow = (1ull << lane) - 1ull;
 	for (uint32_t r = 0; r < kSortTile / kSortBlock; ++r) {
 		const uint32_t j = r * kSortBlock + tid;
 		const bool valid = j < tileN;
-		const uint64_t key = valid ? keysIn[base + j] : 0ull;
-		const uint32_t val = valid ? valsIn[base + j] : 0u;
+		const uint64_t key = valid ? keysIn[tile0 + j] : 0ull;
+		const uint32_t val = valid ? valsIn[tile0 + j] : 0u;
 		const uint32_t dg = valid ? digitOf(key, shift) : 0u;
 		uint64_t same = __ballot(valid);
 		for (uint32_t b = 0; b < 8; ++b) {
@@ -219,38 +228,90 @@ __global__ __launch_bounds__(kSortBlock) void k_sortScatter(const uint64_t *keys
 	}
 }
 
-// ---- exclusive scan of uint32 values: per-tile scans, then the tile
-// totals scanned the same way, then added ----
-__global__ __launch_bounds__(256) void k_scanTile(const uint32_t *in, uint32_t *out, uint32_t n, uint32_t *tileSums) {
-	constexpr uint32_t kPer = kScanTile / 256;
+// exclusive scan of each digit's row of the [digit][tile] table, a block per
+// digit, and the row's total; the scatter adds the digits' starts, so a pass
+// is three launches (five when the whole table was scanned as one array)
+__global__ __launch_bounds__(256) void k_scanRows(uint32_t *table, uint32_t nTiles, uint32_t *totals) {
+	constexpr uint32_t kPer = 8;
 	__shared__ uint32_t part[256];
-	const uint64_t base = (uint64_t)blockIdx.x * kScanTile + (uint64_t)threadIdx.x * kPer;
-	uint32_t v[kPer];
-	uint32_t sum = 0;
-	for (uint32_t k = 0; k < kPer; ++k) {
-		v[k] = (base + k < n) ? in[base + k] : 0u;
-		sum += v[k];
-	}
-	part[threadIdx.x] = sum;
-	__syncthreads();
-	// inclusive scan of the 256 partial sums (Hillis-Steele)
-	for (uint32_t o = 1; o < 256; o <<= 1) {
-		const uint32_t add = threadIdx.x >= o ? part[threadIdx.x - o] : 0u;
+	uint32_t *row = table + (size_t)blockIdx.x * nTiles;
+	uint32_t carry = 0;
+	for (uint32_t t0 = 0; t0 < nTiles; t0 += 256 * kPer) {
+		const uint32_t b = t0 + threadIdx.x * kPer;
+		uint32_t v[kPer], sum = 0;
+		for (uint32_t k = 0; k < kPer; ++k) {
+			v[k] = b + k < nTiles ? row[b + k] : 0u;
+			sum += v[k];
+		}
+		part[threadIdx.x] = sum;
 		__syncthreads();
-		part[threadIdx.x] += add;
+		for (uint32_t o = 1; o < 256; o <<= 1) {
+			const uint32_t add = threadIdx.x >= o ? part[threadIdx.x - o] : 0u;
+			__syncthreads();
+			part[threadIdx.x] += add;
+			__syncthreads();
+		}
+		uint32_t run = carry + part[threadIdx.x] - sum;
+		for (uint32_t k = 0; k < kPer; ++k) {
+			if (b + k < nTiles) row[b + k] = run;
+			run += v[k];
+		}
+		carry += part[255];
 		__syncthreads();
 	}
-	uint32_t run = part[threadIdx.x] - sum;
-	for (uint32_t k = 0; k < kPer; ++k) {
-		if (base + k < n) out[base + k] = run;
-		run += v[k];
-	}
-	if (threadIdx.x == 255) tileSums[blockIdx.x] = part[255];
+	if (threadIdx.x == 0) totals[blockIdx.x] = carry;
 }
 
-__global__ void k_scanAdd(uint32_t *out, uint32_t n, const uint32_t *tileOffsets) {
-	const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i < n) out[i] += tileOffsets[i / kScanTile];
+// exclusive prefix of v over the 256 threads of a block; `sum` gets the total
+__device__ __forceinline__ uint32_t blockPrefix(uint32_t v, uint32_t *lds /* 4 */, uint32_t &sum) {
+	uint32_t incl = v;
+	for (int o = 1; o < 64; o <<= 1) {
+		const uint32_t x = (uint32_t)__shfl_up((int)incl, o);
+		if ((int)(threadIdx.x & 63u) >= o) incl += x;
+	}
+	if ((threadIdx.x & 63u) == 63u) lds[threadIdx.x >> 6] = incl;
+	__syncthreads();
+	uint32_t before = 0;
+	sum = 0;
+	for (uint32_t w = 0; w < 4; ++w) {
+		if (w < (threadIdx.x >> 6)) before += lds[w];
+		sum += lds[w];
+	}
+	return before + incl - v;
+}
+
+// exclusive scan of n values in place by one block of 1024 threads, eight
+// values a thread and turn; returns the total to every thread
+__device__ uint32_t scanByBlock(uint32_t *v, uint32_t n, uint32_t *lds /* 16 */) {
+	constexpr uint32_t kPer = 8;
+	uint32_t carry = 0;
+	for (uint32_t t0 = 0; t0 < n; t0 += 1024 * kPer) {
+		const uint32_t b = t0 + threadIdx.x * kPer;
+		uint32_t x[kPer], sum = 0;
+		for (uint32_t k = 0; k < kPer; ++k) {
+			x[k] = b + k < n ? v[b + k] : 0u;
+			sum += x[k];
+		}
+		uint32_t incl = sum;
+		for (int o = 1; o < 64; o <<= 1) {
+			const uint32_t y = (uint32_t)__shfl_up((int)incl, o);
+			if ((int)(threadIdx.x & 63u) >= o) incl += y;
+		}
+		if ((threadIdx.x & 63u) == 63u) lds[threadIdx.x >> 6] = incl;
+		__syncthreads();
+		uint32_t run = carry + incl - sum, all = 0;
+		for (uint32_t w = 0; w < 16; ++w) {
+			if (w < (threadIdx.x >> 6)) run += lds[w];
+			all += lds[w];
+		}
+		for (uint32_t k = 0; k < kPer; ++k) {
+			if (b + k < n) v[b + k] = run;
+			run += x[k];
+		}
+		carry += all;
+		__syncthreads();
+	}
+	return carry;
 }
 
 __global__ void k_checkSorted(const uint64_t *keys, uint32_t n, uint32_t *err) {
@@ -258,66 +319,46 @@ __global__ void k_checkSorted(const uint64_t *keys, uint32_t n, uint32_t *err) {
 	if (i + 1 < n && keys[i] > keys[i + 1]) atomicOr(err, kErrUnsorted);
 }
 
-// 3. binary radix tree
+// 3. binary radix tree.  digits: 127 - the length of the node's common prefix
+// (at most 64 key bits and 32 of position), so a node's children have smaller
+// digits than it.  A node without a key range (codes out of order) sets the
+// error and becomes two leaves, so that nothing after it reads out of bounds
+// before the host sees the error.
+constexpr uint32_t kDigits = 128;
 __global__ void k_radixTree(const uint64_t *keys, uint32_t n, uint32_t *left, uint32_t *right, uint32_t *first,
-		uint32_t *last, uint32_t *iparent, uint32_t *err) {
+		uint32_t *last, uint64_t *digits, uint32_t *ids, uint32_t *err) {
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
 	if (i + 1 >= n) return;
 	uint32_t lc, rc, lo, hi;
 	if (!radixNode(keys, n, i, lc, rc, lo, hi)) {
 		atomicOr(err, kErrRange);
-		return;
+		lc = kLeafBit | i;
+		rc = kLeafBit | (i + 1);
+		lo = i;
+		hi = i + 1;
 	}
 	left[i] = lc;
 	right[i] = rc;
 	first[i] = lo;
 	last[i] = hi;
-	if (!(lc & kLeafBit)) iparent[lc] = i;
-	if (!(rc & kLeafBit)) iparent[rc] = i;
+	const int d = delta(keys, n, lo, hi);
+	digits[i] = (uint64_t)(kDigits - 1u - (uint32_t)(d < 0 ? 0 : d > 127 ? 127 : d));
+	ids[i] = i;
 }
 
-// 4. node depths by pointer jumping: after round r every node knows its
-// distance to the root if that is below 2^(r+1), and jump[x] is its ancestor
-// 2^(r+1) levels up, or the root
-__global__ void k_depthInit(const uint32_t *iparent, uint32_t ni, uint32_t *depth, uint32_t *jump) {
-	const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
-	if (x >= ni) return;
-	const uint32_t p = iparent[x];
-	depth[x] = (x == 0 || p >= ni) ? 0u : 1u;
-	jump[x] = (x == 0 || p >= ni) ? 0u : p;
-}
-
-__global__ void k_depthJump(uint32_t ni, const uint32_t *depth, const uint32_t *jump, uint32_t *depth2,
-		uint32_t *jump2) {
-	const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
-	if (x >= ni) return;
-	const uint32_t j = jump[x];
-	depth2[x] = depth[x] + depth[j];
-	jump2[x] = jump[j];
-}
-
-// a node not yet at the root after the doublings, or deeper than any valid
-// tree: an error
-constexpr uint32_t kMaxDepth = 128;
-__global__ void k_depthCheck(uint32_t ni, const uint32_t *depth, const uint32_t *jump, uint32_t *err) {
-	const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
-	if (x < ni && (jump[x] != 0 || depth[x] >= kMaxDepth)) atomicOr(err, kErrClimb);
-}
-
-// the first place of each depth (digit) in the sorted order: the scanned
-// digit table's entry of the first tile; out[kMaxDepth] counts the nodes
-// of depth below kMaxDepth
-__global__ void k_digitStarts(const uint32_t *table, uint32_t tiles, uint32_t *out) {
+// 4. the first place of each digit in the sorted order
+__global__ void k_digitStarts(const uint32_t *totals, uint32_t *out, uint32_t *host) {
+	__shared__ uint32_t v[256];
 	const uint32_t d = threadIdx.x;
-	if (d <= kMaxDepth) out[d] = table[(size_t)d * tiles];
-}
-
-// sort keys (depths) and values (node ids) for the counting sort by depth
-__global__ void k_depthKeys(uint32_t ni, const uint32_t *depth, uint64_t *keys, uint32_t *ids) {
-	const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
-	if (x >= ni) return;
-	keys[x] = depth[x];
-	ids[x] = x;
+	v[d] = totals[d];
+	__syncthreads();
+	for (uint32_t o = 1; o < 256; o <<= 1) {
+		const uint32_t add = d >= o ? v[d - o] : 0u;
+		__syncthreads();
+		v[d] += add;
+		__syncthreads();
+	}
+	if (d <= kDigits) out[d] = host[d] = v[d] - totals[d];
 }
 
 __global__ void k_leafBoxes(const GBox *boxes, const uint32_t *vals, uint32_t n, GBox *leafBox) {
@@ -325,14 +366,17 @@ __global__ void k_leafBoxes(const GBox *boxes, const uint32_t *vals, uint32_t n,
 	if (j < n) leafBox[j] = boxes[vals[j]];
 }
 
-// boxes and surface-area costs of the nodes of one depth, deepest level
-// first: the children's are the previous launch's
-__global__ void k_boxLevel(const uint32_t *order, uint32_t cnt, const uint32_t *left, const uint32_t *right,
-		const uint32_t *first, const uint32_t *last, const GBox *leafBox, uint32_t maxLeaf, float ci, GBox *nodeBox,
-		float *cost, uint32_t *leafOK) {
-	const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-	if (e >= cnt) return;
-	const uint32_t x = order[e], l = left[x], r = right[x];
+// what the collapse compares: a node's area, or -1 if it becomes a leaf (an
+// area is zero or more, but for boxes of NaN vertices, which may come out
+// inverted and must not read as a leaf)
+__device__ __forceinline__ float nodeKey(uint32_t leaf, float area) {
+	return leaf ? -1.f : area == -1.f ? 0.f : area;
+}
+
+// box, surface-area cost and leaf decision of node x
+__device__ __forceinline__ void boxNode(uint32_t x, const uint32_t *left, const uint32_t *right, const uint32_t *first,
+		const uint32_t *last, const GBox *leafBox, uint32_t maxLeaf, float ci, GBox *nodeBox, float *cost, float *key) {
+	const uint32_t l = left[x], r = right[x];
 	const GBox a = (l & kLeafBit) ? leafBox[l & ~kLeafBit] : nodeBox[l];
 	const GBox b = (r & kLeafBit) ? leafBox[r & ~kLeafBit] : nodeBox[r];
 	const GBox u = unionBox(a, b);
@@ -340,14 +384,38 @@ __global__ void k_boxLevel(const uint32_t *order, uint32_t cnt, const uint32_t *
 	const float cr = (r & kLeafBit) ? areaOf(b) : cost[r];
 	uint32_t lf;
 	cost[x] = nodeCost(areaOf(u), cl, cr, last[x] - first[x] + 1u, maxLeaf, ci, lf);
-	leafOK[x] = lf;
+	key[x] = nodeKey(lf, areaOf(u));
 	nodeBox[x] = u;
 }
 
+// the nodes of one digit: the children's are done by earlier launches
+__global__ void k_boxLevel(const uint32_t *order, uint32_t cnt, const uint32_t *left, const uint32_t *right,
+		const uint32_t *first, const uint32_t *last, const GBox *leafBox, uint32_t maxLeaf, float ci, GBox *nodeBox,
+		float *cost, float *key) {
+	const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
+	if (e < cnt) boxNode(order[e], left, right, first, last, leafBox, maxLeaf, ci, nodeBox, cost, key);
+}
+
+// the nodes of digits [d0, d1), each a few, by one block with a barrier after
+// each digit: a launch per digit of a handful of nodes costs its launch (a
+// 2.3M-triangle tree has 50 digits, half of them below 2,048 nodes)
+constexpr uint32_t kSmallLevel = 2048;
+__global__ __launch_bounds__(1024) void k_boxSmallLevels(const uint32_t *order, const uint32_t *starts, uint32_t d0,
+		uint32_t d1, const uint32_t *left, const uint32_t *right, const uint32_t *first, const uint32_t *last,
+		const GBox *leafBox, uint32_t maxLeaf, float ci, GBox *nodeBox, float *cost, float *key) {
+	for (uint32_t d = d0; d < d1; ++d) {
+		for (uint32_t e = starts[d] + threadIdx.x; e < starts[d + 1]; e += 1024)
+			boxNode(order[e], left, right, first, last, leafBox, maxLeaf, ci, nodeBox, cost, key);
+		__syncthreads();
+	}
+}
+
 // 3'. clustering (PLOC): clusters start as the sorted leaves
+struct PlocState;
 __global__ void k_plocInit(const GBox *boxes, const uint32_t *vals, uint32_t n, uint32_t *cid, GBox *cbox,
-		GBox *leafBox) {
+		GBox *leafBox, PlocState *st) {
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (i < 4) reinterpret_cast<uint32_t *>(st)[i] = i == 0 ? n : 0u;
 	if (i >= n) return;
 	const GBox b = boxes[vals[i]];
 	leafBox[i] = b;
@@ -355,13 +423,36 @@ __global__ void k_plocInit(const GBox *boxes, const uint32_t *vals, uint32_t n, 
 	cbox[i] = b;
 }
 
+// a round's state, written by the round before: clusters, next node, whether
+// the round pairs places 2k, 2k+1 (one that merged fewer than 1/64 of the
+// clusters is followed by such a forced round)
+struct PlocState {
+	uint32_t nc, nodeBase, forced, pad;
+};
+
+// clusters of at most this many are finished by one block
+constexpr uint32_t kPlocTail = 2048;
+constexpr uint32_t kPlocMaxRounds = 4096;
+
+// the kernels of a round run on an upper bound of clusters that the host
+// knows; the state's count ends them, and a count at or below kPlocTail
+// leaves the rest to the tail
+__device__ __forceinline__ PlocState plocRound(const PlocState *st, uint32_t r) {
+	PlocState s = st[r];
+	if (s.nc <= kPlocTail) s.nc = 0;
+	return s;
+}
+
 // nearest neighbours of a tile of 256 clusters, their boxes and the
 // kPlocRadius on either side staged in LDS (each box is read by 2r+1 threads)
 constexpr uint32_t kPlocTile = 256;
-__global__ __launch_bounds__(kPlocTile) void k_plocNearest(const GBox *cbox, uint32_t nc, uint32_t *nn) {
+__global__ __launch_bounds__(kPlocTile) void k_plocNearest(const GBox *cbox, const PlocState *st, uint32_t r, uint32_t *nn) {
 	constexpr uint32_t kSpan = kPlocTile + 2 * kPlocRadius;
 	__shared__ float tile[kSpan * 6];
 	const uint32_t t0 = blockIdx.x * kPlocTile;
+	const PlocState s = plocRound(st, r);
+	const uint32_t nc = s.forced ? 0u : s.nc;
+	if (t0 >= nc) return;
 	const int64_t base = (int64_t)t0 - kPlocRadius;  // cluster of tile entry 0
 	const float *src = reinterpret_cast<const float *>(cbox);
 	for (uint32_t k = threadIdx.x; k < kSpan * 6; k += kPlocTile) {
@@ -375,35 +466,89 @@ __global__ __launch_bounds__(kPlocTile) void k_plocNearest(const GBox *cbox, uin
 	nn[i] = plocNearestAt([&](uint32_t j) -> const GBox & { return lds[(int64_t)j - base]; }, nc, i, kPlocRadius);
 }
 
-// lead: the lower place of a merging pair (a new node); keep: the place
-// survives the round
-__global__ void k_plocFlags(const uint32_t *nn, uint32_t nc, uint32_t forced, uint32_t *lead, uint32_t *keep) {
-	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i > nc) return;
-	if (i == nc) {  // the scan's total slot
-		lead[i] = 0;
-		keep[i] = 0;
-		return;
+// partners and each cluster's place among the survivors and among the new
+// nodes, within its block: lead (the lower place of a pair, a new node) counts
+// in the upper half, keep (the place survives) in the lower
+__global__ __launch_bounds__(256) void k_plocMark(const uint32_t *nn, const PlocState *st, uint32_t r, uint32_t *prefix,
+		uint32_t *leadSums, uint32_t *keepSums) {
+	const PlocState s = plocRound(st, r);
+	if (blockIdx.x * 256u >= s.nc) return;
+	__shared__ uint32_t lds[4];
+	const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+	uint32_t v = 0;
+	if (i < s.nc) {
+		const uint32_t j = plocPartner(nn, s.nc, i, s.forced != 0);
+		v = (j != kNone && i < j ? 0x10000u : 0u) + (j != kNone && i > j ? 0u : 1u);
 	}
-	const uint32_t j = plocPartner(nn, nc, i, forced != 0);
-	lead[i] = (j != kNone && i < j) ? 1u : 0u;
-	keep[i] = (j != kNone && i > j) ? 0u : 1u;
+	uint32_t sum;
+	const uint32_t p = blockPrefix(v, lds, sum);
+	if (i < s.nc) prefix[i] = p;
+	if (threadIdx.x == 0) {
+		leadSums[blockIdx.x] = sum >> 16;
+		keepSums[blockIdx.x] = sum & 0xffffu;
+	}
 }
 
-__global__ void k_plocApply(const uint32_t *nn, uint32_t nc, uint32_t forced, const uint32_t *cid, const GBox *cbox,
-		const uint32_t *leadOff, const uint32_t *keepOff, uint32_t nodeBase, uint32_t *outCid, GBox *outBox,
-		uint32_t *left, uint32_t *right, GBox *nodeBox) {
-	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= nc) return;
-	const uint32_t j = plocPartner(nn, nc, i, forced != 0);
+// block sums to block starts, and the next round's state
+__global__ __launch_bounds__(1024) void k_plocScan(uint32_t *leadSums, uint32_t *keepSums, PlocState *st, uint32_t r,
+		uint32_t ni, uint32_t *err) {
+	__shared__ uint32_t lds[16];
+	const PlocState s = plocRound(st, r);
+	if (s.nc == 0) {
+		if (threadIdx.x == 0) st[r + 1] = st[r];
+		return;
+	}
+	const uint32_t nb = (s.nc + 255u) / 256u;
+	const uint32_t merged = scanByBlock(leadSums, nb, lds);
+	const uint32_t kept = scanByBlock(keepSums, nb, lds);
+	if (threadIdx.x == 0) {
+		PlocState t = {kept, s.nodeBase + merged, !s.forced && (uint64_t)merged * 64u < s.nc ? 1u : 0u, 0u};
+		if (merged == 0 || merged > s.nc / 2 || kept != s.nc - merged || t.nodeBase > ni) {
+			atomicOr(err, kErrCluster);
+			t = {0u, s.nodeBase, 0u, 0u};
+		}
+		st[r + 1] = t;
+	}
+}
+
+// the arrays of the clustering's binary tree (nodes in the order they are made)
+struct PlocTree {
+	uint32_t *left, *right, *count;
+	GBox *box;
+	float *cost, *key;
+	const GBox *leafBox;
+	uint32_t maxLeaf;
+	float ci;
+};
+
+// node x of children l and r (older nodes or leaves): box, leaves, cost and
+// leaf decision
+__device__ __forceinline__ void plocMake(const PlocTree &T, uint32_t x, uint32_t l, uint32_t r, const GBox &u) {
+	const uint32_t c = plocSize(l, T.count) + plocSize(r, T.count);
+	const float cl = (l & kLeafBit) ? areaOf(T.leafBox[l & ~kLeafBit]) : T.cost[l];
+	const float cr = (r & kLeafBit) ? areaOf(T.leafBox[r & ~kLeafBit]) : T.cost[r];
+	uint32_t lf;
+	T.left[x] = l;
+	T.right[x] = r;
+	T.box[x] = u;
+	T.count[x] = c;
+	T.cost[x] = nodeCost(areaOf(u), cl, cr, c, T.maxLeaf, T.ci, lf);
+	T.key[x] = nodeKey(lf, areaOf(u));
+}
+
+__global__ __launch_bounds__(256) void k_plocApply(const uint32_t *nn, const PlocState *st, uint32_t r,
+		const uint32_t *cid, const GBox *cbox, const uint32_t *prefix, const uint32_t *leadSums,
+		const uint32_t *keepSums, uint32_t ni, uint32_t *outCid, GBox *outBox, PlocTree T) {
+	const PlocState s = plocRound(st, r);
+	const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+	if (i >= s.nc || st[r + 1].nc == 0) return;
+	const uint32_t j = plocPartner(nn, s.nc, i, s.forced != 0);
 	if (j != kNone && i > j) return;  // merged into its lower partner
-	const uint32_t o = keepOff[i];
+	const uint32_t o = keepSums[blockIdx.x] + (prefix[i] & 0xffffu);
 	if (j != kNone) {
-		const uint32_t node = nodeBase + leadOff[i];
+		const uint32_t node = s.nodeBase + leadSums[blockIdx.x] + (prefix[i] >> 16);
 		const GBox u = unionBox(cbox[i], cbox[j]);
-		left[node] = cid[i];
-		right[node] = cid[j];
-		nodeBox[node] = u;
+		if (node < ni) plocMake(T, node, cid[i], cid[j], u);
 		outCid[o] = node;
 		outBox[o] = u;
 	} else {
@@ -412,41 +557,131 @@ __global__ void k_plocApply(const uint32_t *nn, uint32_t nc, uint32_t forced, co
 	}
 }
 
-// leaves per subtree and surface-area costs, the nodes of one round (their
-// children are older)
-__global__ void k_plocCount(uint32_t b, uint32_t e, const uint32_t *left, const uint32_t *right,
-		const GBox *leafBox, const GBox *nodeBox, uint32_t maxLeaf, float ci, uint32_t *count, float *cost,
-		uint32_t *leafOK) {
-	const uint32_t x = b + blockIdx.x * blockDim.x + threadIdx.x;
-	if (x >= e) return;
-	const uint32_t l = left[x], r = right[x];
-	const uint32_t c = plocSize(l, count) + plocSize(r, count);
-	count[x] = c;
-	const float cl = (l & kLeafBit) ? areaOf(leafBox[l & ~kLeafBit]) : cost[l];
-	const float cr = (r & kLeafBit) ? areaOf(leafBox[r & ~kLeafBit]) : cost[r];
-	uint32_t lf;
-	cost[x] = nodeCost(areaOf(nodeBox[x]), cl, cr, c, maxLeaf, ci, lf);
-	leafOK[x] = lf;
+// The last kPlocTail clusters by one block, all their rounds in LDS with
+// barriers: 46 rounds of a 50,000-triangle mesh were 46 times six launches
+// and a wait for the host, most of them for a few hundred clusters.  Each
+// thread has two clusters; a round is the one of the kernels above.
+__global__ __launch_bounds__(1024) void k_plocTail(PlocState *st, uint32_t r0, uint32_t ni, const uint32_t *cidIn,
+		const GBox *cboxIn, PlocTree T, uint32_t *rounds, uint32_t *err) {
+	__shared__ GBox box[kPlocTail];
+	__shared__ uint32_t cid[kPlocTail], nn[kPlocTail];
+	__shared__ uint32_t wsum[16];
+	PlocState s = st[r0];
+	uint32_t r = r0;
+	if (s.nc > kPlocTail) {
+		if (threadIdx.x == 0) atomicOr(err, kErrCluster);
+		return;
+	}
+	for (uint32_t i = threadIdx.x; i < s.nc; i += 1024) {
+		box[i] = cboxIn[i];
+		cid[i] = cidIn[i];
+	}
+	__syncthreads();
+	const uint32_t i0 = 2u * threadIdx.x;
+	while (s.nc > 1 && r < kPlocMaxRounds) {
+		if (!s.forced)
+			for (uint32_t i = threadIdx.x; i < s.nc; i += 1024)
+				nn[i] = plocNearestAt([&](uint32_t j) -> const GBox & { return box[j]; }, s.nc, i, kPlocRadius);
+		__syncthreads();
+		// this thread's two places: their partners and flags, scanned over the block
+		uint32_t part[2], v[2], sum = 0;
+		for (uint32_t k = 0; k < 2; ++k) {
+			const uint32_t i = i0 + k;
+			part[k] = i < s.nc ? plocPartner(nn, s.nc, i, s.forced != 0) : kNone;
+			v[k] = i >= s.nc ? 0u : (part[k] != kNone && i < part[k] ? 0x10000u : 0u) + (part[k] != kNone && i > part[k] ? 0u : 1u);
+			sum += v[k];
+		}
+		uint32_t incl = sum;
+		for (int o = 1; o < 64; o <<= 1) {
+			const uint32_t x = (uint32_t)__shfl_up((int)incl, o);
+			if ((int)(threadIdx.x & 63u) >= o) incl += x;
+		}
+		if ((threadIdx.x & 63u) == 63u) wsum[threadIdx.x >> 6] = incl;
+		__syncthreads();
+		uint32_t at = incl - sum, all = 0;
+		for (uint32_t w = 0; w < 16; ++w) {
+			if (w < (threadIdx.x >> 6)) at += wsum[w];
+			all += wsum[w];
+		}
+		const uint32_t merged = all >> 16, kept = all & 0xffffu;
+		const bool bad = merged == 0 || kept != s.nc - merged || s.nodeBase + merged > ni;
+		GBox nb[2];
+		uint32_t nid[2], to[2] = {kNone, kNone};
+		for (uint32_t k = 0; k < 2 && !bad; ++k) {
+			const uint32_t i = i0 + k, j = part[k];
+			if (i >= s.nc || (j != kNone && i > j)) {
+				at += v[k];
+				continue;
+			}
+			to[k] = at & 0xffffu;
+			if (j != kNone) {
+				nid[k] = s.nodeBase + (at >> 16);
+				nb[k] = unionBox(box[i], box[j]);
+				plocMake(T, nid[k], cid[i], cid[j], nb[k]);
+			} else {
+				nid[k] = cid[i];
+				nb[k] = box[i];
+			}
+			at += v[k];
+		}
+		__syncthreads();
+		if (bad) {
+			if (threadIdx.x == 0) atomicOr(err, kErrCluster);
+			break;
+		}
+		for (uint32_t k = 0; k < 2; ++k)
+			if (to[k] != kNone) {
+				box[to[k]] = nb[k];
+				cid[to[k]] = nid[k];
+			}
+		s.forced = !s.forced && merged * 64u < s.nc ? 1u : 0u;
+		s.nodeBase += merged;
+		s.nc = kept;
+		++r;
+		if (threadIdx.x == 0) st[r] = s;
+		__syncthreads();
+	}
+	if (threadIdx.x == 0) {
+		*rounds = r;
+		if (s.nc != 1 || s.nodeBase != ni) atomicOr(err, kErrCluster);
+	}
 }
 
-// first leaf place of each subtree, top down (the nodes of one round; their
-// parents are younger); leafFirst: the place of each sorted leaf
-__global__ void k_plocFirst(uint32_t b, uint32_t e, const uint32_t *left, const uint32_t *right, const uint32_t *count,
+// first leaf place of each subtree, top down; leafFirst: the place of each
+// sorted leaf
+__device__ __forceinline__ void plocFirst(uint32_t x, const uint32_t *left, const uint32_t *right, const uint32_t *count,
 		uint32_t *first, uint32_t *leafFirst) {
-	const uint32_t x = b + blockIdx.x * blockDim.x + threadIdx.x;
-	if (x >= e) return;
 	const uint32_t f = first[x], l = left[x], r = right[x];
 	const uint32_t fr = f + plocSize(l, count);
 	if (l & kLeafBit) leafFirst[l & ~kLeafBit] = f; else first[l] = f;
 	if (r & kLeafBit) leafFirst[r & ~kLeafBit] = fr; else first[r] = fr;
 }
 
+// the nodes of one round (their parents are younger)
+__global__ void k_plocFirst(uint32_t b, uint32_t e, const uint32_t *left, const uint32_t *right, const uint32_t *count,
+		uint32_t *first, uint32_t *leafFirst) {
+	const uint32_t x = b + blockIdx.x * blockDim.x + threadIdx.x;
+	if (x < e) plocFirst(x, left, right, count, first, leafFirst);
+}
+
+// rounds r1-1 down to r0 by one block (the tail's, below the root)
+__global__ __launch_bounds__(1024) void k_plocFirstTail(const PlocState *st, uint32_t r0, uint32_t r1, uint32_t ni,
+		const uint32_t *left, const uint32_t *right, const uint32_t *count, uint32_t *first, uint32_t *leafFirst) {
+	if (threadIdx.x == 0) first[ni - 1] = 0u;  // the root
+	__syncthreads();
+	for (uint32_t r = r1; r-- > r0;) {
+		for (uint32_t x = st[r].nodeBase + threadIdx.x; x < st[r + 1].nodeBase; x += 1024)
+			plocFirst(x, left, right, count, first, leafFirst);
+		__syncthreads();
+	}
+}
+
 // the clustering's tree in the radix tree's form: internal node x becomes
 // n-2-x (root 0), leaves their places; leaf values and boxes in place order
 __global__ void k_plocFinish(uint32_t n, const uint32_t *left, const uint32_t *right, const uint32_t *count,
-		const uint32_t *first, const GBox *nodeBox, const uint32_t *leafOK, const uint32_t *leafFirst,
+		const uint32_t *first, const GBox *nodeBox, const float *key, const uint32_t *leafFirst,
 		const uint32_t *vals, const GBox *leafBoxIn, uint32_t *left2, uint32_t *right2, uint32_t *first2,
-		uint32_t *last2, GBox *nodeBox2, uint32_t *leafOK2, uint32_t *vals2, GBox *leafBox2) {
+		uint32_t *last2, GBox *nodeBox2, float *key2, uint32_t *vals2, GBox *leafBox2) {
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
 	if (i >= n) return;
 	const uint32_t p = leafFirst[i];
@@ -460,37 +695,154 @@ __global__ void k_plocFinish(uint32_t n, const uint32_t *left, const uint32_t *r
 	first2[y] = first[i];
 	last2[y] = first[i] + count[i] - 1;
 	nodeBox2[y] = nodeBox[i];
-	leafOK2[y] = leafOK[i];
+	key2[y] = key[i];
 }
 
-// 5a. children of each frontier node and how many become inner nodes
-__global__ void k_expand(const uint32_t *frontier, uint32_t nf, uint32_t nInner, const uint32_t *left,
-		const uint32_t *right, const uint32_t *leafOK, const GBox *nodeBox, int width, uint32_t *kids,
-		uint32_t *innerCount, uint32_t *err) {
-	const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-	if (e >= nf) return;
-	const uint32_t b = frontier[e];
-	if (b >= nInner) {  // not an internal node
-		atomicOr(err, kErrExpand);
-		for (int k = 0; k < kMaxWide; ++k) kids[(size_t)kMaxWide * e + k] = kNone;
-		innerCount[e] = 0;
-		return;
+// 5. the breadth-first collapse, level by level.  A level's count and first
+// node are written on the device by the level before, so several levels are
+// launched on upper bounds between two looks of the host.
+struct Level {
+	uint32_t nf, base;
+};
+
+// 5a. children of each frontier node (expandNode's, from the nodes' keys: the
+// areas of the candidates stay in registers and each opened child costs one
+// read of its children and one of their keys), and how many become inner
+// nodes, summed over the block
+template <int W>
+__global__ __launch_bounds__(256) void k_expand(const uint32_t *frontier, const Level *lv, uint32_t l, uint32_t nInner,
+		const uint32_t *left, const uint32_t *right, const float *key, uint32_t *kids, uint32_t *prefix, uint32_t *sums,
+		uint32_t *err) {
+	const uint32_t nf = lv[l].nf;
+	if (blockIdx.x * 256u >= nf) return;
+	__shared__ uint32_t lds[4];
+	const uint32_t e = blockIdx.x * 256u + threadIdx.x;
+	uint32_t inner = 0;
+	if (e < nf) {
+		const uint32_t b = frontier[e];
+		uint32_t ch[W];
+		float a[W];
+#pragma unroll
+		for (int k = 0; k < W; ++k) {
+			ch[k] = kNone;
+			a[k] = -1.f;
+		}
+		auto keyOf = [key](uint32_t c) { return (c & kLeafBit) ? -1.f : key[c]; };
+		if (b < nInner) {
+			ch[0] = left[b];
+			ch[1] = right[b];
+			a[0] = keyOf(ch[0]);
+			a[1] = keyOf(ch[1]);
+			for (int nch = 2; nch < W; ++nch) {
+				int pick = -1;
+				float best = -1.f;
+				uint32_t c = 0;
+#pragma unroll
+				for (int k = 0; k < W; ++k)
+					if (a[k] > best) {
+						best = a[k];
+						pick = k;
+						c = ch[k];
+					}
+				if (pick < 0) break;
+				const uint32_t cl = left[c], cr = right[c];
+				const float al = keyOf(cl), ar = keyOf(cr);
+#pragma unroll
+				for (int k = W - 1; k > 0; --k)
+					if (k > pick + 1) {
+						ch[k] = ch[k - 1];
+						a[k] = a[k - 1];
+					}
+#pragma unroll
+				for (int k = 0; k < W; ++k) {
+					if (k == pick) {
+						ch[k] = cl;
+						a[k] = al;
+					}
+					if (k == pick + 1) {
+						ch[k] = cr;
+						a[k] = ar;
+					}
+				}
+			}
+		} else
+			atomicOr(err, kErrExpand);  // not an internal node
+#pragma unroll
+		for (int k = 0; k < W; ++k) {
+			// a child that stays a node has its area as key, zero or more (or a NaN's)
+			const bool leaf = ch[k] == kNone || (ch[k] & kLeafBit) || a[k] == -1.f;
+			kids[(size_t)W * e + k] = ch[k];
+			inner += leaf ? 0u : 1u;
+		}
 	}
-	uint32_t ch[kMaxWide];
-	innerCount[e] = expandNode(b, left, right, leafOK, nodeBox, width, ch);
-	for (int k = 0; k < kMaxWide; ++k) kids[(size_t)kMaxWide * e + k] = ch[k];
+	uint32_t sum;
+	const uint32_t p = blockPrefix(inner, lds, sum);
+	if (e < nf) prefix[e] = p;
+	if (threadIdx.x == 0) sums[blockIdx.x] = sum;
 }
 
-// 5b. the frontier's wide nodes; inner children get slots after the level
-__global__ void k_emit(uint32_t nf, const uint32_t *kids, const uint32_t *innerOff, const uint32_t *first,
-		const uint32_t *last, const uint32_t *leafOK, const GBox *leafBox, const GBox *nodeBox, uint32_t levelBase,
-		uint32_t layout, void *nodes, uint32_t *next) {
-	const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-	if (e >= nf) return;
-	uint32_t ch[kMaxWide];
-	for (int k = 0; k < kMaxWide; ++k) ch[k] = kids[(size_t)kMaxWide * e + k];
-	emitNode(ch, innerOff[e], first, last, leafOK, leafBox, nodeBox, levelBase + nf, layout, nodes, levelBase + e,
-			next);
+// 5b. block sums to block starts, and the next level (none, with the error
+// set, if its nodes would not fit)
+__global__ __launch_bounds__(1024) void k_levelScan(uint32_t *sums, Level *lv, uint32_t l, uint32_t capNodes,
+		uint32_t *host, uint32_t *err) {
+	__shared__ uint32_t lds[16];
+	const Level v = lv[l];
+	const uint32_t total = scanByBlock(sums, (v.nf + 255u) / 256u, lds);
+	if (threadIdx.x == 0) {
+		Level n = {total, v.base + v.nf};
+		if ((uint64_t)n.base + n.nf > capNodes) {
+			atomicOr(err, kErrExpand);
+			n.nf = 0;
+		}
+		lv[l + 1] = n;
+		host[0] = n.nf;
+		host[1] = n.base;
+		if (v.nf) host[2] = l + 1;  // levels with nodes
+	}
+}
+
+// 5c. the level's wide nodes, W lanes each (emitNode's record); inner children
+// get slots after the level
+template <int W, class Node>
+__global__ __launch_bounds__(256) void k_emit(const Level *lv, uint32_t l, const uint32_t *kids, const uint32_t *prefix,
+		const uint32_t *sums, const uint32_t *first, const uint32_t *last, const float *key, const GBox *leafBox,
+		const GBox *nodeBox, Node *nodes, uint32_t *next) {
+	const Level v = lv[l];
+	const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+	const uint32_t e = t / W;
+	const int c = (int)(t % W);
+	if (e >= v.nf || lv[l + 1].base != v.base + v.nf) return;
+	const uint32_t kid = kids[(size_t)W * e + c];
+	const bool some = kid != kNone;
+	const bool tri = some && (kid & kLeafBit);
+	const bool leaf = tri || (some && key[kid] == -1.f);
+	const uint32_t lane = threadIdx.x & 63u, shift = lane & ~(uint32_t)(W - 1);
+	const uint32_t innerMask = (uint32_t)(__ballot(some && !leaf) >> shift) & ((1u << W) - 1u);
+	const int n = __popc((uint32_t)(__ballot(some) >> shift) & ((1u << W) - 1u));
+	GBox b;
+	for (int k = 0; k < 3; ++k) { b.lo[k] = INFINITY; b.hi[k] = -INFINITY; }
+	uint32_t ref = LRH_CHILD_EMPTY;
+	if (some) b = tri ? leafBox[kid & ~kLeafBit] : nodeBox[kid];
+	if (leaf)
+		ref = tri ? leafRef(kid & ~kLeafBit, 1u) : leafRef(first[kid], last[kid] - first[kid] + 1u);
+	else if (some && lv[l + 1].nf) {
+		const uint32_t slot = sums[e / 256u] + prefix[e] + (uint32_t)__popc(innerMask & ((1u << c) - 1u));
+		ref = v.base + v.nf + slot;
+		next[slot] = kid;
+	}
+	Node *out = nodes + v.base + e;
+	if constexpr (std::is_same<Node, lrh_node4f>::value)
+		lrhdev::floatNodeLanes(b, c, n, ref, out);
+	else
+		lrhdev::quantizeNodeLanes<W>(b, c, n, ref, out);
+}
+
+__global__ void k_rootLevel(uint32_t *frontier, Level *lv, uint32_t *host) {
+	if (threadIdx.x != 0 || blockIdx.x != 0) return;
+	frontier[0] = 0u;
+	lv[0] = {1u, 0u};
+	host[0] = 1u;
+	host[1] = host[2] = 0u;
 }
 
 // a scene of at most maxLeaf triangles: one node with one leaf
@@ -543,10 +895,11 @@ struct Scratch {
 	std::vector<std::pair<void *, size_t>> held;
 	char *cur = nullptr;
 	size_t left = 0;
-	uint32_t *pin = nullptr;  // 2 KiB of pinned host memory for the readbacks (word 0: error, 1-3: counts, 128+: depths)
-	explicit Scratch(const LrhGpuAlloc &al) : a(al) {
-		GB_CHECK(hipHostMalloc(reinterpret_cast<void **>(&pin), 2048, hipHostMallocDefault));
-	}
+	// LRH_BUILD_PINNED bytes of pinned host memory that kernels write and the
+	// host reads after a wait (word 0: error, 1: rounds, 4-6: the collapse's
+	// level, 128+: digit starts)
+	uint32_t *pin = nullptr;
+	explicit Scratch(const LrhGpuAlloc &al) : a(al), pin(static_cast<uint32_t *>(al.pinned(al.ctx))) {}
 	template <class T>
 	T *get(size_t count) {
 		const size_t bytes = (std::max<size_t>(count * sizeof(T), 16) + 255) & ~size_t(255);
@@ -565,25 +918,21 @@ struct Scratch {
 	}
 	~Scratch() {
 		for (auto &h : held) a.release(a.ctx, h.first, h.second);
-		(void)hipHostFree(pin);
+		a.unpin(a.ctx, pin);
 	}
 };
 
 inline unsigned grid(size_t n, unsigned b) { return (unsigned)((n + b - 1) / b); }
 
-// exclusive scan of n values in place of out (in may equal out); the tile
-// sums are scanned by the same routine, so the depth is log_2048(n)
-void exclusiveScan(Scratch &S, const uint32_t *in, uint32_t *out, uint32_t n, hipStream_t st) {
-	if (n == 0) return;
-	const uint32_t tiles = grid(n, kScanTile);
-	uint32_t *sums = S.get<uint32_t>(tiles);
-	hipLaunchKernelGGL(k_scanTile, dim3(tiles), dim3(256), 0, st, in, out, n, sums);
+// one stable pass of the radix sort over the eight bits from `shift`
+void sortPass(const uint64_t *kIn, const uint32_t *vIn, uint32_t n, uint32_t shift, uint32_t *table, uint32_t *totals,
+		uint64_t *kOut, uint32_t *vOut, uint32_t *err, hipStream_t st) {
+	const uint32_t tiles = grid(n, kSortTile);
+	hipLaunchKernelGGL(k_sortCount, dim3(tiles), dim3(kSortBlock), 0, st, kIn, n, shift, tiles, table);
+	hipLaunchKernelGGL(k_scanRows, dim3(256), dim3(256), 0, st, table, tiles, totals);
+	hipLaunchKernelGGL(k_sortScatter, dim3(tiles), dim3(kSortBlock), 0, st, kIn, vIn, n, shift, tiles, table, totals, kOut,
+			vOut, err);
 	GB_CHECK(hipGetLastError());
-	if (tiles > 1) {
-		exclusiveScan(S, sums, sums, tiles, st);
-		hipLaunchKernelGGL(k_scanAdd, dim3(grid(n, 256)), dim3(256), 0, st, out, n, sums);
-		GB_CHECK(hipGetLastError());
-	}
 }
 
 // waits for the stream (and the readbacks queued before) and returns the
@@ -598,151 +947,127 @@ std::string errorText(uint32_t e) {
 	std::string s = "device build: ";
 	if (e & kErrUnsorted) s += "sorted Morton codes out of order; ";
 	if (e & kErrRange) s += "radix tree node without a key range (codes not in order); ";
-	if (e & kErrClimb) s += "radix tree deeper than any valid tree (or not rooted); ";
-	if (e & kErrExpand) s += "collapse reached a non-internal node; ";
+	if (e & kErrExpand) s += "collapse reached a non-internal node, or more nodes than the tree can have; ";
+	if (e & kErrCluster) s += "clustering round without a consistent merge count; ";
 	return s;
 }
 
-// boxes, costs and leaf decisions of the radix tree's nodes bottom-up with a
+// Boxes, costs and leaf decisions of the radix tree's nodes bottom-up with a
 // kernel boundary between levels instead of a fenced walk per leaf (a walk
 // publishes each box to the other XCDs' caches by an agent-scope fence,
-// which writes back and invalidates L2 on every step): depths by pointer
-// jumping, nodes sorted by depth, then one launch per level from the
-// deepest.
-void boxesByDepth(Scratch &S, const GBox *boxes, const uint32_t *vals, uint32_t n, const uint32_t *left,
-		const uint32_t *right, const uint32_t *first, const uint32_t *last, const uint32_t *iparent, uint32_t maxLeaf,
-		float ci, hipStream_t st, uint32_t *err, GBox *leafBox, GBox *nodeBox, uint32_t *leafOK) {
-	const uint32_t ni = n - 1;
-	uint32_t *dA = S.get<uint32_t>(ni), *dB = S.get<uint32_t>(ni), *jA = S.get<uint32_t>(ni),
-			 *jB = S.get<uint32_t>(ni), *order = S.get<uint32_t>(ni), *starts = S.get<uint32_t>(kMaxDepth + 1);
-	uint64_t *dKeys = S.get<uint64_t>(ni), *dKeysOut = S.get<uint64_t>(ni);
+// which writes back and invalidates L2 on every step).  A node's common
+// prefix is shorter than its children's, so nodes go by the length of their
+// prefix, which the radix tree knows, one launch per length from the longest
+// (depths would be fewer levels, but took seven rounds of pointer jumping);
+// runs of lengths with few nodes go to one block.
+void boxesByPrefix(Scratch &S, const GBox *boxes, const uint32_t *vals, uint32_t n, const uint32_t *left,
+		const uint32_t *right, const uint32_t *first, const uint32_t *last, const uint64_t *digits, const uint32_t *ids,
+		uint32_t maxLeaf, float ci, hipStream_t st, uint32_t *err, GBox *leafBox, GBox *nodeBox, float *key) {
+	const uint32_t ni = n - 1, tiles = grid(ni, kSortTile);
+	uint32_t *order = S.get<uint32_t>(ni), *starts = S.get<uint32_t>(256), *totals = S.get<uint32_t>(256);
+	uint64_t *digitsOut = S.get<uint64_t>(ni);
+	uint32_t *table = S.get<uint32_t>((size_t)256 * tiles);
 	float *cost = S.get<float>(ni);
-	hipLaunchKernelGGL(k_depthInit, dim3(grid(ni, 256)), dim3(256), 0, st, iparent, ni, dA, jA);
-	// depth < kMaxDepth = 2^7: seven doublings reach the root
-	for (int r = 0; r < 7; ++r) {
-		hipLaunchKernelGGL(k_depthJump, dim3(grid(ni, 256)), dim3(256), 0, st, ni, dA, jA, dB, jB);
-		std::swap(dA, dB);
-		std::swap(jA, jB);
-	}
-	hipLaunchKernelGGL(k_depthCheck, dim3(grid(ni, 256)), dim3(256), 0, st, ni, dA, jA, err);
-	GB_CHECK(hipGetLastError());
-	if (const uint32_t e = readError(S, err, st)) throw std::runtime_error(errorText(e));
-	// nodes in depth order: one stable pass of the radix sort (depth < 2^8
-	// is one digit) with the node ids as values, so no counter is contended;
-	// the scanned digit table gives where each depth starts
-	const uint32_t tiles = grid(ni, kSortTile);
-	uint32_t *table = S.get<uint32_t>((size_t)256 * tiles), *ids = S.get<uint32_t>(ni);
-	hipLaunchKernelGGL(k_depthKeys, dim3(grid(ni, 256)), dim3(256), 0, st, ni, dA, dKeys, ids);
-	hipLaunchKernelGGL(k_sortCount, dim3(tiles), dim3(kSortBlock), 0, st, dKeys, ni, 0u, tiles, table);
-	GB_CHECK(hipGetLastError());
-	exclusiveScan(S, table, table, 256u * tiles, st);
-	hipLaunchKernelGGL(k_sortScatter, dim3(tiles), dim3(kSortBlock), 0, st, dKeys, ids, ni, 0u, tiles, table, dKeysOut,
-			order, err);
-	hipLaunchKernelGGL(k_digitStarts, dim3(1), dim3(256), 0, st, table, tiles, starts);
-	GB_CHECK(hipGetLastError());
-	GB_CHECK(hipMemcpyAsync(S.pin + 128, starts, (kMaxDepth + 1) * 4, hipMemcpyDeviceToHost, st));
-	if (const uint32_t e = readError(S, err, st)) throw std::runtime_error(errorText(e));
-	uint32_t off[kMaxDepth + 1], h[kMaxDepth];
-	std::copy(S.pin + 128, S.pin + 128 + kMaxDepth + 1, off);
-	for (uint32_t d = 0; d < kMaxDepth; ++d) {
-		if (off[d + 1] < off[d]) throw std::runtime_error("device build: depth table out of order");
-		h[d] = off[d + 1] - off[d];
-	}
-	if (off[0] != 0 || off[kMaxDepth] != ni)
-		throw std::runtime_error("device build: radix tree nodes not all below the root");
+	sortPass(digits, ids, ni, 0u, table, totals, digitsOut, order, err, st);
+	hipLaunchKernelGGL(k_digitStarts, dim3(1), dim3(256), 0, st, totals, starts, S.pin + 128);
 	hipLaunchKernelGGL(k_leafBoxes, dim3(grid(n, 256)), dim3(256), 0, st, boxes, vals, n, leafBox);
 	GB_CHECK(hipGetLastError());
-	for (uint32_t d = kMaxDepth; d-- > 0;) {
-		const uint32_t cnt = h[d];
-		if (!cnt) continue;
-		hipLaunchKernelGGL(k_boxLevel, dim3(grid(cnt, 256)), dim3(256), 0, st, order + off[d], cnt, left, right, first,
-				last, leafBox, maxLeaf, ci, nodeBox, cost, leafOK);
+	if (const uint32_t e = readError(S, err, st)) throw std::runtime_error(errorText(e));
+	uint32_t off[kDigits + 1];
+	std::copy(S.pin + 128, S.pin + 128 + kDigits + 1, off);
+	for (uint32_t d = 0; d < kDigits; ++d)
+		if (off[d + 1] < off[d]) throw std::runtime_error("device build: prefix table out of order");
+	if (off[0] != 0 || off[kDigits] != ni) throw std::runtime_error("device build: radix tree nodes not all in the table");
+	for (uint32_t d = 0; d < kDigits;) {
+		const uint32_t cnt = off[d + 1] - off[d];
+		if (cnt > kSmallLevel) {
+			hipLaunchKernelGGL(k_boxLevel, dim3(grid(cnt, 256)), dim3(256), 0, st, order + off[d], cnt, left, right, first,
+					last, leafBox, maxLeaf, ci, nodeBox, cost, key);
+			++d;
+			continue;
+		}
+		uint32_t d1 = d + 1;
+		while (d1 < kDigits && off[d1 + 1] - off[d1] <= kSmallLevel) ++d1;
+		if (off[d1] > off[d])
+			hipLaunchKernelGGL(k_boxSmallLevels, dim3(1), dim3(1024), 0, st, order, starts, d, d1, left, right, first, last,
+					leafBox, maxLeaf, ci, nodeBox, cost, key);
+		d = d1;
 	}
 	GB_CHECK(hipGetLastError());
-	if (const uint32_t e = readError(S, err, st)) throw std::runtime_error(errorText(e));
 }
 
-// the clustering's binary tree over the n >= 2 sorted leaves, written in the
+// The clustering's binary tree over the n >= 2 sorted leaves, written in the
 // radix tree's form (left / right / first / last / nodeBox, root 0, leaf
 // places contiguous per subtree); vals and leafBox are repointed to the
 // leaves in place order.  Each round: nearest neighbours, the merge and keep
-// flags scanned, then the pairs merged and the clusters compacted.  The host
-// reads the round's merge count; a round that merges fewer than 1/64 of the
-// clusters is followed by a forced round that pairs places 2k, 2k+1, so the
-// number of rounds is bounded by the size alone.  (Natural rounds merge a
-// third of the clusters at first and a tenth or less near the top, where
-// boxes overlap; forcing there would cost tree quality.)
-void plocTree(Scratch &S, const GBox *boxes, uint32_t n, uint32_t maxLeaf, float ci, hipStream_t st, uint32_t *&vals,
-		GBox *&leafBox, uint32_t *left, uint32_t *right, uint32_t *first, uint32_t *last, GBox *nodeBox,
-		uint32_t *leafOK, uint32_t *roundsOut) {
+// flags scanned, then the pairs merged and the clusters compacted.  A round
+// that merges fewer than 1/64 of the clusters is followed by a forced round
+// that pairs places 2k, 2k+1, so the number of rounds is bounded by the size
+// alone.  (Natural rounds merge a third of the clusters at first and a tenth
+// or less near the top, where boxes overlap; forcing there would cost tree
+// quality.)  Rounds find their sizes on the device; the host looks at them
+// every kPlocBatch rounds, to shrink the grids and to stop.
+void plocTree(Scratch &S, const GBox *boxes, uint32_t n, uint32_t maxLeaf, float ci, hipStream_t st, uint32_t *err,
+		uint32_t *&vals, GBox *&leafBox, uint32_t *left, uint32_t *right, uint32_t *first, uint32_t *last, GBox *nodeBox,
+		float *key, uint32_t *roundsOut) {
+	constexpr uint32_t kPlocBatch = 6;
 	const uint32_t ni = n - 1;
-	uint32_t *cidA = S.get<uint32_t>(n), *cidB = S.get<uint32_t>(n), *nn = S.get<uint32_t>(n);
+	uint32_t *cidA = S.get<uint32_t>(n), *cidB = S.get<uint32_t>(n), *nn = S.get<uint32_t>(n), *prefix = S.get<uint32_t>(n);
 	GBox *cboxA = S.get<GBox>(n), *cboxB = S.get<GBox>(n);
-	uint32_t *lead = S.get<uint32_t>((size_t)n + 1), *keep = S.get<uint32_t>((size_t)n + 1),
-			 *leadOff = S.get<uint32_t>((size_t)n + 1), *keepOff = S.get<uint32_t>((size_t)n + 1);
-	hipLaunchKernelGGL(k_plocInit, dim3(grid(n, 256)), dim3(256), 0, st, boxes, vals, n, cidA, cboxA, leafBox);
+	uint32_t *leadSums = S.get<uint32_t>(grid(n, 256)), *keepSums = S.get<uint32_t>(grid(n, 256));
+	PlocState *state = S.get<PlocState>(kPlocMaxRounds + 1);
+	uint32_t *rounds = S.get<uint32_t>(1);
+	PlocTree T = {S.get<uint32_t>(ni), S.get<uint32_t>(ni), S.get<uint32_t>(ni), S.get<GBox>(ni), S.get<float>(ni),
+			S.get<float>(ni), leafBox, maxLeaf, ci};
+	hipLaunchKernelGGL(k_plocInit, dim3(grid(n, 256)), dim3(256), 0, st, boxes, vals, n, cidA, cboxA, leafBox, state);
 	GB_CHECK(hipGetLastError());
-	std::vector<uint32_t> roundStart{0};
-	uint32_t nc = n, nodeBase = 0;
-	bool forced = false;
-	// fewer than 1/64 merged forces the next round, which halves: at most
-	// 2 * 31 slow rounds, 63 single merges below 64 clusters, and
-	// log(2^31) / log(64/63) others
-	const uint32_t kMaxRounds = 4096;
-	while (nc > 1) {
-		if (roundStart.size() > kMaxRounds) throw std::runtime_error("device build: clustering did not converge");
-		if (!forced)
-			hipLaunchKernelGGL(k_plocNearest, dim3(grid(nc, kPlocTile)), dim3(kPlocTile), 0, st, cboxA, nc, nn);
-		hipLaunchKernelGGL(k_plocFlags, dim3(grid((size_t)nc + 1, 256)), dim3(256), 0, st, nn, nc, forced ? 1u : 0u,
-				lead, keep);
-		GB_CHECK(hipGetLastError());
-		exclusiveScan(S, lead, leadOff, nc + 1, st);
-		exclusiveScan(S, keep, keepOff, nc + 1, st);
-		hipLaunchKernelGGL(k_plocApply, dim3(grid(nc, 256)), dim3(256), 0, st, nn, nc, forced ? 1u : 0u, cidA, cboxA,
-				leadOff, keepOff, nodeBase, cidB, cboxB, left, right, nodeBox);
-		GB_CHECK(hipGetLastError());
-		GB_CHECK(hipMemcpyAsync(S.pin + 1, leadOff + nc, 4, hipMemcpyDeviceToHost, st));
-		GB_CHECK(hipMemcpyAsync(S.pin + 2, keepOff + nc, 4, hipMemcpyDeviceToHost, st));
-		GB_CHECK(hipStreamSynchronize(st));
-		const uint32_t merged = S.pin[1], kept = S.pin[2];
-		if (merged == 0 || merged > nc / 2 || kept != nc - merged || nodeBase + merged > ni)
-			throw std::runtime_error("device build: clustering round without a consistent merge count");
-		nodeBase += merged;
-		roundStart.push_back(nodeBase);
-		forced = !forced && (uint64_t)merged * 64u < nc;
-		nc = kept;
+	std::vector<PlocState> host(kPlocMaxRounds + 1);
+	uint32_t r = 0, ub = n;
+	while (ub > kPlocTail) {
+		for (uint32_t k = 0; k < kPlocBatch; ++k, ++r) {
+			if (r >= kPlocMaxRounds) throw std::runtime_error("device build: clustering did not converge");
+			hipLaunchKernelGGL(k_plocNearest, dim3(grid(ub, kPlocTile)), dim3(kPlocTile), 0, st, cboxA, state, r, nn);
+			hipLaunchKernelGGL(k_plocMark, dim3(grid(ub, 256)), dim3(256), 0, st, nn, state, r, prefix, leadSums, keepSums);
+			hipLaunchKernelGGL(k_plocScan, dim3(1), dim3(1024), 0, st, leadSums, keepSums, state, r, ni, err);
+			hipLaunchKernelGGL(k_plocApply, dim3(grid(ub, 256)), dim3(256), 0, st, nn, state, r, cidA, cboxA, prefix,
+					leadSums, keepSums, ni, cidB, cboxB, T);
+			GB_CHECK(hipGetLastError());
+			std::swap(cidA, cidB);
+			std::swap(cboxA, cboxB);
+		}
+		GB_CHECK(hipMemcpyAsync(S.pin + 8, state + (r - kPlocBatch), (kPlocBatch + 1) * sizeof(PlocState),
+				hipMemcpyDeviceToHost, st));
+		if (const uint32_t e = readError(S, err, st)) throw std::runtime_error(errorText(e));
+		std::copy_n(reinterpret_cast<const PlocState *>(S.pin + 8), kPlocBatch + 1, host.begin() + (r - kPlocBatch));
+		ub = host[r].nc;
+	}
+	// the rounds after the count fell to the tail's changed nothing but the
+	// buffers' roles: the clusters are where the last real round put them
+	uint32_t r0 = r;
+	while (r0 > 0 && host[r0 - 1].nc <= kPlocTail && host[r0 - 1].nc == host[r0].nc) --r0;
+	if ((r - r0) & 1u) {
 		std::swap(cidA, cidB);
 		std::swap(cboxA, cboxB);
 	}
-	if (nodeBase != ni) throw std::runtime_error("device build: clustering left nodes unmade");
-	*roundsOut = (uint32_t)roundStart.size() - 1;
-	// leaves per subtree, oldest round first; first places, newest first
-	uint32_t *count = S.get<uint32_t>(ni), *firstP = S.get<uint32_t>(ni), *leafFirst = S.get<uint32_t>(n),
-			 *leafP = S.get<uint32_t>(ni);
-	float *cost = S.get<float>(ni);
-	for (size_t r = 0; r + 1 < roundStart.size(); ++r) {
-		const uint32_t b = roundStart[r], e = roundStart[r + 1];
-		hipLaunchKernelGGL(k_plocCount, dim3(grid(e - b, 256)), dim3(256), 0, st, b, e, left, right, leafBox, nodeBox,
-				maxLeaf, ci, count, cost, leafP);
+	hipLaunchKernelGGL(k_plocTail, dim3(1), dim3(1024), 0, st, state, r0, ni, cidA, cboxA, T, rounds, err);
+	GB_CHECK(hipMemcpyAsync(S.pin + 1, rounds, 4, hipMemcpyDeviceToHost, st));
+	if (const uint32_t e = readError(S, err, st)) throw std::runtime_error(errorText(e));
+	const uint32_t r1 = S.pin[1];
+	*roundsOut = r1;
+	// first places, newest round first
+	uint32_t *firstP = S.get<uint32_t>(ni), *leafFirst = S.get<uint32_t>(n);
+	hipLaunchKernelGGL(k_plocFirstTail, dim3(1), dim3(1024), 0, st, state, r0, r1, ni, T.left, T.right, T.count, firstP,
+			leafFirst);
+	for (uint32_t k = r0; k-- > 0;) {
+		const uint32_t b = host[k].nodeBase, e = host[k + 1].nodeBase;
+		if (e > b)
+			hipLaunchKernelGGL(k_plocFirst, dim3(grid(e - b, 256)), dim3(256), 0, st, b, e, T.left, T.right, T.count, firstP,
+					leafFirst);
 	}
-	hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, st, firstP + (ni - 1), 1u, 0u);  // the root, node n-2
-	for (size_t r = roundStart.size() - 1; r-- > 0;) {
-		const uint32_t b = roundStart[r], e = roundStart[r + 1];
-		hipLaunchKernelGGL(k_plocFirst, dim3(grid(e - b, 256)), dim3(256), 0, st, b, e, left, right, count, firstP,
-				leafFirst);
-	}
-	GB_CHECK(hipGetLastError());
-	// the radix tree's form, written into the caller's arrays; the binary
-	// tree's own are copied aside first
-	uint32_t *leftP = S.get<uint32_t>(ni), *rightP = S.get<uint32_t>(ni);
-	GBox *boxP = S.get<GBox>(ni);
-	GB_CHECK(hipMemcpyAsync(leftP, left, (size_t)ni * 4, hipMemcpyDeviceToDevice, st));
-	GB_CHECK(hipMemcpyAsync(rightP, right, (size_t)ni * 4, hipMemcpyDeviceToDevice, st));
-	GB_CHECK(hipMemcpyAsync(boxP, nodeBox, (size_t)ni * sizeof(GBox), hipMemcpyDeviceToDevice, st));
 	uint32_t *vals2 = S.get<uint32_t>(n);
 	GBox *leafBox2 = S.get<GBox>(n);
-	hipLaunchKernelGGL(k_plocFinish, dim3(grid(n, 256)), dim3(256), 0, st, n, leftP, rightP, count, firstP, boxP,
-			leafP, leafFirst, vals, leafBox, left, right, first, last, nodeBox, leafOK, vals2, leafBox2);
+	hipLaunchKernelGGL(k_plocFinish, dim3(grid(n, 256)), dim3(256), 0, st, n, T.left, T.right, T.count, firstP, T.box,
+			T.key, leafFirst, vals, leafBox, left, right, first, last, nodeBox, key, vals2, leafBox2);
 	GB_CHECK(hipGetLastError());
 	vals = vals2;
 	leafBox = leafBox2;
@@ -784,6 +1109,13 @@ void lrhGpuBuildBVH(const LrhGpuBuildIn &in, const LrhGpuAlloc &a, hipStream_t s
 	const size_t capNodes = std::max<uint32_t>(n > 1 ? n - 1 : 1, 1);
 	void *nodes = a.alloc(a.ctx, capNodes * nodeSz);
 	uint32_t nodeCount = 0, depth = 0;
+	auto allocRecords = [&]() {
+		if (out->tris) return;
+		out->triBytes = (size_t)n * sizeof(lrh_tri);
+		out->tris = a.alloc(a.ctx, out->triBytes);
+		out->invPermBytes = (size_t)n * 4;
+		out->invPerm = static_cast<uint32_t *>(a.alloc(a.ctx, out->invPermBytes));
+	};
 	try {
 		if (n <= in.maxLeaf) {
 			hipLaunchKernelGGL(k_identity, dim3(grid(n, 256)), dim3(256), 0, st, boxes, n, vals, leafBox);
@@ -797,75 +1129,79 @@ void lrhGpuBuildBVH(const LrhGpuBuildIn &in, const LrhGpuAlloc &a, hipStream_t s
 			GB_CHECK(hipGetLastError());
 			// stable LSD radix sort, 8 passes of 8 bits; an even number of
 			// passes leaves the result in keys / vals
-			const uint32_t tiles = grid(n, kSortTile);
-			uint32_t *table = S.get<uint32_t>((size_t)256 * tiles);
+			uint32_t *table = S.get<uint32_t>((size_t)256 * grid(n, kSortTile)), *totals = S.get<uint32_t>(256);
 			uint64_t *kIn = keys, *kOut = keysB;
 			uint32_t *vIn = vals, *vOut = valsB;
 			for (uint32_t shift = 0; shift < 64; shift += 8) {
-				hipLaunchKernelGGL(k_sortCount, dim3(tiles), dim3(kSortBlock), 0, st, kIn, n, shift, tiles, table);
-				GB_CHECK(hipGetLastError());
-				exclusiveScan(S, table, table, 256u * tiles, st);
-				hipLaunchKernelGGL(k_sortScatter, dim3(tiles), dim3(kSortBlock), 0, st, kIn, vIn, n, shift, tiles, table,
-						kOut, vOut, err);
-				GB_CHECK(hipGetLastError());
+				sortPass(kIn, vIn, n, shift, table, totals, kOut, vOut, err, st);
 				std::swap(kIn, kOut);
 				std::swap(vIn, vOut);
 			}
 			hipLaunchKernelGGL(k_checkSorted, dim3(grid(n, 256)), dim3(256), 0, st, keys, n, err);
 			GB_CHECK(hipGetLastError());
-			if (const uint32_t e = readError(S, err, st)) throw std::runtime_error(errorText(e));
+			allocRecords();  // (while the sort runs)
 
 			const uint32_t ni = n - 1;
 			uint32_t *left = S.get<uint32_t>(ni), *right = S.get<uint32_t>(ni), *first = S.get<uint32_t>(ni),
 					 *last = S.get<uint32_t>(ni);
 			GBox *nodeBox = S.get<GBox>(ni);
-			uint32_t *leafOK = S.get<uint32_t>(ni);
+			float *key = S.get<float>(ni);
 			if (in.method == 1) {
-				plocTree(S, boxes, n, in.maxLeaf, in.travCost, st, vals, leafBox, left, right, first, last, nodeBox,
-						leafOK, &out->plocRounds);
-			} else {
-				uint32_t *iparent = S.get<uint32_t>(ni);
-				hipLaunchKernelGGL(k_fill, dim3(grid(ni, 256)), dim3(256), 0, st, iparent, ni, kNone);  // root: none
-				hipLaunchKernelGGL(k_radixTree, dim3(grid(ni, 256)), dim3(256), 0, st, keys, n, left, right, first,
-						last, iparent, err);
-				GB_CHECK(hipGetLastError());
 				if (const uint32_t e = readError(S, err, st)) throw std::runtime_error(errorText(e));
-				boxesByDepth(S, boxes, vals, n, left, right, first, last, iparent, in.maxLeaf, in.travCost, st, err,
-						leafBox, nodeBox, leafOK);
+				plocTree(S, boxes, n, in.maxLeaf, in.travCost, st, err, vals, leafBox, left, right, first, last, nodeBox, key,
+						&out->plocRounds);
+			} else {
+				// the sorted keys' other buffers hold the digits and ids
+				hipLaunchKernelGGL(k_radixTree, dim3(grid(ni, 256)), dim3(256), 0, st, keys, n, left, right, first, last, keysB,
+						valsB, err);
+				GB_CHECK(hipGetLastError());
+				boxesByPrefix(S, boxes, vals, n, left, right, first, last, keysB, valsB, in.maxLeaf, in.travCost, st, err,
+						leafBox, nodeBox, key);
 			}
 
-			// breadth-first collapse: level frontiers of binary node ids
+			// breadth-first collapse: level frontiers of binary node ids; a level
+			// has at most `width` times the nodes of the one before, which the host
+			// knows after each batch of levels
+			constexpr uint32_t kMaxLevels = 160;
 			uint32_t *fA = S.get<uint32_t>(ni), *fB = S.get<uint32_t>(ni);
-			uint32_t *kids = S.get<uint32_t>((size_t)kMaxWide * ni), *cnt = S.get<uint32_t>(ni + 1),
-					 *off = S.get<uint32_t>(ni + 1);
-			hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, st, fA, 1u, 0u);  // the root
-			uint32_t nf = 1, levelBase = 0;
+			uint32_t *kids = S.get<uint32_t>((size_t)width * ni), *prefix = S.get<uint32_t>(ni),
+					 *sums = S.get<uint32_t>(grid(ni, 256));
+			Level *lv = S.get<Level>(kMaxLevels + 1);
+			hipLaunchKernelGGL(k_rootLevel, dim3(1), dim3(64), 0, st, fA, lv, S.pin + 4);
+			uint32_t nf = 1, l = 0;
 			while (nf) {
-				if ((size_t)levelBase + nf > capNodes) throw std::runtime_error("device build: node capacity");
-				if (depth > 128) throw std::runtime_error("device build: collapse deeper than any valid tree");
-				hipLaunchKernelGGL(k_expand, dim3(grid(nf, 256)), dim3(256), 0, st, fA, nf, ni, left, right, leafOK,
-						nodeBox, width, kids, cnt, err);
-				hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, st, cnt + nf, 1u, 0u);
-				GB_CHECK(hipGetLastError());
-				exclusiveScan(S, cnt, off, nf + 1, st);
-				hipLaunchKernelGGL(k_emit, dim3(grid(nf, 256)), dim3(256), 0, st, nf, kids, off, first, last, leafOK,
-						leafBox, nodeBox, levelBase, in.layout, nodes, fB);
-				GB_CHECK(hipGetLastError());
-				GB_CHECK(hipMemcpyAsync(S.pin + 3, off + nf, 4, hipMemcpyDeviceToHost, st));
+				// down to a level that may hold 4,096 nodes at first, then two at a time
+				const uint32_t batch = l == 0 ? (width == 8 ? 5u : 7u) : 2u;
+				uint64_t ub = nf;
+				for (uint32_t k = 0; k < batch; ++k, ++l, ub = std::min<uint64_t>(ub * width, ni)) {
+					if (l >= kMaxLevels) throw std::runtime_error("device build: collapse deeper than any valid tree");
+					const dim3 ge(grid(ub, 256)), gm(grid(ub * width, 256)), b(256);
+					if (width == 8)
+						hipLaunchKernelGGL(k_expand<8>, ge, b, 0, st, fA, lv, l, ni, left, right, key, kids, prefix, sums, err);
+					else
+						hipLaunchKernelGGL(k_expand<4>, ge, b, 0, st, fA, lv, l, ni, left, right, key, kids, prefix, sums, err);
+					hipLaunchKernelGGL(k_levelScan, dim3(1), dim3(1024), 0, st, sums, lv, l, (uint32_t)capNodes, S.pin + 4, err);
+					if (in.layout == 2)
+						hipLaunchKernelGGL((k_emit<8, lrh_node8q>), gm, b, 0, st, lv, l, kids, prefix, sums, first, last, key,
+								leafBox, nodeBox, static_cast<lrh_node8q *>(nodes), fB);
+					else if (in.layout == 1)
+						hipLaunchKernelGGL((k_emit<4, lrh_node4f>), gm, b, 0, st, lv, l, kids, prefix, sums, first, last, key,
+								leafBox, nodeBox, static_cast<lrh_node4f *>(nodes), fB);
+					else
+						hipLaunchKernelGGL((k_emit<4, lrh_node4q>), gm, b, 0, st, lv, l, kids, prefix, sums, first, last, key,
+								leafBox, nodeBox, static_cast<lrh_node4q *>(nodes), fB);
+					GB_CHECK(hipGetLastError());
+					std::swap(fA, fB);
+				}
 				if (const uint32_t e = readError(S, err, st)) throw std::runtime_error(errorText(e));
-				const uint32_t nextN = S.pin[3];
-				levelBase += nf;
-				nf = nextN;
-				std::swap(fA, fB);
-				++depth;
+				nf = S.pin[4];
 			}
+			depth = S.pin[6];
+			const uint32_t levelBase = S.pin[5];
 			nodeCount = levelBase;
 		}
 		// triangle records in leaf order
-		out->triBytes = (size_t)n * sizeof(lrh_tri);
-		out->tris = a.alloc(a.ctx, out->triBytes);
-		out->invPermBytes = (size_t)n * 4;
-		out->invPerm = static_cast<uint32_t *>(a.alloc(a.ctx, out->invPermBytes));
+		allocRecords();
 		hipLaunchKernelGGL(k_records, dim3(grid(n, 256)), dim3(256), 0, st, in.verts, in.tris, tbase, vbase,
 				in.nMeshes, vals, n, static_cast<lrh_tri *>(out->tris), out->invPerm);
 		GB_CHECK(hipGetLastError());

@@ -39,14 +39,13 @@ enum : uint32_t {
 	kErrUnsorted = 1u,   // sorted codes out of order
 	kErrRange = 2u,      // a radix-tree node found no range (keys not in order around it)
 	kErrClimb = 4u,      // a radix-tree node deeper than any valid tree (or not below the root)
-	kErrExpand = 8u,     // a frontier entry that is not an internal node
+	kErrExpand = 8u,     // a frontier entry that is not an internal node (or more nodes than the tree has)
+	kErrCluster = 16u,   // a clustering round without a consistent merge count
 };
 
 // radix sort: 8-bit digits, tiles of kSortTile keys per block
 constexpr uint32_t kSortTile = 2048u;
 constexpr uint32_t kSortBlock = 256u;
-// exclusive scan: tiles of kScanTile values per block
-constexpr uint32_t kScanTile = 2048u;
 
 LRH_DN inline uint32_t meshOf(const uint32_t *base, uint32_t nMeshes, uint32_t i) {
 	uint32_t lo = 0, hi = nMeshes;  // last mesh whose base <= i
@@ -204,6 +203,8 @@ LRH_DN inline float nodeCost(float A, float cl, float cr, uint32_t N, uint32_t m
 // cost chose as a leaf
 LRH_DN inline bool leafChild(uint32_t c, const uint32_t *leafOK) { return (c & kLeafBit) || leafOK[c]; }
 
+// (steps 4a and 4b are the sequential form; the device writes the same nodes
+// from the nodes' areas and with a lane per child)
 // 4a. the children of internal node b (Morton order): its two, then the
 // largest-area child that is not a leaf split until there are `width` (4 or
 // 8); returns how many of them become inner nodes

@@ -108,6 +108,43 @@ def test_device_build_equals_cpu_emulation(gpu_device, emu, tmp_path, scene, lay
     dsc.close()
 
 
+def _build_edge_scene(kind, n):
+    """Few or many triangles spread at random, or n copies of one triangle
+    (equal codes: the tree goes by position, every clustering area ties), or
+    a row of triangles of doubling size (a deep tree of few nodes a level)."""
+    rng = np.random.default_rng(n)
+    tri = rng.normal(size=(n, 1, 3)) + rng.normal(0.0, 0.05, (n, 3, 3))
+    if kind == "copies":
+        tri[:] = tri[0]
+    elif kind == "row":
+        tri = tri[:1] * np.exp2(-np.arange(n) % 60)[:, None, None]
+    return [scenes.Mesh(tri.reshape(-1, 3).astype(np.float32),
+                        np.arange(3 * n, dtype=np.uint32).reshape(-1, 3))]
+
+
+@pytest.mark.parametrize("builder", list(BUILDERS))
+@pytest.mark.parametrize("kind,n,layout,max_leaf", [
+    ("spread", 2, 2, 1), ("spread", 257, 2, 4), ("spread", 2047, 2, 4), ("spread", 2048, 0, 4), ("spread", 2049, 1, 1),
+    ("spread", 4099, 2, 1), ("spread", 70001, 2, 2), ("copies", 300, 2, 4), ("copies", 9000, 2, 1), ("row", 3000, 0, 1),
+    ("row", 120, 2, 1)])
+def test_device_build_edges_equal_cpu_emulation(gpu_device, emu, tmp_path, kind, n, layout, max_leaf, builder):
+    """Node and record bytes equal the emulation's where the build changes its
+    launches: clusters around the 2,048 that one block finishes, tree levels
+    around the 2,048 nodes that share a launch, levels of one block and of
+    many, odd remainders of the 256-node blocks."""
+    from tests.test_lbvh_cpu import run_emu
+    _case("devbuild_edges", kind=kind, n=n, layout=layout, max_leaf=max_leaf, builder=builder)
+    meshes = _build_edge_scene(kind, n)
+    info, nodes, tris = run_emu(emu, tmp_path, meshes, max_leaf, layout, method=builder)
+    assert info["err"] == 0
+    dsc = gpu_device.scene_bvh(meshes, layout=layout, max_leaf=max_leaf, builder=BUILDERS[builder])
+    nb, pb = dsc.download()
+    assert dsc.info()["nodeCount"] == info["nodes"]
+    assert nb.tobytes() == nodes.tobytes()
+    assert pb.tobytes() == tris.tobytes()
+    dsc.close()
+
+
 @pytest.mark.parametrize("builder", list(BUILDERS))
 @pytest.mark.parametrize("layout", [0, 1, 2])
 def test_device_build_trace_parity(gpu_device, layout, builder):
