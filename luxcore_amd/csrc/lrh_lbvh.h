@@ -41,6 +41,7 @@ enum : uint32_t {
 	kErrClimb = 4u,      // a radix-tree node deeper than any valid tree (or not below the root)
 	kErrExpand = 8u,     // a frontier entry that is not an internal node (or more nodes than the tree has)
 	kErrCluster = 16u,   // a clustering round without a consistent merge count
+	kErrIndex = 32u,     // a triangle's vertex index outside its mesh
 };
 
 // radix sort: 8-bit digits, tiles of kSortTile keys per block
@@ -66,12 +67,8 @@ LRH_DN inline void loadTri(const float *verts, const uint32_t *tris, const uint3
 	}
 }
 
-// 1. leaf box of triangle i (the host builder's triangleBox)
-LRH_DN inline GBox primBox(const float *verts, const uint32_t *tris, const uint32_t *tbase, const uint32_t *vbase,
-		uint32_t nMeshes, uint32_t i) {
-	const uint32_t m = meshOf(tbase, nMeshes, i);
-	float p[3][3];
-	loadTri(verts, tris, vbase, m, i, p);
+// 1. leaf box of a triangle (the host builder's triangleBox)
+LRH_DN inline GBox boxOf(const float p[3][3]) {
 	GBox b;
 	for (int k = 0; k < 3; ++k) {
 		b.lo[k] = minT(p[0][k], p[1][k]);
@@ -89,6 +86,12 @@ LRH_DN inline GBox primBox(const float *verts, const uint32_t *tris, const uint3
 		b.hi[k] += e;
 	}
 	return b;
+}
+LRH_DN inline GBox primBox(const float *verts, const uint32_t *tris, const uint32_t *tbase, const uint32_t *vbase,
+		uint32_t nMeshes, uint32_t i) {
+	float p[3][3];
+	loadTri(verts, tris, vbase, meshOf(tbase, nMeshes, i), i, p);
+	return boxOf(p);
 }
 
 LRH_DN inline uint64_t spread21(uint32_t v) {

@@ -146,6 +146,24 @@ def test_device_build_edges_equal_cpu_emulation(gpu_device, emu, tmp_path, kind,
 
 
 @pytest.mark.parametrize("builder", list(BUILDERS))
+@pytest.mark.parametrize("n", [1, 3, 257, 5000])
+def test_device_build_refuses_vertex_index(gpu_device, n, builder):
+    """An index at the end of its mesh (a valid vertex of the next one, or the
+    end of the last) is refused as the host's check words it, whatever the
+    build's path, before any kernel follows it; the device goes on."""
+    _case("devbuild_index", n=n, builder=builder)
+    good = _build_edge_scene("spread", n)[0]
+    for where in (0, 1):
+        meshes = [scenes.Mesh(good.verts, good.tris.copy()) for _ in range(2)]
+        meshes[where].tris[n - 1, 1] = 3 * n
+        with pytest.raises(D.LrhError, match=f"mesh {where}: vertex index out of range"):
+            gpu_device.scene_bvh(meshes, layout=2, max_leaf=4, builder=BUILDERS[builder])
+    dsc = gpu_device.scene_bvh([good], layout=2, max_leaf=4, builder=BUILDERS[builder])
+    assert dsc.download()[1].size == 48 * n
+    dsc.close()
+
+
+@pytest.mark.parametrize("builder", list(BUILDERS))
 @pytest.mark.parametrize("layout", [0, 1, 2])
 def test_device_build_trace_parity(gpu_device, layout, builder):
     _case("devbuild_parity", layout=layout, builder=builder)
