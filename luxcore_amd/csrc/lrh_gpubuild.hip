@@ -58,9 +58,10 @@ __global__ void k_fill(uint32_t *p, uint32_t n, uint32_t v) {
 // 1. leaf boxes and centre bounds: a grid-stride loop, the bounds reduced
 // in registers, across the wave by lane exchanges and across the block in
 // LDS, one partial result a block (six atomics a block to the same line
-// bounded the kernel: 105 us for 2.29M triangles, now 35 and 10 for the reduction).  A vertex index outside its mesh sets the
-// error and is not followed; the host looks at the error before anything else
-// reads vertices, so meshes need no pass over their indices on the host first.
+// bounded the kernel: 105 us for 2.29M triangles, now 38 and 5 for the
+// reduction).  A vertex index outside its mesh sets the error and is not
+// followed; the host looks at the error before anything else reads vertices,
+// so meshes need no pass over their indices on the host first.
 constexpr uint32_t kPrimBlocks = 2048;
 __device__ __forceinline__ uint32_t minU(uint32_t a, uint32_t b) { return a < b ? a : b; }
 __device__ __forceinline__ uint32_t maxU(uint32_t a, uint32_t b) { return a > b ? a : b; }
@@ -119,6 +120,7 @@ __global__ __launch_bounds__(256) void k_prims(const float *__restrict__ verts, 
 __global__ __launch_bounds__(384) void k_bounds(const uint32_t *partial, uint32_t nBlocks, uint32_t *cb) {
 	const uint32_t k = threadIdx.x >> 6, lane = threadIdx.x & 63u;
 	uint32_t v = k < 3 ? 0xffffffffu : 0u;
+#pragma unroll 8
 	for (uint32_t b = lane; b < nBlocks; b += 64) {
 		const uint32_t x = partial[6 * b + k];
 		v = k < 3 ? minU(v, x) : maxU(v, x);
@@ -142,13 +144,23 @@ __global__ void k_morton(const GBox *boxes, uint32_t n, const uint32_t *cbIn, ui
 }
 
 // ---- radix sort pass: per-tile digit counts, table [digit][tile] ----
+// tiles of kSortTile keys, or of kSortTileSmall up to kSortSmall keys: there
+// the large tiles leave compute units without a block, and a tile's eight
+// rounds run one after another (the scatter of 50,000 keys: 12.8 us, now 6)
+constexpr uint32_t kSortTileSmall = 512, kSortSmall = 512 * 1024;
+uint32_t sortTiles(uint32_t n) {
+	const uint32_t tile = n <= kSortSmall ? kSortTileSmall : kSortTile;
+	return (uint32_t)(((uint64_t)n + tile - 1) / tile);
+}
+
+template <uint32_t TILE>
 __global__ __launch_bounds__(kSortBlock) void k_sortCount(const uint64_t *keys, uint32_t n, uint32_t shift,
 		uint32_t nTiles, uint32_t *table) {
 	__shared__ uint32_t cnt[256];
 	cnt[threadIdx.x] = 0;
 	__syncthreads();
-	const uint64_t base = (uint64_t)blockIdx.x * kSortTile;
-	for (uint32_t j = threadIdx.x; j < kSortTile; j += kSortBlock) {
+	const uint64_t base = (uint64_t)blockIdx.x * TILE;
+	for (uint32_t j = threadIdx.x; j < TILE; j += kSortBlock) {
 		const uint64_t idx = base + j;
 		if (idx < n) atomicAdd(&cnt[digitOf(keys[idx], shift)], 1u);
 	}
@@ -165,6 +177,7 @@ __global__ __launch_bounds__(kSortBlock) void k_sortCount(const uint64_t *keys, 
 // values are first placed in LDS in that order, then written out in place
 // order, so consecutive threads write consecutive addresses of one digit's
 // run (its global start from the scanned [digit][tile] table). ----
+template <uint32_t TILE>
 __global__ __launch_bounds__(kSortBlock) void k_sortScatter(const uint64_t *keysIn, const uint32_t *valsIn, uint32_t n,
 		uint32_t shift, uint32_t nTiles, const uint32_t *offsets, const uint32_t *totals, uint64_t *keysOut,
 		uint32_t *valsOut, uint32_t *err) {
@@ -174,11 +187,11 @@ __global__ __launch_bounds__(kSortBlock) void k_sortScatter(const uint64_t *keys
 	__shared__ uint32_t off[256];    // global start of each digit's run for this tile
 	__shared__ uint32_t start[256];  // each digit's start within the tile
 	__shared__ uint32_t base[256];   // each digit's start in the whole output
-	__shared__ uint64_t sKey[kSortTile];
-	__shared__ uint32_t sVal[kSortTile];
+	__shared__ uint64_t sKey[TILE];
+	__shared__ uint32_t sVal[TILE];
 	const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
-	const uint64_t tile0 = (uint64_t)blockIdx.x * kSortTile;
-	const uint32_t tileN = (uint32_t)((n - tile0) < kSortTile ? (n - tile0) : kSortTile);
+	const uint64_t tile0 = (uint64_t)blockIdx.x * TILE;
+	const uint32_t tileN = (uint32_t)((n - tile0) < TILE ? (n - tile0) : TILE);
 	// the tile's digit counts, scanned to starts
 	run[tid] = 0;
 	for (uint32_t w = 0; w < kWaves; ++w) wcnt[w][tid] = 0;
@@ -202,7 +215,7 @@ __global__ __launch_bounds__(kSortBlock) void k_sortScatter(const uint64_t *keys
 	run[tid] = 0;
 	__syncthreads();
 	const uint64_t lanesBelow = (1ull << lane) - 1ull;
-	for (uint32_t r = 0; r < kSortTile / kSortBlock; ++r) {
+	for (uint32_t r = 0; r < TILE / kSortBlock; ++r) {
 		const uint32_t j = r * kSortBlock + tid;
 		const bool valid = j < tileN;
 		const uint64_t key = valid ? keysIn[tile0 + j] : 0ull;
@@ -221,7 +234,7 @@ __global__ __launch_bounds__(kSortBlock) void k_sortScatter(const uint64_t *keys
 			uint32_t before = run[dg];
 			for (uint32_t w = 0; w < wave; ++w) before += wcnt[w][dg];
 			const uint32_t p = start[dg] + before + rank;
-			if (p < kSortTile) {
+			if (p < TILE) {
 				sKey[p] = key;
 				sVal[p] = val;
 			} else {
@@ -443,7 +456,8 @@ __global__ void k_plocInit(const GBox *boxes, const uint32_t *vals, uint32_t n, 
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
 	if (i < 4) reinterpret_cast<uint32_t *>(st)[i] = i == 0 ? n : 0u;
 	if (i >= n) return;
-	const GBox b = boxes[vals[i]];
+	const uint32_t v = vals[i];
+	const GBox b = boxes[v < n ? v : 0u];  // (a failed sort's values are reported later)
 	leafBox[i] = b;
 	cid[i] = kLeafBit | i;
 	cbox[i] = b;
@@ -469,27 +483,64 @@ __device__ __forceinline__ PlocState plocRound(const PlocState *st, uint32_t r) 
 	return s;
 }
 
-// nearest neighbours of a tile of 256 clusters, their boxes and the
-// kPlocRadius on either side staged in LDS (each box is read by 2r+1 threads)
-constexpr uint32_t kPlocTile = 256;
-__global__ __launch_bounds__(kPlocTile) void k_plocNearest(const GBox *cbox, const PlocState *st, uint32_t r, uint32_t *nn) {
-	constexpr uint32_t kSpan = kPlocTile + 2 * kPlocRadius;
+// plocNearestAt by L neighbouring lanes, each with every L-th place: of equal
+// areas the lowest place wins, which is the order of the pairs (a pair with a
+// lower place comes first by its lower end or, above i, by its upper)
+template <uint32_t L, class BoxAt>
+__device__ __forceinline__ uint32_t plocNearestLanes(const BoxAt &box, uint32_t nc, uint32_t i, uint32_t sub) {
+	float best = INFINITY;
+	uint32_t arg = kNone;
+	if (i < nc) {
+		const uint32_t lo = i > kPlocRadius ? i - kPlocRadius : 0u;
+		const uint32_t hi = (nc - 1u - i > kPlocRadius) ? i + kPlocRadius : nc - 1u;
+		const GBox ci = box(i);
+		for (uint32_t j = lo + sub; j <= hi; j += L) {
+			if (j == i) continue;
+			const float a = mergedArea(ci, box(j));
+			if (a < best || arg == kNone) {
+				best = a;
+				arg = j;
+			}
+		}
+	}
+	for (uint32_t o = L / 2; o > 0; o >>= 1) {
+		const float a = __shfl_xor(best, (int)o);
+		const uint32_t g = (uint32_t)__shfl_xor((int)arg, (int)o);
+		if (a < best || (a == best && g < arg)) {
+			best = a;
+			arg = g;
+		}
+	}
+	return arg == kNone ? i : arg;
+}
+
+// nearest neighbours of a tile of 256/L clusters, their boxes and the
+// kPlocRadius on either side staged in LDS (each box is read by 2r+1 threads);
+// L lanes a cluster.  A lane a cluster leaves a chain of 32 LDS reads and few
+// waves to hide it up to kPlocSplit clusters, where four share it (50,000
+// clusters: 12 us a round, now 5).
+constexpr uint32_t kPlocSplit = 256 * 1024;
+template <uint32_t L>
+__global__ __launch_bounds__(256) void k_plocNearest(const GBox *cbox, const PlocState *st, uint32_t r, uint32_t *nn) {
+	constexpr uint32_t kTile = 256 / L;
+	constexpr uint32_t kSpan = kTile + 2 * kPlocRadius;
 	__shared__ float tile[kSpan * 6];
-	const uint32_t t0 = blockIdx.x * kPlocTile;
+	const uint32_t t0 = blockIdx.x * kTile;
 	const PlocState s = plocRound(st, r);
 	const uint32_t nc = s.forced ? 0u : s.nc;
 	if (t0 >= nc) return;
 	const int64_t base = (int64_t)t0 - kPlocRadius;  // cluster of tile entry 0
 	const float *src = reinterpret_cast<const float *>(cbox);
-	for (uint32_t k = threadIdx.x; k < kSpan * 6; k += kPlocTile) {
+	for (uint32_t k = threadIdx.x; k < kSpan * 6; k += 256) {
 		const int64_t j = base + k / 6;
 		tile[k] = (j >= 0 && j < (int64_t)nc) ? src[j * 6 + k % 6] : 0.f;
 	}
 	__syncthreads();
-	const uint32_t i = t0 + threadIdx.x;
-	if (i >= nc) return;
+	const uint32_t i = t0 + threadIdx.x / L;
 	const GBox *lds = reinterpret_cast<const GBox *>(tile);
-	nn[i] = plocNearestAt([&](uint32_t j) -> const GBox & { return lds[(int64_t)j - base]; }, nc, i, kPlocRadius);
+	const uint32_t x = plocNearestLanes<L>([&](uint32_t j) -> const GBox & { return lds[(int64_t)j - base]; }, nc, i,
+			threadIdx.x % L);
+	if (i < nc && threadIdx.x % L == 0) nn[i] = x;
 }
 
 // partners and each cluster's place among the survivors and among the new
@@ -517,11 +568,11 @@ __global__ __launch_bounds__(256) void k_plocMark(const uint32_t *nn, const Ploc
 
 // block sums to block starts, and the next round's state
 __global__ __launch_bounds__(1024) void k_plocScan(uint32_t *leadSums, uint32_t *keepSums, PlocState *st, uint32_t r,
-		uint32_t ni, uint32_t *err) {
+		uint32_t ni, PlocState *host, uint32_t *err) {
 	__shared__ uint32_t lds[16];
 	const PlocState s = plocRound(st, r);
 	if (s.nc == 0) {
-		if (threadIdx.x == 0) st[r + 1] = st[r];
+		if (threadIdx.x == 0) st[r + 1] = *host = st[r];
 		return;
 	}
 	const uint32_t nb = (s.nc + 255u) / 256u;
@@ -533,7 +584,7 @@ __global__ __launch_bounds__(1024) void k_plocScan(uint32_t *leadSums, uint32_t 
 			atomicOr(err, kErrCluster);
 			t = {0u, s.nodeBase, 0u, 0u};
 		}
-		st[r + 1] = t;
+		st[r + 1] = *host = t;
 	}
 }
 
@@ -586,7 +637,17 @@ __global__ __launch_bounds__(256) void k_plocApply(const uint32_t *nn, const Plo
 // The last kPlocTail clusters by one block, all their rounds in LDS with
 // barriers: 46 rounds of a 50,000-triangle mesh were 46 times six launches
 // and a wait for the host, most of them for a few hundred clusters.  Each
-// thread has two clusters; a round is the one of the kernels above.
+// thread has two clusters; a round is the one of the kernels above, its
+// neighbour search with more lanes a cluster as clusters get fewer (the tail of
+// 50,000 triangles: 283 us, now 196).
+template <uint32_t L>
+__device__ __forceinline__ void plocTailNearest(const GBox *box, uint32_t nc, uint32_t *nn) {
+	for (uint32_t b = 0; b < nc; b += 1024 / L) {
+		const uint32_t i = b + threadIdx.x / L;
+		const uint32_t x = plocNearestLanes<L>([&](uint32_t j) -> const GBox & { return box[j]; }, nc, i, threadIdx.x % L);
+		if (i < nc && threadIdx.x % L == 0) nn[i] = x;
+	}
+}
 __global__ __launch_bounds__(1024) void k_plocTail(PlocState *st, uint32_t r0, uint32_t ni, const uint32_t *cidIn,
 		const GBox *cboxIn, PlocTree T, uint32_t *rounds, uint32_t *err) {
 	__shared__ GBox box[kPlocTail];
@@ -605,9 +666,11 @@ __global__ __launch_bounds__(1024) void k_plocTail(PlocState *st, uint32_t r0, u
 	__syncthreads();
 	const uint32_t i0 = 2u * threadIdx.x;
 	while (s.nc > 1 && r < kPlocMaxRounds) {
-		if (!s.forced)
-			for (uint32_t i = threadIdx.x; i < s.nc; i += 1024)
-				nn[i] = plocNearestAt([&](uint32_t j) -> const GBox & { return box[j]; }, s.nc, i, kPlocRadius);
+		if (!s.forced) {
+			if (s.nc <= 256) plocTailNearest<16>(box, s.nc, nn);
+			else if (s.nc <= 1024) plocTailNearest<4>(box, s.nc, nn);
+			else plocTailNearest<1>(box, s.nc, nn);
+		}
 		__syncthreads();
 		// this thread's two places: their partners and flags, scanned over the block
 		uint32_t part[2], v[2], sum = 0;
@@ -953,11 +1016,13 @@ inline unsigned grid(size_t n, unsigned b) { return (unsigned)((n + b - 1) / b);
 // one stable pass of the radix sort over the eight bits from `shift`
 void sortPass(const uint64_t *kIn, const uint32_t *vIn, uint32_t n, uint32_t shift, uint32_t *table, uint32_t *totals,
 		uint64_t *kOut, uint32_t *vOut, uint32_t *err, hipStream_t st) {
-	const uint32_t tiles = grid(n, kSortTile);
-	hipLaunchKernelGGL(k_sortCount, dim3(tiles), dim3(kSortBlock), 0, st, kIn, n, shift, tiles, table);
+	const uint32_t tiles = sortTiles(n);
+	const bool small = n <= kSortSmall;
+	hipLaunchKernelGGL(small ? k_sortCount<kSortTileSmall> : k_sortCount<kSortTile>, dim3(tiles), dim3(kSortBlock), 0, st,
+			kIn, n, shift, tiles, table);
 	hipLaunchKernelGGL(k_scanRows, dim3(256), dim3(256), 0, st, table, tiles, totals);
-	hipLaunchKernelGGL(k_sortScatter, dim3(tiles), dim3(kSortBlock), 0, st, kIn, vIn, n, shift, tiles, table, totals, kOut,
-			vOut, err);
+	hipLaunchKernelGGL(small ? k_sortScatter<kSortTileSmall> : k_sortScatter<kSortTile>, dim3(tiles), dim3(kSortBlock), 0,
+			st, kIn, vIn, n, shift, tiles, table, totals, kOut, vOut, err);
 	GB_CHECK(hipGetLastError());
 }
 
@@ -993,7 +1058,7 @@ std::string errorText(uint32_t e) {
 void boxesByPrefix(Scratch &S, const GBox *boxes, const uint32_t *vals, uint32_t n, const uint32_t *left,
 		const uint32_t *right, const uint32_t *first, const uint32_t *last, const uint64_t *digits, const uint32_t *ids,
 		uint32_t maxLeaf, float ci, hipStream_t st, uint32_t *err, GBox *leafBox, GBox *nodeBox, float *key) {
-	const uint32_t ni = n - 1, tiles = grid(ni, kSortTile);
+	const uint32_t ni = n - 1, tiles = sortTiles(ni);
 	uint32_t *order = S.get<uint32_t>(ni), *starts = S.get<uint32_t>(256), *totals = S.get<uint32_t>(256);
 	uint64_t *digitsOut = S.get<uint64_t>(ni);
 	uint32_t *table = S.get<uint32_t>((size_t)256 * tiles);
@@ -1048,29 +1113,31 @@ void plocTree(Scratch &S, const GBox *boxes, uint32_t n, uint32_t maxLeaf, float
 	GBox *cboxA = S.get<GBox>(n), *cboxB = S.get<GBox>(n);
 	uint32_t *leadSums = S.get<uint32_t>(grid(n, 256)), *keepSums = S.get<uint32_t>(grid(n, 256));
 	PlocState *state = S.get<PlocState>(kPlocMaxRounds + 1);
-	uint32_t *rounds = S.get<uint32_t>(1);
 	PlocTree T = {S.get<uint32_t>(ni), S.get<uint32_t>(ni), S.get<uint32_t>(ni), S.get<GBox>(ni), S.get<float>(ni),
 			S.get<float>(ni), leafBox, maxLeaf, ci};
 	hipLaunchKernelGGL(k_plocInit, dim3(grid(n, 256)), dim3(256), 0, st, boxes, vals, n, cidA, cboxA, leafBox, state);
 	GB_CHECK(hipGetLastError());
 	std::vector<PlocState> host(kPlocMaxRounds + 1);
+	host[0] = {n, 0u, 0u, 0u};
+	PlocState *seen = reinterpret_cast<PlocState *>(S.pin + 8);
 	uint32_t r = 0, ub = n;
 	while (ub > kPlocTail) {
 		for (uint32_t k = 0; k < kPlocBatch; ++k, ++r) {
 			if (r >= kPlocMaxRounds) throw std::runtime_error("device build: clustering did not converge");
-			hipLaunchKernelGGL(k_plocNearest, dim3(grid(ub, kPlocTile)), dim3(kPlocTile), 0, st, cboxA, state, r, nn);
+			if (ub <= kPlocSplit)
+				hipLaunchKernelGGL(k_plocNearest<4>, dim3(grid(ub, 64)), dim3(256), 0, st, cboxA, state, r, nn);
+			else
+				hipLaunchKernelGGL(k_plocNearest<1>, dim3(grid(ub, 256)), dim3(256), 0, st, cboxA, state, r, nn);
 			hipLaunchKernelGGL(k_plocMark, dim3(grid(ub, 256)), dim3(256), 0, st, nn, state, r, prefix, leadSums, keepSums);
-			hipLaunchKernelGGL(k_plocScan, dim3(1), dim3(1024), 0, st, leadSums, keepSums, state, r, ni, err);
+			hipLaunchKernelGGL(k_plocScan, dim3(1), dim3(1024), 0, st, leadSums, keepSums, state, r, ni, seen + k, err);
 			hipLaunchKernelGGL(k_plocApply, dim3(grid(ub, 256)), dim3(256), 0, st, nn, state, r, cidA, cboxA, prefix,
 					leadSums, keepSums, ni, cidB, cboxB, T);
 			GB_CHECK(hipGetLastError());
 			std::swap(cidA, cidB);
 			std::swap(cboxA, cboxB);
 		}
-		GB_CHECK(hipMemcpyAsync(S.pin + 8, state + (r - kPlocBatch), (kPlocBatch + 1) * sizeof(PlocState),
-				hipMemcpyDeviceToHost, st));
 		if (const uint32_t e = readError(S, err, st)) throw std::runtime_error(errorText(e));
-		std::copy_n(reinterpret_cast<const PlocState *>(S.pin + 8), kPlocBatch + 1, host.begin() + (r - kPlocBatch));
+		std::copy_n(seen, kPlocBatch, host.begin() + (r - kPlocBatch + 1));
 		ub = host[r].nc;
 	}
 	// the rounds after the count fell to the tail's changed nothing but the
@@ -1081,8 +1148,7 @@ void plocTree(Scratch &S, const GBox *boxes, uint32_t n, uint32_t maxLeaf, float
 		std::swap(cidA, cidB);
 		std::swap(cboxA, cboxB);
 	}
-	hipLaunchKernelGGL(k_plocTail, dim3(1), dim3(1024), 0, st, state, r0, ni, cidA, cboxA, T, rounds, err);
-	GB_CHECK(hipMemcpyAsync(S.pin + 1, rounds, 4, hipMemcpyDeviceToHost, st));
+	hipLaunchKernelGGL(k_plocTail, dim3(1), dim3(1024), 0, st, state, r0, ni, cidA, cboxA, T, S.pin + 1, err);
 	if (const uint32_t e = readError(S, err, st)) throw std::runtime_error(errorText(e));
 	const uint32_t r1 = S.pin[1];
 	*roundsOut = r1;
@@ -1164,7 +1230,7 @@ void lrhGpuBuildBVH(const LrhGpuBuildIn &in, const LrhGpuAlloc &a, hipStream_t s
 			GB_CHECK(hipGetLastError());
 			// stable LSD radix sort, 8 passes of 8 bits; an even number of
 			// passes leaves the result in keys / vals
-			uint32_t *table = S.get<uint32_t>((size_t)256 * grid(n, kSortTile)), *totals = S.get<uint32_t>(256);
+			uint32_t *table = S.get<uint32_t>((size_t)256 * sortTiles(n)), *totals = S.get<uint32_t>(256);
 			uint64_t *kIn = keys, *kOut = keysB;
 			uint32_t *vIn = vals, *vOut = valsB;
 			for (uint32_t shift = 0; shift < 64; shift += 8) {
@@ -1182,7 +1248,6 @@ void lrhGpuBuildBVH(const LrhGpuBuildIn &in, const LrhGpuAlloc &a, hipStream_t s
 			GBox *nodeBox = S.get<GBox>(ni);
 			float *key = S.get<float>(ni);
 			if (in.method == 1) {
-				if (const uint32_t e = readError(S, err, st)) throw std::runtime_error(errorText(e));
 				plocTree(S, boxes, n, in.maxLeaf, in.travCost, st, err, vals, leafBox, left, right, first, last, nodeBox, key,
 						&out->plocRounds);
 			} else {

@@ -125,13 +125,15 @@ def _build_edge_scene(kind, n):
 @pytest.mark.parametrize("builder", list(BUILDERS))
 @pytest.mark.parametrize("kind,n,layout,max_leaf", [
     ("spread", 2, 2, 1), ("spread", 257, 2, 4), ("spread", 2047, 2, 4), ("spread", 2048, 0, 4), ("spread", 2049, 1, 1),
-    ("spread", 4099, 2, 1), ("spread", 70001, 2, 2), ("copies", 300, 2, 4), ("copies", 9000, 2, 1), ("row", 3000, 0, 1),
+    ("spread", 4099, 2, 1), ("spread", 70001, 2, 2), ("spread", 262145, 2, 4), ("spread", 524288, 2, 4),
+    ("spread", 524289, 2, 4), ("copies", 300, 2, 4), ("copies", 9000, 2, 1), ("row", 3000, 0, 1),
     ("row", 120, 2, 1)])
 def test_device_build_edges_equal_cpu_emulation(gpu_device, emu, tmp_path, kind, n, layout, max_leaf, builder):
     """Node and record bytes equal the emulation's where the build changes its
     launches: clusters around the 2,048 that one block finishes, tree levels
     around the 2,048 nodes that share a launch, levels of one block and of
-    many, odd remainders of the 256-node blocks."""
+    many, odd remainders of the 256-node blocks, the sort's two tiles (524,288
+    keys) and the neighbour search's two splits (262,144 clusters)."""
     from tests.test_lbvh_cpu import run_emu
     _case("devbuild_edges", kind=kind, n=n, layout=layout, max_leaf=max_leaf, builder=builder)
     meshes = _build_edge_scene(kind, n)
