@@ -213,7 +213,11 @@ struct lrh_device {
 	}
 	void pinGive(void *p) {
 		std::lock_guard<std::mutex> g(poolMu);
-		pinPool.push_back(p);
+		try {
+			pinPool.push_back(p);
+		} catch (...) {  // (called while a build's scratch is given back)
+			(void)hipHostFree(p);
+		}
 	}
 	void drainPool() {
 		std::lock_guard<std::mutex> g(poolMu);

@@ -52,10 +52,36 @@ __device__ __forceinline__ void writeMasked(lrh_ray_rec *r) {
 	r->pad[0] = r->pad[1] = 0.f;
 }
 
-__global__ void lrh_camera_kernel(LrhCameraParams C, lrh_ray_rec *rays) {
+// The 48-byte records of a wave's lanes (those in `mask`) to consecutive
+// places, through the wave's 3 KiB of LDS: stored by their own lanes, each of
+// the three store instructions of a record wrote a third of 24 lines, here
+// eight whole lines (the three steps of 921,600 paths: 242 us, 196 with
+// this, 179 with the loads of a step issued together as well; their bytes at
+// the rate of a large copy: 174).  Called by the whole wave.
+struct __attribute__((aligned(4))) Quarter {  // (a caller's records are aligned to their floats)
+	uint32_t w[4];
+};
+template <class Rec>
+__device__ __forceinline__ void storeRecords(uint4 *lds, Rec *dst, const Rec &r, uint64_t mask) {
+	static_assert(sizeof(Rec) == 48, "three 16-byte parts");
+	const uint32_t lane = threadIdx.x & 63u;
+	uint32_t w[12];
+	__builtin_memcpy(w, &r, 48);
+	for (int k = 0; k < 3; ++k) lds[3 * lane + k] = make_uint4(w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]);
+	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+	for (uint32_t k = 0; k < 3; ++k) {
+		const uint32_t c = k * 64 + lane;
+		const uint4 v = lds[c];
+		if ((mask >> (c / 3)) & 1ull) reinterpret_cast<Quarter *>(dst)[c] = Quarter{{v.x, v.y, v.z, v.w}};
+	}
+	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+}
+
+__global__ __launch_bounds__(256) void lrh_camera_kernel(LrhCameraParams C, lrh_ray_rec *rays) {
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
 	const uint32_t n = C.width * C.height;
-	if (i >= n) return;
 	const uint32_t x = i % C.width, y = i / C.width;
 	const float px = ((float)x + 0.5f) / (float)C.width * 2.f - 1.f;
 	const float py = 1.f - ((float)y + 0.5f) / (float)C.height * 2.f;
@@ -70,7 +96,8 @@ __global__ void lrh_camera_kernel(LrhCameraParams C, lrh_ray_rec *rays) {
 	r.time = 0.f;
 	r.flags = 0u;
 	r.pad[0] = r.pad[1] = 0.f;
-	rays[i] = r;
+	__shared__ uint4 stage[4][192];
+	storeRecords(stage[threadIdx.x >> 6], rays + (i - (threadIdx.x & 63u)), r, __ballot(i < n));
 }
 
 // one bounce of ray i; returns the number of live rays it wrote (0..2)
@@ -159,35 +186,43 @@ __device__ __forceinline__ void cosineDir(const float n[3], float u1, float u2, 
 	for (int k = 0; k < 3; ++k) d[k] = v[k] * dl;
 }
 
-__device__ uint32_t shadeOne(const LrhShadeParams &P, uint32_t i) {
-	LrhPath path = P.paths[i];
+struct ShadeOut {
+	LrhPath path;
+	lrh_ray_rec next, shadow;
+	uint32_t live;
+	bool write;
+};
+
+__device__ __forceinline__ void shadeOne(const LrhShadeParams &P, uint32_t i, ShadeOut &O) {
+	O.live = 0;
+	O.write = false;
+	LrhPath &path = O.path;
+	path = P.paths[i];
+	const lrh_ray_rec ray = P.rays[i];
+	lrh_hit_rec hit = P.hits[i];
 	const bool pending = path.dl[0] != 0.f || path.dl[1] != 0.f || path.dl[2] != 0.f;
 	// a path already ended when the previous step ran (pad = 1) and with no
 	// light pending: that step and the one that ended it masked its slots of
 	// both ray buffers and of the shadow buffer, so there is nothing to do
-	if (!path.alive && path.pad && !pending) return 0;
+	if (!path.alive && path.pad && !pending) return;
+	O.write = true;
+	writeMasked(&O.next);
+	writeMasked(&O.shadow);
+	// (keeps the hit's load up here, beside the path's: three dependent waits
+	// on memory were four)
+	asm volatile("" : "+v"(hit.meshIndex), "+v"(hit.triangleIndex), "+v"(hit.t));
 	// the previous step's shadow ray: its light counts if nothing blocked it
 	if (P.shadowHits && pending && P.shadowHits[i].meshIndex == 0xffffffffu)
 		for (int k = 0; k < 3; ++k) path.rad[k] = path.rad[k] + path.dl[k];
 	for (int k = 0; k < 3; ++k) path.dl[k] = 0.f;
-	lrh_ray_rec *next = P.next + i;
-	lrh_ray_rec *shadow = P.shadow + i;
 	if (!path.alive) {
 		path.pad = 1u;
-		writeMasked(next);
-		writeMasked(shadow);
-		P.paths[i] = path;
-		return 0;
+		return;
 	}
-	const lrh_ray_rec ray = P.rays[i];
-	const lrh_hit_rec hit = P.hits[i];
 	if ((ray.flags & 1u) || hit.meshIndex >= P.nMeshes ||
 			hit.triangleIndex >= P.meshTriBase[hit.meshIndex + 1] - P.meshTriBase[hit.meshIndex]) {
 		path.alive = 0u;
-		writeMasked(next);
-		writeMasked(shadow);
-		P.paths[i] = path;
-		return 0;
+		return;
 	}
 	LrhMaterial m;
 	if (hit.meshIndex < P.nMaterials)
@@ -208,8 +243,6 @@ __device__ uint32_t shadeOne(const LrhShadeParams &P, uint32_t i) {
 	if (depth == 0)  // a light seen directly
 		for (int k = 0; k < 3; ++k) path.rad[k] = path.rad[k] + path.thr[k] * m.le[k];
 	const bool diffuse = m.kd[0] > 0.f || m.kd[1] > 0.f || m.kd[2] > 0.f;
-	uint32_t live = 0;
-	bool shadowWritten = false;
 	if (P.nLights && diffuse) {
 		const float u0 = rnd(P.seed, pix, depth, 3), u1 = rnd(P.seed, pix, depth, 4), u2 = rnd(P.seed, pix, depth, 5);
 		uint32_t j = (uint32_t)(u0 * (float)P.nLights);
@@ -239,12 +272,10 @@ __device__ uint32_t shadeOne(const LrhShadeParams &P, uint32_t i) {
 			o.time = ray.time;
 			o.flags = 0u;
 			o.pad[0] = o.pad[1] = 0.f;
-			*shadow = o;
-			shadowWritten = true;
-			++live;
+			O.shadow = o;
+			++O.live;
 		}
 	}
-	if (!shadowWritten) writeMasked(shadow);
 	const uint32_t depth1 = depth + 1;
 	bool alive = depth1 < P.maxDepth && diffuse;
 	if (alive && depth1 >= P.rrDepth) {
@@ -266,14 +297,11 @@ __device__ uint32_t shadeOne(const LrhShadeParams &P, uint32_t i) {
 		o.time = ray.time;
 		o.flags = 0u;
 		o.pad[0] = o.pad[1] = 0.f;
-		*next = o;
-		++live;
-	} else
-		writeMasked(next);
+		O.next = o;
+		++O.live;
+	}
 	path.depth = depth1;
 	path.alive = alive ? 1u : 0u;
-	P.paths[i] = path;
-	return live;
 }
 
 __device__ __forceinline__ void countLive(uint32_t *counter, uint32_t live) {
@@ -290,28 +318,41 @@ __global__ void lrh_bounce_kernel(LrhBounceParams P) {
 	countLive(P.liveCount, live);
 }
 
-__global__ void lrh_shade_kernel(LrhShadeParams P) {
+__device__ __forceinline__ uint32_t shadeWave(const LrhShadeParams &P, uint32_t i) {
+	__shared__ uint4 stage[4][192];
+	ShadeOut O;
+	O.live = 0;
+	O.write = false;
+	if (i < P.count) shadeOne(P, i, O);
+	const uint64_t mask = __ballot(O.write);
+	if (!mask) return 0;
+	const uint32_t first = i - (threadIdx.x & 63u);
+	uint4 *lds = stage[threadIdx.x >> 6];
+	storeRecords(lds, P.next + first, O.next, mask);
+	storeRecords(lds, P.shadow + first, O.shadow, mask);
+	storeRecords(lds, P.paths + first, O.path, mask);
+	return O.live;
+}
+
+__global__ __launch_bounds__(256) void lrh_shade_kernel(LrhShadeParams P) {
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-	uint32_t live = 0;
-	if (i < P.count) live = shadeOne(P, i);
+	const uint32_t live = shadeWave(P, i);
 	countLive(P.liveCount, live);
 }
 
-__global__ void lrh_shade_batch_kernel(LrhShadeBatchArgs A) {
+__global__ __launch_bounds__(256) void lrh_shade_batch_kernel(LrhShadeBatchArgs A) {
 	// the item of this block (uniform over the block: scalar loads of the
 	// kernel arguments)
 	uint32_t k = 0;
 	while (k + 1 < A.n && blockIdx.x >= A.blockStart[k + 1]) ++k;
 	const LrhShadeParams &P = A.p[k];
 	const uint32_t i = (blockIdx.x - A.blockStart[k]) * blockDim.x + threadIdx.x;
-	uint32_t live = 0;
-	if (i < P.count) live = shadeOne(P, i);
+	const uint32_t live = shadeWave(P, i);
 	countLive(P.liveCount, live);
 }
 
-__global__ void lrh_paths_init_kernel(LrhPath *paths, uint32_t count) {
+__global__ __launch_bounds__(256) void lrh_paths_init_kernel(LrhPath *paths, uint32_t count) {
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= count) return;
 	LrhPath p;
 	for (int k = 0; k < 3; ++k) {
 		p.thr[k] = 1.f;
@@ -321,7 +362,8 @@ __global__ void lrh_paths_init_kernel(LrhPath *paths, uint32_t count) {
 	p.depth = 0u;
 	p.alive = 1u;
 	p.pad = 0u;
-	paths[i] = p;
+	__shared__ uint4 stage[4][192];
+	storeRecords(stage[threadIdx.x >> 6], paths + (i - (threadIdx.x & 63u)), p, __ballot(i < count));
 }
 
 }  // namespace

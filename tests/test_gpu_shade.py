@@ -161,3 +161,50 @@ def test_shade_batch_equals_per_buffer_shading(gpu_device, tmp_path):
     with pytest.raises(D.LrhError, match="LRH_SHADE_BATCH_MAX"):
         dev.shade_batch([items[0]] * (D.SHADE_BATCH_MAX + 1), mb, len(mats), lb, len(lights))
     scene.close()
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 257, 1000])
+def test_shade_ragged_counts_write_their_records_only(gpu_device, tmp_path, n):
+    """Waves and blocks that end inside the records: camera rays, fresh paths
+    and two shading steps of n paths are the first n of 1,024's, record by
+    record, and nothing beyond is written; a path that ended a step before
+    keeps its slots (its lane takes no part in its wave's stores)."""
+    print(f"[case] shade ragged {n}", flush=True)
+    sf = _scene(tmp_path)
+    dev = gpu_device
+    scene = P.scene_on_device(dev, sf)
+    mats, lights = sf.materials(), sf.light_triangles()
+    mb, lb = dev.upload(mats), dev.upload(lights)
+    orig, target, up, fov = sf.camera
+    full, guard = 1024, np.full(1024 * 12, 0x5a5a5a5a, np.uint32)
+
+    def step(count, rb, hb, pb):
+        nb, sb = dev.upload(guard), dev.upload(guard)
+        dev.shade(scene, mb, len(mats), lb, len(lights), rb, hb, None, pb, nb, sb, count, max_depth=2, rr_depth=0,
+                  rr_survive=0.5, seed=9)
+        dev.sync()
+        return [dev.download(b, np.uint32, full * 12).reshape(full, 12) for b in (pb, nb, sb)]
+
+    hb = dev.alloc(full * 20)
+    rays = dev.upload(guard)
+    dev.camera_rays(rays, orig, target, up, fov, full // 32, 32)
+    dev.trace(scene, rays, hb, full, 0)
+    outs = {}
+    for count in (full, n):
+        pb = dev.upload(guard)
+        dev.paths_init(pb, count)
+        dev.sync()
+        outs[count] = [[dev.download(pb, np.uint32, full * 12).reshape(full, 12)]]
+        for _ in range(3):  # two steps end every path, the third finds them ended
+            outs[count].append(step(count, rays, hb, pb))
+    for a, b in zip(outs[full], outs[n]):
+        for x, y in zip(a, b):
+            assert np.array_equal(x[:n], y[:n])
+            assert n == full or (y[n:] == 0x5a5a5a5a).all()
+    one = dev.upload(guard)
+    dev.camera_rays(one, orig, target, up, fov, n, 1)
+    dev.sync()
+    got = dev.download(one, np.uint32, full * 12).reshape(full, 12)
+    assert (got[n:] == 0x5a5a5a5a).all()
+    assert (got[:n, 9] == 0).all() and np.array_equal(got[:n, :3], np.tile(got[0, :3], (n, 1)))
+    scene.close()
