@@ -227,7 +227,7 @@ def extra_workloads(args, dev):
     scs = wl.scenes
     for rbuf in wl.ray_bufs + wl.hit_bufs:
         rbuf.free()
-    sopts = D.trace_opts(256, 8, 0, 12)
+    sopts = D.trace_opts(256, 8, 0, 40)
     w = serve.Server(dev, scs, opts=sopts)
     w.run(serve.poisson_specs(1000.0, 0.004, len(scs), seed=99))
     w.close()

@@ -147,7 +147,7 @@ typedef struct {
 	unsigned int blocksPerCU;
 	unsigned int refillThreshold;  /* refill a wave when fewer than this many lanes are live; 0 = default */
 	unsigned int leafTris;         /* triangles a lane tests per traversal pass; the rest of its leaf waits
-	                                  for the next pass; 0 = default (the whole leaf) */
+	                                  for the next pass; 0 = default (two; the whole leaf in two-level scenes) */
 	unsigned int gridPercent;      /* share of the occupancy-derived grid (blocksPerCU 0); 0 = 100 */
 } lrh_trace_opts;
 
@@ -456,7 +456,7 @@ int lrh_server_plain_batch(lrh_server *srv, const lrh_trace_opts *opts, unsigned
 int lrh_server_destroy(lrh_server *srv);
 /* Launch-shape autotuner of a batched trace: times each candidate shape
  * (NULL: the LRH_AUTOTUNE_SHAPES built-in ones, block size {128, 256} x LDS
- * stack {4, 8, 16} x refill threshold {4, 8, 12, 16, 24}) on the actual items
+ * stack {4, 8, 16} x refill threshold {8, 12, 16, 24, 40}) on the actual items
  * (resident batches, median of 3 launches after 2 warm-ups) and keeps the
  * fastest; candidateMs (optional, one per candidate) gets each time, NaN for
  * a shape the device refuses.  With cachePath and key (no spaces), the result

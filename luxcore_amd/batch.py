@@ -23,7 +23,7 @@ from . import device as D
 DEFAULT_CACHE = os.path.join(os.path.expanduser("~"), ".cache", "lrhip", "autotune.txt")
 
 # the library's built-in candidates (LRH_AUTOTUNE_SHAPES of them), in its order
-SHAPES = [(b, l, r) for b, l, r in itertools.product((128, 256), (4, 8, 16), (4, 8, 12, 16, 24))]
+SHAPES = [(b, l, r) for b, l, r in itertools.product((128, 256), (4, 8, 16), (8, 12, 16, 24, 40))]
 
 
 def signature(dev, scenes_info, counts, extra=""):

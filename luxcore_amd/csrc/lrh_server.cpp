@@ -785,7 +785,7 @@ int lrh_autotune_batch(lrh_device *dev, const lrh_batch_item *items, unsigned in
 		} else {
 			for (unsigned blk : {128u, 256u})
 				for (unsigned lds : {4u, 8u, 16u})
-					for (unsigned ref : {4u, 8u, 12u, 16u, 24u}) {
+					for (unsigned ref : {8u, 12u, 16u, 24u, 40u}) {
 						lrh_trace_opts o{};
 						o.blockSize = blk;
 						o.ldsStack = lds;
