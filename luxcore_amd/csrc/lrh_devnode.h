@@ -160,27 +160,49 @@ LRH_DN inline void floatNode(const GBox *cb, int n, const uint32_t child[4], lrh
 }
 
 #if defined(__HIPCC__)
-// The same node written by W neighbouring lanes of a wave, lane c (0..W-1)
-// with child c: one lane per child instead of one thread per node, whose
-// children's roundings (a division and a few compares each, six per child)
-// would run one after another.  All W lanes call it together; lane c < n has
-// the child's box and reference, the others pass any box and
-// LRH_CHILD_EMPTY.  Returns the union of the boxes to all of them: min and
-// max are exact, so its order does not show in the bytes, and a NaN bound (a
-// triangle of NaN vertices, which no ray meets) is left out of it.
-template <int W, class Node>
-__device__ inline GBox quantizeNodeLanes(const GBox &b, int c, int n, uint32_t child, Node *out) {
-	GBox u = b;
-	for (int k = 0; k < 3; ++k) {
-		if (c >= n) {
+// Union of the boxes of the first n of W neighbouring lanes (lane c, 0..W-1,
+// with box c), to all of them: the sequential writers' fold by minT and maxT.
+// Min and max of numbers are exact in any order; a NaN (a triangle of NaN
+// vertices) hides the boxes before it from the fold and is kept only from
+// the last place, and zeros of either sign are equal, so a wave that holds
+// one takes the boxes in order.
+template <int W>
+__device__ inline GBox unionLanes(const GBox &b, int c, int n) {
+	bool inOrder = false;
+	for (int k = 0; k < 3; ++k) inOrder |= c < n && !(fabsf(b.lo[k]) > 0.f && fabsf(b.hi[k]) > 0.f);
+	GBox u;
+	if (__ballot(inOrder)) {
+		for (int k = 0; k < 3; ++k) {
 			u.lo[k] = INFINITY;
 			u.hi[k] = -INFINITY;
+			for (int j = 0; j < W; ++j) {
+				const float lo = __shfl(b.lo[k], j, W), hi = __shfl(b.hi[k], j, W);
+				u.lo[k] = j < n ? minT(u.lo[k], lo) : u.lo[k];
+				u.hi[k] = j < n ? maxT(u.hi[k], hi) : u.hi[k];
+			}
 		}
+		return u;
+	}
+	for (int k = 0; k < 3; ++k) {
+		u.lo[k] = c < n ? b.lo[k] : INFINITY;
+		u.hi[k] = c < n ? b.hi[k] : -INFINITY;
 		for (int o = W / 2; o > 0; o >>= 1) {
 			u.lo[k] = fminf(__shfl_xor(u.lo[k], o), u.lo[k]);
 			u.hi[k] = fmaxf(__shfl_xor(u.hi[k], o), u.hi[k]);
 		}
 	}
+	return u;
+}
+
+// The same node written by W neighbouring lanes of a wave, lane c (0..W-1)
+// with child c: one lane per child instead of one thread per node, whose
+// children's roundings (a division and a few compares each, six per child)
+// would run one after another.  All W lanes call it together; lane c < n has
+// the child's box and reference, the others pass any box and
+// LRH_CHILD_EMPTY.  Returns the union of the boxes to all of them.
+template <int W, class Node>
+__device__ inline GBox quantizeNodeLanes(const GBox &b, int c, int n, uint32_t child, Node *out) {
+	const GBox u = unionLanes<W>(b, c, n);
 	uint8_t *const qlo[3] = {out->qlo_x, out->qlo_y, out->qlo_z};
 	uint8_t *const qhi[3] = {out->qhi_x, out->qhi_y, out->qhi_z};
 	for (int k = 0; k < 3; ++k) {
@@ -203,22 +225,12 @@ __device__ inline GBox quantizeNodeLanes(const GBox &b, int c, int n, uint32_t c
 
 // the fp32 node (lrh_node4f) by four lanes, likewise
 __device__ inline GBox floatNodeLanes(const GBox &b, int c, int n, uint32_t child, lrh_node4f *out) {
-	GBox u = b;
-	for (int k = 0; k < 3; ++k)
-		if (c >= n) {
-			u.lo[k] = INFINITY;
-			u.hi[k] = -INFINITY;
-		}
-	out->lo_x[c] = u.lo[0]; out->lo_y[c] = u.lo[1]; out->lo_z[c] = u.lo[2];
-	out->hi_x[c] = u.hi[0]; out->hi_y[c] = u.hi[1]; out->hi_z[c] = u.hi[2];
+	const bool some = c < n;
+	out->lo_x[c] = some ? b.lo[0] : INFINITY; out->lo_y[c] = some ? b.lo[1] : INFINITY; out->lo_z[c] = some ? b.lo[2] : INFINITY;
+	out->hi_x[c] = some ? b.hi[0] : -INFINITY; out->hi_y[c] = some ? b.hi[1] : -INFINITY; out->hi_z[c] = some ? b.hi[2] : -INFINITY;
 	out->child[c] = child;
 	out->pad[c] = 0;
-	for (int k = 0; k < 3; ++k)
-		for (int o = 2; o > 0; o >>= 1) {
-			u.lo[k] = fminf(__shfl_xor(u.lo[k], o), u.lo[k]);
-			u.hi[k] = fmaxf(__shfl_xor(u.hi[k], o), u.hi[k]);
-		}
-	return u;
+	return unionLanes<4>(b, c, n);
 }
 #endif
 

@@ -148,6 +148,28 @@ def test_device_build_edges_equal_cpu_emulation(gpu_device, emu, tmp_path, kind,
 
 
 @pytest.mark.parametrize("builder", list(BUILDERS))
+@pytest.mark.parametrize("layout", [0, 1, 2])
+def test_device_build_of_nan_vertices_equals_cpu_emulation(gpu_device, emu, tmp_path, layout, builder):
+    """Triangles with a NaN coordinate bring NaN bounds into nodes at every
+    height: a node's frame is what the sequential writer makes of them."""
+    from tests.test_lbvh_cpu import run_emu
+    _case("devbuild_nan", layout=layout, builder=builder)
+    mesh = _build_edge_scene("spread", 3001)[0]
+    rng = np.random.default_rng(7)
+    for t in rng.choice(3001, 40, replace=False):
+        mesh.verts[mesh.tris[t, rng.integers(3)], rng.integers(3)] = np.nan
+    info, nodes, tris = run_emu(emu, tmp_path, [mesh], 2, layout, method=builder)
+    assert info["err"] == 0
+    dsc = gpu_device.scene_bvh([mesh], layout=layout, max_leaf=2, builder=BUILDERS[builder])
+    nb, pb = dsc.download()
+    assert nb.tobytes() == nodes.tobytes()
+    recs = pb.view(TRI)
+    for field in TRI.names:   # (the sign of an edge's NaN is the processor's)
+        assert np.array_equal(recs[field], tris[field], equal_nan=recs[field].dtype.kind == "f")
+    dsc.close()
+
+
+@pytest.mark.parametrize("builder", list(BUILDERS))
 @pytest.mark.parametrize("n", [1, 3, 257, 5000])
 def test_device_build_refuses_vertex_index(gpu_device, n, builder):
     """An index at the end of its mesh (a valid vertex of the next one, or the
