@@ -211,8 +211,10 @@ DEVI void testNodeF(const lrh_node4f *__restrict__ nodes, uint32_t idx, const Lo
 // those of a finite double, and no distance is a NaN), and a comparator is one
 // v_min_f64 and one v_max_f64, each issued in 4 cycles like any fp32 minimum,
 // where comparing and exchanging two registers takes one compare and four
-// selects of 4 cycles each.  Equal distances order by reference, not by the
-// network, which a closest hit does not see.
+// selects of 4 cycles each.  Equal distances order by reference.  Of hits at
+// the same distance the first one tested is reported, so every kernel and the
+// drain visit a closest ray's children in this order (and an any-hit ray's in
+// the network's): its hit is then its own, whatever launch it is part of.
 DEVI double key64(float t, uint32_t c) { return __hiloint2double((int)asu(t), (int)c); }
 DEVI float keyT(double k) { return asf((uint32_t)__double2hiint(k)); }
 DEVI uint32_t keyC(double k) { return (uint32_t)__double2loint(k); }
@@ -478,14 +480,17 @@ DEVI uint32_t dpp(uint32_t x) {
 }
 constexpr int kXor1 = 0xb1, kXor2 = 0x4e, kXor3 = 0x1b, kHalfMirror = 0x141;  // quad_perm, row_half_mirror
 
-// how many of the group's W keys are below this lane's
+// how many of the group's W keys (key64) are below this lane's
+template <int CTRL>
+DEVI double dppKey(double k) {
+	return __hiloint2double((int)dpp<CTRL>((uint32_t)__double2hiint(k)), (int)dpp<CTRL>((uint32_t)__double2loint(k)));
+}
 template <int W>
-DEVI uint32_t groupRank(int key) {
-	const uint32_t k = (uint32_t)key;
-	uint32_t n = ((int)dpp<kXor1>(k) < key) + ((int)dpp<kXor2>(k) < key) + ((int)dpp<kXor3>(k) < key);
+DEVI uint32_t groupRank(double key) {
+	uint32_t n = (dppKey<kXor1>(key) < key) + (dppKey<kXor2>(key) < key) + (dppKey<kXor3>(key) < key);
 	if (W == 8) {
-		const uint32_t m = dpp<kHalfMirror>(k);
-		n += ((int)m < key) + ((int)dpp<kXor1>(m) < key) + ((int)dpp<kXor2>(m) < key) + ((int)dpp<kXor3>(m) < key);
+		const double m = dppKey<kHalfMirror>(key);
+		n += (m < key) + (dppKey<kXor1>(m) < key) + (dppKey<kXor2>(m) < key) + (dppKey<kXor3>(m) < key);
 	}
 	return n;
 }
@@ -683,12 +688,12 @@ DEVI void drain(const LrhTraceParams &P, Stack &st, SceneView &v, LocalRay &r, f
 			// (INFINITY is a miss, as in the tests by lane: a hit's key lies below every miss's)
 			const bool hit = a <= b && a < INFINITY && child != LRH_CHILD_EMPTY;
 			const uint32_t n = (uint32_t)__popc((uint32_t)(__ballot(hit) >> (lane & ~(W - 1u))) & ((1u << W) - 1u));
-			if (ANY) {
+			if (anyq) {
 				float t = hit ? a : INFINITY;
 				groupSort<W>(c, t, child);
 				drainPush(st, c < n, st.sp + (n - 1u - c), st.sp + n, child, t, P.error);
 			} else {
-				const uint32_t rank = groupRank<W>((int)(hit ? (asu(a) & ~7u) | c : 0x7f800000u | c));
+				const uint32_t rank = groupRank<W>(key64(hit ? a : INFINITY, child));
 				drainPush(st, hit, st.sp + (n - 1u - rank), st.sp + n, child, a, P.error);
 			}
 			if (__ballot(st.sp + n > st.depth)) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // spilled entries written by other lanes
@@ -972,8 +977,11 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 					float t8[8];
 					uint32_t c8[8];
 					testNode8Q(reinterpret_cast<const lrh_node8q *>(v.nodes), cur, r, mint, best, t8, c8);
-					// an any-hit ray reports the first blocker it meets: its order is kept to the network's
-					if (ANY) sort8(t8, c8);
+					// an any-hit ray reports the first blocker it meets: its order is kept to the
+					// network's.  In a batch of both kinds each ray takes its own sort: 899 us for
+					// 3.9M rays, where one network whose comparators also compare a closest ray's
+					// references takes 944 (and the network alone, with no order of ties, 889).
+					if (ANY && (!BATCH || (v.flags & LRH_ITEM_ANY))) sort8(t8, c8);
 					else sort8Closest(t8, c8);
 					bool ok = true;
 					// sorted: the lanes that push entry k also push k-1..1; a
@@ -996,7 +1004,7 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 					testNodeQ(reinterpret_cast<const lrh_node4q *>(v.nodes), cur, r, mint, best, t4, c4);
 				else
 					testNodeF(reinterpret_cast<const lrh_node4f *>(v.nodes), cur, r, mint, best, t4, c4);
-				if (ANY) sort4(t4, c4);
+				if (ANY && (!BATCH || (v.flags & LRH_ITEM_ANY))) sort4(t4, c4);
 				else sort4Closest(t4, c4);
 				bool ok = true;
 				if (t4[3] != INFINITY) ok = ok && push(st, c4[3], t4[3], P.error);
