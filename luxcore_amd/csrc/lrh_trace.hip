@@ -29,11 +29,18 @@
 #include "lrh_layout.h"
 #include "lrh_kernels.h"
 #include "lrh_motion_dev.h"
+#include "lrh_stack.h"
 
 #define LRH_SENTINEL 0xfffffffeu
 #define DEVI __device__ __forceinline__
 
 namespace {
+
+using Stack = lrhstack::Stack<uint2>;
+using lrhstack::drainPop;
+using lrhstack::drainPush;
+using lrhstack::overfull;
+using lrhstack::pop;
 
 DEVI float asf(uint32_t u) { return __uint_as_float(u); }
 DEVI uint32_t asu(float f) { return __float_as_uint(f); }
@@ -306,41 +313,8 @@ DEVI void sort8Closest(float t[8], uint32_t c[8]) {
 	for (int i = 0; i < 8; ++i) { t[i] = keyT(k[i]); c[i] = keyC(k[i]); }
 }
 
-// ---- stack: top ldsDepth entries in LDS (ring), the rest spilled ----
-struct Stack {
-	uint2 *lds;
-	uint2 *spill;
-	uint32_t shift;     // log2 of blockDim
-	uint32_t lane;      // threadIdx / global lane
-	uint32_t gstride;
-	uint32_t glane0;    // of thread 0: the spill column is glane0 + lane
-	uint32_t mask;      // ldsDepth - 1
-	uint32_t depth;     // ldsDepth
-	uint32_t spillDepth;
-	uint32_t sp;
-};
-
 DEVI bool push(Stack &s, uint32_t ref, float t, uint32_t *err) {
-	uint2 *e = &s.lds[((s.sp & s.mask) << s.shift) + s.lane];
-	if (s.sp >= s.depth) {
-		const uint32_t k = s.sp - s.depth;
-		if (k >= s.spillDepth) {
-			atomicOr(err, 1u);
-			return false;
-		}
-		s.spill[(size_t)k * s.gstride + s.glane0 + s.lane] = *e;
-	}
-	*e = make_uint2(ref, asu(t));
-	++s.sp;
-	return true;
-}
-
-DEVI uint2 pop(Stack &s) {
-	--s.sp;
-	uint2 *e = &s.lds[((s.sp & s.mask) << s.shift) + s.lane];
-	const uint2 v = *e;
-	if (s.sp >= s.depth) *e = s.spill[(size_t)(s.sp - s.depth) * s.gstride + s.glane0 + s.lane];
-	return v;
+	return lrhstack::push(s, make_uint2(ref, asu(t)), [err]() { atomicOr(err, 1u); });
 }
 
 // ---- ray tickets ----
@@ -547,37 +521,6 @@ DEVI float groupMin(float x) {
 
 DEVI void waveFence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 
-// Pushes the entries of the lanes with `has` set, lane's own at place `i` of
-// the ray's stack (places sp .. top-1, one lane each): the top `depth`
-// places live in the LDS ring, what they displace and what lies below them
-// goes to the spill array.
-DEVI void drainPush(const Stack &s, bool has, uint32_t i, uint32_t top, uint32_t ref, float t, uint32_t *err) {
-	if (!has) return;
-	const uint2 entry = make_uint2(ref, asu(t));
-	if (i + s.depth < top) {
-		if (i < s.spillDepth) s.spill[(size_t)i * s.gstride + s.glane0 + s.lane] = entry;
-		else atomicOr(err, 1u);
-		return;
-	}
-	uint2 *e = &s.lds[((i & s.mask) << s.shift) + s.lane];
-	int old = (int)i - (int)s.depth;
-	if (old >= (int)s.sp) old -= (int)s.depth;
-	if (old >= 0) {
-		if ((uint32_t)old < s.spillDepth) s.spill[(size_t)old * s.gstride + s.glane0 + s.lane] = *e;
-		else atomicOr(err, 1u);
-	}
-	*e = entry;
-}
-
-// pops the top entry, for all lanes of the group (lane 0 refills the ring)
-DEVI uint2 drainPop(Stack &s, bool leader) {
-	--s.sp;
-	uint2 *e = &s.lds[((s.sp & s.mask) << s.shift) + s.lane];
-	const uint2 v = *e;
-	if (s.sp >= s.depth && leader) *e = s.spill[(size_t)(s.sp - s.depth) * s.gstride + s.glane0 + s.lane];
-	return v;
-}
-
 template <int LAYOUT, bool TWO, bool ANY, bool BATCH>
 DEVI void drain(const LrhTraceParams &P, Stack &st, SceneView &v, LocalRay &r, float wo[3], float wd[3], float mint,
 		float best, float time, float hb1, float hb2, uint32_t hTri, uint32_t hMesh, uint32_t cur, float curT,
@@ -633,6 +576,7 @@ DEVI void drain(const LrhTraceParams &P, Stack &st, SceneView &v, LocalRay &r, f
 	const bool two = TWO && (v.flags & LRH_ITEM_TWO);
 	const bool anyq = ANY && (v.flags & LRH_ITEM_ANY);
 	const bool leader = c == 0;
+	const auto full = [err = P.error]() { atomicOr(err, 1u); };
 	waveFence();
 	for (uint32_t steps = 0; __ballot(rid != kNoRay); ++steps) {
 		if (rid == kNoRay) continue;
@@ -691,10 +635,10 @@ DEVI void drain(const LrhTraceParams &P, Stack &st, SceneView &v, LocalRay &r, f
 			if (anyq) {
 				float t = hit ? a : INFINITY;
 				groupSort<W>(c, t, child);
-				drainPush(st, c < n, st.sp + (n - 1u - c), st.sp + n, child, t, P.error);
+				drainPush(st, c < n, st.sp + (n - 1u - c), st.sp + n, make_uint2(child, asu(t)), full);
 			} else {
 				const uint32_t rank = groupRank<W>(key64(hit ? a : INFINITY, child));
-				drainPush(st, hit, st.sp + (n - 1u - rank), st.sp + n, child, a, P.error);
+				drainPush(st, hit, st.sp + (n - 1u - rank), st.sp + n, make_uint2(child, asu(a)), full);
 			}
 			if (__ballot(st.sp + n > st.depth)) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // spilled entries written by other lanes
 			st.sp += n;
@@ -705,10 +649,6 @@ DEVI void drain(const LrhTraceParams &P, Stack &st, SceneView &v, LocalRay &r, f
 				waveFence();
 				cur = e.x;
 				curT = asf(e.y);
-			}
-			if (steps > kMaxSteps) {
-				if (leader) atomicOr(P.error, 2u);
-				done = true;
 			}
 		}
 		if (!done && cur != LRH_CHILD_EMPTY && (cur & LRH_CHILD_LEAF)) {
@@ -725,7 +665,7 @@ DEVI void drain(const LrhTraceParams &P, Stack &st, SceneView &v, LocalRay &r, f
 				}
 				obj = in.object;
 				inInst = true;
-				drainPush(st, leader, st.sp, st.sp + 1u, LRH_SENTINEL, -INFINITY, P.error);
+				drainPush(st, leader, st.sp, st.sp + 1u, make_uint2(LRH_SENTINEL, asu(-INFINITY)), full);
 				if (st.sp >= st.depth) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
 				++st.sp;
 				waveFence();
@@ -755,6 +695,10 @@ DEVI void drain(const LrhTraceParams &P, Stack &st, SceneView &v, LocalRay &r, f
 					}
 				}
 			}
+		}
+		if ((steps & 255u) == 255u) {  // (neither in a valid tree; an entry without room has set the error)
+			if (leader && steps > kMaxSteps) atomicOr(P.error, 2u);
+			done = done || steps > kMaxSteps || overfull(st);
 		}
 		if (done || (cur == LRH_CHILD_EMPTY && st.sp == 0)) {
 			if (leader) {
