@@ -1284,6 +1284,8 @@ int lrh_scene_download(lrh_scene *s, void *nodes, size_t nodeBytes, void *prims,
 // ---------------------------------------------------------------------------
 namespace {
 
+constexpr unsigned kDefaultBlock = 256;
+
 struct LaunchShape {
 	unsigned block, lds, blocks, refill, spillDepth, leafTris, waveRays;
 	size_t ldsBytes;
@@ -1317,7 +1319,7 @@ LaunchShape chooseShape(lrh_device *dev, unsigned layout, bool two, bool any, bo
 	// 4-wide ones at 1,500,000 579 and 605).
 	L.drain = !two || batch || count <= simds * 1024u;
 	L.waveRays = sparse ? drainRays : 64u;
-	L.block = (o && o->blockSize) ? o->blockSize : sparse && count <= drainRays * simds ? 64 : 256;
+	L.block = (o && o->blockSize) ? o->blockSize : kDefaultBlock;
 	if (L.block != 64 && L.block != 128 && L.block != 256) throw Error(LRH_EINVAL, "blockSize must be 64, 128 or 256");
 	L.lds = (o && o->ldsStack) ? o->ldsStack : 8;
 	if (L.lds < 4 || L.lds > 64 || pow2floor(L.lds) != L.lds)
@@ -1328,8 +1330,13 @@ LaunchShape chooseShape(lrh_device *dev, unsigned layout, bool two, bool any, bo
 	// triangles each, 863 / 875 / 896).  Two-level scenes test whole leaves.
 	L.leafTris = (o && o->leafTris) ? o->leafTris : 2u;
 	if (L.leafTris > 8) throw Error(LRH_EINVAL, "leafTris must be 0..8");
-	L.ldsBytes = (size_t)L.lds * L.block * sizeof(uint2) + extraLds;
-	if (L.ldsBytes > 65536) throw Error(LRH_ERANGE, "LDS stack, node cache and item table exceed 64 KiB per block");
+	// (what is accepted does not depend on the count: a small launch's smaller
+	// blocks are chosen after the check.  A block's ticket pool adds 16 bytes;
+	// a compute unit has 160 KiB)
+	auto ldsOf = [&](unsigned block) { return (size_t)L.lds * block * sizeof(uint2) + extraLds; };
+	if (ldsOf(L.block) > 65536) throw Error(LRH_ERANGE, "LDS stack, node cache and item table exceed 64 KiB per block");
+	if (!(o && o->blockSize) && sparse && count <= drainRays * simds) L.block = 64;
+	L.ldsBytes = ldsOf(L.block);
 	const unsigned pct = (o && o->gridPercent) ? o->gridPercent : 100u;
 	if (pct > 100) throw Error(LRH_EINVAL, "gridPercent must be 0..100");
 	int perCU = (o && o->blocksPerCU) ? (int)o->blocksPerCU : 0;
@@ -1585,9 +1592,10 @@ int lrh_trace_noalloc(lrh_scene *s, const void *rays, void *hits, unsigned int c
 		const bool any = query == LRH_QUERY_ANY;
 		LaunchShape L = chooseShape(dev, s->layout, s->twoLevel, any, false, count, s->maxDepth, 0, nullptr);
 		// the persistent grid is capped at the lanes whose spill stacks fit
-		const size_t blockBytes = (size_t)L.spillDepth * sizeof(uint2) * L.block;
-		const size_t maxBlocks = (LRH_NOALLOC_SCRATCH_BYTES - kScratchCounterBytes) / blockBytes;
-		if (maxBlocks == 0)
+		const size_t laneBytes = (size_t)L.spillDepth * sizeof(uint2), blockBytes = laneBytes * kDefaultBlock;
+		const size_t spillBytes = LRH_NOALLOC_SCRATCH_BYTES - kScratchCounterBytes;
+		const size_t maxBlocks = spillBytes / (laneBytes * L.block);
+		if (spillBytes < blockBytes)  // (whatever the blocks of this count)
 			throw Error(LRH_ERANGE, "tree depth " + std::to_string(s->maxDepth) + " needs " +
 					std::to_string(blockBytes) + " bytes of spill stack per block, beyond the " +
 					std::to_string((unsigned long long)LRH_NOALLOC_SCRATCH_BYTES) + "-byte no-alloc scratch");
