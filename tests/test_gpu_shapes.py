@@ -55,3 +55,24 @@ def test_noalloc_of_small_launches(workload, count, query):
     assert np.array_equal(dev.download(hb, HIT_DTYPE, count), want)
     rb.free()
     hb.free()
+
+
+@pytest.mark.parametrize("count", [30011, 49152])
+def test_noalloc_of_a_small_launch_on_a_capped_grid(gpu_device, count):
+    """The shared start over a tree whose spill stacks leave room for fewer
+    lanes than it asks for: the rest of the rays come through the tickets."""
+    dev = gpu_device
+    sc = dev.scene_bvh(scenes.plain_scene(seed=1, n_random=20000), layout=2)
+    lane_bytes = 8 * (7 * (sc.info()["maxDepth"] + 2) + 4 - 8)
+    assert 128 * 1024 * 1024 // lane_bytes < 8 * count
+    rays = scenes.plain_rays(count, seed=17)
+    init = np.zeros(count, HIT_DTYPE)
+    for query in (0, 1):
+        want = dev.trace_numpy(sc, rays, query=query, hits_init=init)
+        rb, hb = dev.upload(rays), dev.upload(init)
+        D.check(D.lib().lrh_trace_noalloc(sc.h, rb.ptr, hb.ptr, count, query, None))
+        dev.sync()
+        assert np.array_equal(dev.download(hb, HIT_DTYPE, count), want)
+        rb.free()
+        hb.free()
+    sc.close()
