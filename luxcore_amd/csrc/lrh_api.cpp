@@ -1301,7 +1301,7 @@ unsigned pow2floor(unsigned v) {
 // launch shape of one persistent trace: block size, LDS stack depth, grid
 // from the occupancy of the kernel variant, and the spill depth the tree
 // depth needs (3 pushes per level plus the object sentinel)
-LaunchShape chooseShape(lrh_device *dev, unsigned layout, bool two, bool any, bool batch, unsigned count,
+LaunchShape chooseShape(lrh_device *dev, unsigned layout, bool two, bool any, int batch, unsigned count,
 		unsigned maxDepth, size_t extraLds, const lrh_trace_opts *o, bool counting = false) {
 	LaunchShape L;
 	// A small launch starts in the drain, which shares a ray among as many
@@ -1342,7 +1342,7 @@ LaunchShape chooseShape(lrh_device *dev, unsigned layout, bool two, bool any, bo
 	int perCU = (o && o->blocksPerCU) ? (int)o->blocksPerCU : 0;
 	if (!perCU) {
 		const uint64_t key = ((uint64_t)layout << 40) | ((uint64_t)two << 39) | ((uint64_t)any << 38) |
-				((uint64_t)batch << 37) | ((uint64_t)L.drain << 36) | ((uint64_t)L.ldsBytes << 8) | (L.block >> 6);
+				((uint64_t)(batch != 0) << 37) | ((uint64_t)L.drain << 36) | ((uint64_t)(batch == LRH_BATCH_MIXED) << 35) | ((uint64_t)L.ldsBytes << 8) | (L.block >> 6);
 		std::lock_guard<std::mutex> g(dev->mu);
 		auto it = dev->occ.find(key);
 		if (it == dev->occ.end()) {
@@ -1427,7 +1427,7 @@ int traceImpl(lrh_scene *s, const void *rays, void *hits, unsigned int count, un
 		dev->activate();
 		hipStream_t st = stream ? (hipStream_t)stream : dev->stream;
 		const bool any = query == LRH_QUERY_ANY;
-		const LaunchShape L = chooseShape(dev, s->layout, s->twoLevel, any, false, count, s->maxDepth, 0, opts,
+		const LaunchShape L = chooseShape(dev, s->layout, s->twoLevel, any, 0, count, s->maxDepth, 0, opts,
 				statsOut != nullptr);
 		const unsigned nLanes = L.blocks * L.block;
 		lrh_device::Workspace &w = workspace(dev, st, (size_t)nLanes * L.spillDepth * sizeof(uint2));
@@ -1448,7 +1448,7 @@ int traceImpl(lrh_scene *s, const void *rays, void *hits, unsigned int count, un
 		P.error = dev->dError;
 		P.stats = w.stats;
 		if (statsOut) HIPCHK(hipMemsetAsync(w.stats, 0, LRH_TRACE_STATS * sizeof(unsigned long long), st));
-		HIPCHK(lrhLaunchTrace(s->layout, s->twoLevel, any, statsOut != nullptr, false, L.drain, dim3(L.blocks), dim3(L.block),
+		HIPCHK(lrhLaunchTrace(s->layout, s->twoLevel, any, statsOut != nullptr, 0, L.drain, dim3(L.blocks), dim3(L.block),
 				L.ldsBytes, st, P));
 		dev->rays += count;
 		if (statsOut) {
@@ -1464,7 +1464,8 @@ struct BatchTable {
 	std::vector<uint32_t> starts;
 	unsigned layout = 0;
 	bool two = false;
-	bool any = false;  // some items are any-hit queries
+	bool any = false;        // some items are any-hit queries
+	int kind = LRH_BATCH;    // LRH_BATCH_MIXED: and some are not
 	unsigned maxDepth = 0;
 	uint64_t total = 0;
 	// the distinct scenes of the batch with their generation at creation
@@ -1506,6 +1507,7 @@ BatchTable makeTable(lrh_device *dev, const lrh_batch_item *items, unsigned n) {
 		if (j == 0) T.layout = s->layout;
 		else if (s->layout != T.layout) throw Error(LRH_EINVAL, "all scenes of a batch must share the node layout");
 		T.two = T.two || s->twoLevel;
+		if (j > 0 && T.any != (it.query == LRH_QUERY_ANY)) T.kind = LRH_BATCH_MIXED;
 		T.any = T.any || it.query == LRH_QUERY_ANY;
 		T.maxDepth = std::max(T.maxDepth, s->maxDepth);
 		bool seen = false;
@@ -1590,7 +1592,7 @@ int lrh_trace_noalloc(lrh_scene *s, const void *rays, void *hits, unsigned int c
 		dev->activate();
 		hipStream_t st = stream ? (hipStream_t)stream : dev->stream;
 		const bool any = query == LRH_QUERY_ANY;
-		LaunchShape L = chooseShape(dev, s->layout, s->twoLevel, any, false, count, s->maxDepth, 0, nullptr);
+		LaunchShape L = chooseShape(dev, s->layout, s->twoLevel, any, 0, count, s->maxDepth, 0, nullptr);
 		// the persistent grid is capped at the lanes whose spill stacks fit
 		const size_t laneBytes = (size_t)L.spillDepth * sizeof(uint2), blockBytes = laneBytes * kDefaultBlock;
 		const size_t spillBytes = LRH_NOALLOC_SCRATCH_BYTES - kScratchCounterBytes;
@@ -1621,7 +1623,7 @@ int lrh_trace_noalloc(lrh_scene *s, const void *rays, void *hits, unsigned int c
 		P.leafTris = L.leafTris;
 		P.error = dev->dError;
 		P.stats = nullptr;
-		HIPCHK(lrhLaunchTrace(s->layout, s->twoLevel, any, false, false, L.drain, dim3(L.blocks), dim3(L.block), L.ldsBytes, st,
+		HIPCHK(lrhLaunchTrace(s->layout, s->twoLevel, any, false, 0, L.drain, dim3(L.blocks), dim3(L.block), L.ldsBytes, st,
 				P));
 		dev->rays += count;
 	});
@@ -1637,7 +1639,7 @@ int lrh_batch_create(lrh_device *dev, const lrh_batch_item *items, unsigned int 
 		b->dev = dev;
 		b->T = makeTable(dev, items, nItems);
 		const size_t extra = ((nItems + 1) * sizeof(uint32_t) + 15) & ~(size_t)15;
-		b->L = chooseShape(dev, b->T.layout, b->T.two, b->T.any, true, (unsigned)std::max<uint64_t>(b->T.total, 1),
+		b->L = chooseShape(dev, b->T.layout, b->T.two, b->T.any, b->T.kind, (unsigned)std::max<uint64_t>(b->T.total, 1),
 				b->T.maxDepth, extra, opts);
 		const unsigned nLanes = b->L.blocks * b->L.block;
 		b->descs.alloc(dev, b->T.descs.size() * sizeof(LrhBatchDesc));
@@ -1677,7 +1679,7 @@ int lrh_batch_launch(lrh_batch *b, void *stream) {
 		if (b->T.total == 0) return;
 		checkBatchScenes(b);
 		hipStream_t st = stream ? (hipStream_t)stream : b->dev->stream;
-		HIPCHK(lrhLaunchTrace(b->T.layout, b->T.two, b->T.any, false, true, true, dim3(b->L.blocks), dim3(b->L.block),
+		HIPCHK(lrhLaunchTrace(b->T.layout, b->T.two, b->T.any, false, b->T.kind, true, dim3(b->L.blocks), dim3(b->L.block),
 				b->L.ldsBytes, st, b->P));
 		b->dev->rays += b->T.total;
 	});
@@ -1694,7 +1696,7 @@ int lrh_batch_capture(lrh_batch *b, void *stream) {
 		HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
 		hipError_t le = hipSuccess;
 		if (b->T.total)
-			le = lrhLaunchTrace(b->T.layout, b->T.two, b->T.any, false, true, true, dim3(b->L.blocks), dim3(b->L.block),
+			le = lrhLaunchTrace(b->T.layout, b->T.two, b->T.any, false, b->T.kind, true, dim3(b->L.blocks), dim3(b->L.block),
 					b->L.ldsBytes, st, b->P);
 		const hipError_t ce = hipStreamEndCapture(st, &b->graph);
 		HIPCHK(le);
@@ -1742,7 +1744,7 @@ int lrh_trace_batch(lrh_device *dev, const lrh_batch_item *items, unsigned int n
 		BatchTable T = makeTable(dev, items, nItems);
 		if (T.total == 0) return;
 		const size_t extra = ((nItems + 1) * sizeof(uint32_t) + 15) & ~(size_t)15;
-		const LaunchShape L = chooseShape(dev, T.layout, T.two, T.any, true, (unsigned)T.total, T.maxDepth, extra, opts);
+		const LaunchShape L = chooseShape(dev, T.layout, T.two, T.any, T.kind, (unsigned)T.total, T.maxDepth, extra, opts);
 		const unsigned nLanes = L.blocks * L.block;
 		lrh_device::Workspace &w = workspace(dev, st, (size_t)nLanes * L.spillDepth * sizeof(uint2));
 		{
@@ -1780,7 +1782,7 @@ int lrh_trace_batch(lrh_device *dev, const lrh_batch_item *items, unsigned int n
 		P.items = dDesc;
 		P.itemStart = dStart;
 		P.nItems = nItems;
-		HIPCHK(lrhLaunchTrace(T.layout, T.two, T.any, false, true, true, dim3(L.blocks), dim3(L.block), L.ldsBytes, st, P));
+		HIPCHK(lrhLaunchTrace(T.layout, T.two, T.any, false, T.kind, true, dim3(L.blocks), dim3(L.block), L.ldsBytes, st, P));
 		dev->rays += T.total;
 	});
 }

@@ -61,11 +61,16 @@ struct LrhTraceParams {
 	uint32_t nItems;
 };
 
+/* `batch` of a launch: its items are all of one query kind (`any` says which),
+ * or of both, each ray then going by its item's flag */
+#define LRH_BATCH 1
+#define LRH_BATCH_MIXED 2
+
 hipError_t lrhLaunchReset(uint32_t *p, uint32_t n, hipStream_t s);
-hipError_t lrhOccupancy(int layout, bool two, bool any, bool batch, bool drain, int block, size_t lds,
+hipError_t lrhOccupancy(int layout, bool two, bool any, int batch, bool drain, int block, size_t lds,
 		int *blocksPerCU);
 /* `drain` chooses between the two builds of a two-level trace (count, batch: ignored) */
-hipError_t lrhLaunchTrace(int layout, bool two, bool any, bool count, bool batch, bool drain, dim3 grid, dim3 block,
+hipError_t lrhLaunchTrace(int layout, bool two, bool any, bool count, int batch, bool drain, dim3 grid, dim3 block,
 		size_t lds, hipStream_t s, const LrhTraceParams &P);
 
 #endif

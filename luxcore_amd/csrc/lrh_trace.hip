@@ -522,7 +522,7 @@ DEVI float groupMin(float x) {
 
 DEVI void waveFence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 
-template <int LAYOUT, bool TWO, bool ANY, bool BATCH>
+template <int LAYOUT, bool TWO, bool ANY, int BATCH>
 DEVI void drain(const LrhTraceParams &P, Stack &st, SceneView &v, LocalRay &r, float wo[3], float wd[3], float mint,
 		float best, float time, float hb1, float hb2, uint32_t hTri, uint32_t hMesh, uint32_t cur, float curT,
 		uint32_t obj, bool inInst, uint32_t rid) {
@@ -575,7 +575,7 @@ DEVI void drain(const LrhTraceParams &P, Stack &st, SceneView &v, LocalRay &r, f
 	const uint32_t taken = shu(rid);  // (every exchange with all lanes active)
 	rid = group < nLive ? taken : kNoRay;
 	const bool two = TWO && (v.flags & LRH_ITEM_TWO);
-	const bool anyq = ANY && (v.flags & LRH_ITEM_ANY);
+	const bool anyq = ANY && (BATCH == LRH_BATCH || (v.flags & LRH_ITEM_ANY));
 	const bool leader = c == 0;
 	const auto full = [err = P.error]() { atomicOr(err, 1u); };
 	waveFence();
@@ -715,7 +715,7 @@ DEVI void drain(const LrhTraceParams &P, Stack &st, SceneView &v, LocalRay &r, f
 	}
 }
 
-template <int LAYOUT, bool TWO, bool ANY, bool COUNT, bool BATCH, bool DRAIN>
+template <int LAYOUT, bool TWO, bool ANY, bool COUNT, int BATCH, bool DRAIN>
 __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 	extern __shared__ uint2 ldsStack[];  // [ldsDepth][blockDim] stack; batched: then item starts
 	const uint32_t lane = __lane_id();
@@ -926,7 +926,7 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 					// network's.  In a batch of both kinds each ray takes its own sort: 899 us for
 					// 3.9M rays, where one network whose comparators also compare a closest ray's
 					// references takes 944 (and the network alone, with no order of ties, 889).
-					if (ANY && (!BATCH || (v.flags & LRH_ITEM_ANY))) sort8(t8, c8);
+					if (ANY && (BATCH != LRH_BATCH_MIXED || (v.flags & LRH_ITEM_ANY))) sort8(t8, c8);
 					else sort8Closest(t8, c8);
 					bool ok = true;
 					// sorted: the lanes that push entry k also push k-1..1; a
@@ -949,7 +949,7 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 					testNodeQ(reinterpret_cast<const lrh_node4q *>(v.nodes), cur, r, mint, best, t4, c4);
 				else
 					testNodeF(reinterpret_cast<const lrh_node4f *>(v.nodes), cur, r, mint, best, t4, c4);
-				if (ANY && (!BATCH || (v.flags & LRH_ITEM_ANY))) sort4(t4, c4);
+				if (ANY && (BATCH != LRH_BATCH_MIXED || (v.flags & LRH_ITEM_ANY))) sort4(t4, c4);
 				else sort4Closest(t4, c4);
 				bool ok = true;
 				if (t4[3] != INFINITY) ok = ok && push(st, c4[3], t4[3], P.error);
@@ -974,7 +974,7 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 		}
 		if (atLeaf) {
 			const bool two = TWO && (v.flags & LRH_ITEM_TWO);
-			const bool anyq = ANY && (v.flags & LRH_ITEM_ANY);
+			const bool anyq = ANY && (BATCH == LRH_BATCH || (v.flags & LRH_ITEM_ANY));
 			const uint32_t start = cur & LRH_LEAF_START_MASK;
 			uint32_t cnt = ((cur >> LRH_LEAF_START_BITS) & 7u) + 1u;
 			cur = LRH_CHILD_EMPTY;
@@ -1082,14 +1082,14 @@ __device__ __forceinline__ void traceBody(const LrhTraceParams &P) {
 // Single-level traces are built for 7 waves per SIMD (at most 72 VGPRs),
 // batched ones over 8-wide nodes (per-lane item view) for 5: at 6 the loop
 // spills (a batch of 3.9M rays 1,032 us, at 5 983 us).
-template <int LAYOUT, bool ANY, bool COUNT, bool BATCH>
+template <int LAYOUT, bool ANY, bool COUNT, int BATCH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void lrh_trace_kernel(LrhTraceParams P) {
 	traceBody<LAYOUT, false, ANY, COUNT, BATCH, !COUNT>(P);
 }
 
-template <bool ANY>
+template <bool ANY, int BATCH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void lrh_trace8b_kernel(LrhTraceParams P) {
-	traceBody<2, false, ANY, false, true, true>(P);
+	traceBody<2, false, ANY, false, BATCH, true>(P);
 }
 
 // Two-level traces inline the motion sample, which reads its motion record
@@ -1099,12 +1099,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void l
 // VGPRs; at 6 it spills 10), batched 8-wide ones for 4 (at 5 it spills 37).
 // With the drain, which holds a second motion sample, the loop spills; so
 // a launch that the drain is a small part of goes without.
-template <int LAYOUT, bool ANY, bool COUNT, bool BATCH>
+template <int LAYOUT, bool ANY, bool COUNT, int BATCH>
 __global__ __launch_bounds__(256) void lrh_trace2_kernel(LrhTraceParams P) {
 	traceBody<LAYOUT, true, ANY, COUNT, BATCH, false>(P);
 }
 
-template <bool ANY, bool BATCH>
+template <bool ANY, int BATCH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BATCH ? 4 : 5))) void lrh_trace28_kernel(
 		LrhTraceParams P) {
 	traceBody<2, true, ANY, false, BATCH, false>(P);
@@ -1112,12 +1112,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BATCH ? 4 :
 
 template <bool ANY>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void lrh_trace2q_kernel(LrhTraceParams P) {
-	traceBody<0, true, ANY, false, false, false>(P);
+	traceBody<0, true, ANY, false, 0, false>(P);
 }
 
 template <int LAYOUT, bool ANY>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void lrh_trace2_drain_kernel(LrhTraceParams P) {
-	traceBody<LAYOUT, true, ANY, false, false, true>(P);
+	traceBody<LAYOUT, true, ANY, false, 0, true>(P);
 }
 
 __global__ void lrh_reset_kernel(uint32_t *p, uint32_t n) {
@@ -1130,25 +1130,28 @@ __global__ void lrh_reset_kernel(uint32_t *p, uint32_t n) {
 // ---------------------------------------------------------------------------
 typedef void (*KernelFn)(LrhTraceParams);
 
-template <int L, bool A>
-static const void *kernelOf(bool two, bool count, bool batch, bool drain) {
-	if (batch) {
-		if (L == 2)
-			return two ? (const void *)&lrh_trace28_kernel<A, true> : (const void *)&lrh_trace8b_kernel<A>;
-		return two ? (const void *)&lrh_trace2_kernel<L == 2 ? 0 : L, A, false, true>
-				: (const void *)&lrh_trace_kernel<L == 2 ? 0 : L, A, false, true>;
-	}
-	if (!two) return count ? (const void *)&lrh_trace_kernel<L, A, true, false> : (const void *)&lrh_trace_kernel<L, A, false, false>;
-	if (count) return (const void *)&lrh_trace2_kernel<L, A, true, false>;
-	if (drain) return (const void *)&lrh_trace2_drain_kernel<L, A>;
-	if (L == 0) return (const void *)&lrh_trace2q_kernel<A>;
-	if (L == 2) return (const void *)&lrh_trace28_kernel<A, false>;
-	return (const void *)&lrh_trace2_kernel<1, A, false, false>;
+template <int L, bool A, int B>
+static const void *batchKernelOf(bool two) {
+	if (L == 2)
+		return two ? (const void *)&lrh_trace28_kernel<A, B> : (const void *)&lrh_trace8b_kernel<A, B>;
+	return two ? (const void *)&lrh_trace2_kernel<L == 2 ? 0 : L, A, false, B>
+			: (const void *)&lrh_trace_kernel<L == 2 ? 0 : L, A, false, B>;
 }
 
-// `any` of a batch: some of its items are any-hit queries.  The counting
-// variants are not offered for batches and have no drain.
-static const void *kernelPtr(int layout, bool two, bool any, bool count, bool batch, bool drain) {
+template <int L, bool A>
+static const void *kernelOf(bool two, bool count, int batch, bool drain) {
+	if (batch == LRH_BATCH_MIXED) return batchKernelOf<L, true, LRH_BATCH_MIXED>(two);
+	if (batch) return batchKernelOf<L, A, LRH_BATCH>(two);
+	if (!two) return count ? (const void *)&lrh_trace_kernel<L, A, true, 0> : (const void *)&lrh_trace_kernel<L, A, false, 0>;
+	if (count) return (const void *)&lrh_trace2_kernel<L, A, true, 0>;
+	if (drain) return (const void *)&lrh_trace2_drain_kernel<L, A>;
+	if (L == 0) return (const void *)&lrh_trace2q_kernel<A>;
+	if (L == 2) return (const void *)&lrh_trace28_kernel<A, 0>;
+	return (const void *)&lrh_trace2_kernel<1, A, false, 0>;
+}
+
+// The counting variants are not offered for batches and have no drain.
+static const void *kernelPtr(int layout, bool two, bool any, bool count, int batch, bool drain) {
 	switch (layout * 2 + (any ? 1 : 0)) {
 	case 0: return kernelOf<0, false>(two, count, batch, drain);
 	case 1: return kernelOf<0, true>(two, count, batch, drain);
@@ -1165,14 +1168,14 @@ hipError_t lrhLaunchReset(uint32_t *p, uint32_t n, hipStream_t s) {
 	return hipGetLastError();
 }
 
-hipError_t lrhOccupancy(int layout, bool two, bool any, bool batch, bool drain, int block, size_t lds,
+hipError_t lrhOccupancy(int layout, bool two, bool any, int batch, bool drain, int block, size_t lds,
 		int *blocksPerCU) {
 	const void *k = kernelPtr(layout, two, any, false, batch, drain);
 	if (!k) return hipErrorInvalidDeviceFunction;
 	return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocksPerCU, k, block, lds);
 }
 
-hipError_t lrhLaunchTrace(int layout, bool two, bool any, bool count, bool batch, bool drain, dim3 grid, dim3 block,
+hipError_t lrhLaunchTrace(int layout, bool two, bool any, bool count, int batch, bool drain, dim3 grid, dim3 block,
 		size_t lds, hipStream_t s, const LrhTraceParams &P) {
 	void *args[] = {(void *)&P};
 	const void *k = kernelPtr(layout, two, any, count, batch, drain);
