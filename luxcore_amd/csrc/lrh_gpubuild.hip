@@ -483,9 +483,12 @@ __device__ __forceinline__ PlocState plocRound(const PlocState *st, uint32_t r) 
 	return s;
 }
 
-// plocNearestAt by L neighbouring lanes, each with every L-th place: of equal
-// areas the lowest place wins, which is the order of the pairs (a pair with a
-// lower place comes first by its lower end or, above i, by its upper)
+// The nearest neighbour of cluster i within kPlocRadius places: the smallest
+// merged area, of equal areas the first pair by (lower, upper) place, so the
+// first of all pairs is mutual and every round merges.  By L neighbouring
+// lanes, each with every L-th place: of equal areas the lowest place wins, which
+// is the order of the pairs (a pair with a lower place comes first by its lower
+// end or, above i, by its upper)
 template <uint32_t L, class BoxAt>
 __device__ __forceinline__ uint32_t plocNearestLanes(const BoxAt &box, uint32_t nc, uint32_t i, uint32_t sub) {
 	float best = INFINITY;
@@ -794,10 +797,11 @@ struct Level {
 	uint32_t nf, base;
 };
 
-// 5a. children of each frontier node (expandNode's, from the nodes' keys: the
-// areas of the candidates stay in registers and each opened child costs one
-// read of its children and one of their keys), and how many become inner
-// nodes, summed over the block
+// 5a. children of each frontier node (its two, then the largest that is not a
+// leaf opened until there are W; from the nodes' keys, so the areas of the
+// candidates stay in registers and each opened child costs one read of its
+// children and one of their keys), and how many become inner nodes, summed
+// over the block
 template <int W>
 __global__ __launch_bounds__(256) void k_expand(const uint32_t *frontier, const Level *lv, uint32_t l, uint32_t nInner,
 		const uint32_t *left, const uint32_t *right, const float *key, uint32_t *kids, uint32_t *prefix, uint32_t *sums,
@@ -890,8 +894,8 @@ __global__ __launch_bounds__(1024) void k_levelScan(uint32_t *sums, Level *lv, u
 	}
 }
 
-// 5c. the level's wide nodes, W lanes each (emitNode's record); inner children
-// get slots after the level
+// 5c. the level's wide nodes, W lanes each; inner children get slots after
+// the level
 template <int W, class Node>
 __global__ __launch_bounds__(256) void k_emit(const Level *lv, uint32_t l, const uint32_t *kids, const uint32_t *prefix,
 		const uint32_t *sums, const uint32_t *first, const uint32_t *last, const float *key, const GBox *leafBox,

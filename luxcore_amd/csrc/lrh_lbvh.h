@@ -9,11 +9,13 @@
  *   3. a node of the binary radix tree over the sorted codes (Karras,
  *      "Maximizing Parallelism in the Construction of BVHs, Octrees, and k-d
  *      Trees", HPG 2012), equal codes ordered by position; or the nearest
- *      neighbour and partner of a cluster in a PLOC round;
- *   4. a node's surface-area cost and leaf decision, the expansion of a
- *      binary node into up to four or eight children (largest area first)
- *      and the wide record it becomes;
+ *      neighbour's area and partner of a cluster in a PLOC round;
+ *   4. a node's surface-area cost and leaf decision;
  *   5. the triangle record, bit for bit the host builder's.
+ * What the kernels do with several lanes (a cluster's nearest neighbour, the
+ * expansion of a binary node into up to four or eight children and the wide
+ * record it becomes) the emulation has in its sequential form; that both
+ * give the same bytes is tested.
  * Every search loop is bounded: keys that are not in order make the range
  * search fail (radixNode returns false) instead of looping.
  */
@@ -38,7 +40,6 @@ constexpr uint32_t kNone = 0xffffffffu;
 enum : uint32_t {
 	kErrUnsorted = 1u,   // sorted codes out of order
 	kErrRange = 2u,      // a radix-tree node found no range (keys not in order around it)
-	kErrClimb = 4u,      // a radix-tree node deeper than any valid tree (or not below the root)
 	kErrExpand = 8u,     // a frontier entry that is not an internal node (or more nodes than the tree has)
 	kErrCluster = 16u,   // a clustering round without a consistent merge count
 	kErrIndex = 32u,     // a triangle's vertex index outside its mesh
@@ -87,13 +88,6 @@ LRH_DN inline GBox boxOf(const float p[3][3]) {
 	}
 	return b;
 }
-LRH_DN inline GBox primBox(const float *verts, const uint32_t *tris, const uint32_t *tbase, const uint32_t *vbase,
-		uint32_t nMeshes, uint32_t i) {
-	float p[3][3];
-	loadTri(verts, tris, vbase, meshOf(tbase, nMeshes, i), i, p);
-	return boxOf(p);
-}
-
 LRH_DN inline uint64_t spread21(uint32_t v) {
 	uint64_t x = v & 0x1fffffu;
 	x = (x | (x << 32)) & 0x1f00000000ffffull;
@@ -181,10 +175,6 @@ LRH_DN inline bool radixNode(const uint64_t *keys, int64_t n, int64_t i, uint32_
 	return true;
 }
 
-LRH_DN inline uint32_t countOf(uint32_t c, const uint32_t *first, const uint32_t *last) {
-	return (c & kLeafBit) ? 1u : last[c] - first[c] + 1u;
-}
-
 LRH_DN inline float areaOf(const GBox &b) {
 	const float dx = b.hi[0] - b.lo[0], dy = b.hi[1] - b.lo[1], dz = b.hi[2] - b.lo[2];
 	if (!(dx >= 0.f)) return 0.f;
@@ -202,81 +192,10 @@ LRH_DN inline float nodeCost(float A, float cl, float cr, uint32_t N, uint32_t m
 	return leaf ? asLeaf : split;
 }
 
-// a child that becomes a leaf of the wide tree: a triangle, or a node the
-// cost chose as a leaf
-LRH_DN inline bool leafChild(uint32_t c, const uint32_t *leafOK) { return (c & kLeafBit) || leafOK[c]; }
-
-// (steps 4a and 4b are the sequential form; the device writes the same nodes
-// from the nodes' areas and with a lane per child)
-// 4a. the children of internal node b (Morton order): its two, then the
-// largest-area child that is not a leaf split until there are `width` (4 or
-// 8); returns how many of them become inner nodes
-constexpr int kMaxWide = 8;
-LRH_DN inline uint32_t expandNode(uint32_t b, const uint32_t *left, const uint32_t *right, const uint32_t *leafOK,
-		const GBox *nodeBox, int width, uint32_t kids[kMaxWide]) {
-	uint32_t ch[kMaxWide] = {left[b], right[b], kNone, kNone, kNone, kNone, kNone, kNone};
-	int nch = 2;
-	while (nch < width) {
-		int pick = -1;
-		float best = -1.f;
-		for (int k = 0; k < nch; ++k) {
-			if (leafChild(ch[k], leafOK)) continue;
-			const float a = areaOf(nodeBox[ch[k]]);
-			if (a > best) {
-				best = a;
-				pick = k;
-			}
-		}
-		if (pick < 0) break;
-		const uint32_t c = ch[pick];
-		for (int k = nch; k > pick + 1; --k) ch[k] = ch[k - 1];
-		ch[pick] = left[c];
-		ch[pick + 1] = right[c];
-		++nch;
-	}
-	uint32_t inner = 0;
-	for (int k = 0; k < kMaxWide; ++k) {
-		kids[k] = ch[k];
-		if (ch[k] != kNone && !leafChild(ch[k], leafOK)) ++inner;
-	}
-	return inner;
-}
+constexpr int kMaxWide = 8;  // the widest node's children
 
 LRH_DN inline uint32_t leafRef(uint32_t start, uint32_t count) {
 	return LRH_CHILD_LEAF | ((count - 1u) << LRH_LEAF_START_BITS) | start;
-}
-
-// 4b. the wide node of a frontier entry: leaf children reference their key
-// range, inner children the slots innerOff, innerOff+1, ... after the level
-// (their binary ids go to next[slot])
-LRH_DN inline void emitNode(const uint32_t kids[kMaxWide], uint32_t innerOff, const uint32_t *first,
-		const uint32_t *last, const uint32_t *leafOK, const GBox *leafBox, const GBox *nodeBox, uint32_t childBase,
-		uint32_t layout, void *nodes, uint32_t nodeIndex, uint32_t *next) {
-	GBox cb[kMaxWide];
-	uint32_t ref[kMaxWide];
-	for (int k = 0; k < kMaxWide; ++k) ref[k] = LRH_CHILD_EMPTY;
-	int n = 0;
-	uint32_t slot = innerOff;
-	for (int k = 0; k < kMaxWide; ++k) {
-		const uint32_t c = kids[k];
-		if (c == kNone) continue;
-		cb[n] = (c & kLeafBit) ? leafBox[c & ~kLeafBit] : nodeBox[c];
-		if (leafChild(c, leafOK)) {
-			const uint32_t start = (c & kLeafBit) ? (c & ~kLeafBit) : first[c];
-			ref[n] = leafRef(start, countOf(c, first, last));
-		} else {
-			ref[n] = childBase + slot;
-			next[slot] = c;
-			++slot;
-		}
-		++n;
-	}
-	if (layout == 0)
-		lrhdev::quantizeNode(cb, n, ref, reinterpret_cast<lrh_node4q *>(nodes) + nodeIndex);
-	else if (layout == 2)
-		lrhdev::quantizeNode8(cb, n, ref, reinterpret_cast<lrh_node8q *>(nodes) + nodeIndex);
-	else
-		lrhdev::floatNode(cb, n, ref, reinterpret_cast<lrh_node4f *>(nodes) + nodeIndex);
 }
 
 // 5. triangle record of global triangle i, as the host builder writes it
@@ -322,39 +241,6 @@ LRH_DN inline GBox unionBox(const GBox &a, const GBox &b) {
 LRH_DN inline float mergedArea(const GBox &a, const GBox &b) {
 	const float x = areaOf(unionBox(a, b));
 	return x == x ? x : INFINITY;
-}
-
-// nearest neighbour of cluster i among places [i - r, i + r]: the smallest
-// merged area, equal areas by the pair's (lower, upper) place, so the pair
-// with the smallest such key of all is mutual and every round merges
-// (box(j) returns cluster j's box: the array itself, or a tile of it staged
-// in LDS; the arithmetic is the same either way)
-template <class BoxAt>
-LRH_DN inline uint32_t plocNearestAt(const BoxAt &box, uint32_t nc, uint32_t i, uint32_t r) {
-	const uint32_t lo = i > r ? i - r : 0u;
-	const uint32_t hi = (nc - 1u - i > r) ? i + r : nc - 1u;
-	float best = INFINITY;
-	uint32_t arg = i;
-	const GBox ci = box(i);
-	for (uint32_t j = lo; j <= hi; ++j) {
-		if (j == i) continue;
-		const float a = mergedArea(ci, box(j));
-		bool better = arg == i || a < best;
-		if (arg != i && a == best) {
-			const uint32_t p0 = i < j ? i : j, q0 = i < j ? j : i;
-			const uint32_t p1 = i < arg ? i : arg, q1 = i < arg ? arg : i;
-			better = p0 < p1 || (p0 == p1 && q0 < q1);
-		}
-		if (better) {
-			best = a;
-			arg = j;
-		}
-	}
-	return arg;
-}
-
-LRH_DN inline uint32_t plocNearest(const GBox *c, uint32_t nc, uint32_t i, uint32_t r) {
-	return plocNearestAt([c](uint32_t j) -> const GBox & { return c[j]; }, nc, i, r);
 }
 
 // cluster i's partner this round (kNone: none): its nearest neighbour when

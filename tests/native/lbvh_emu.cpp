@@ -34,6 +34,116 @@ using namespace lrhlbvh;
 
 namespace {
 
+constexpr uint32_t kErrClimb = 4u;  // a radix-tree node deeper than any valid tree (or not below the root)
+
+// ---- the sequential form of what the kernels do with several lanes ----
+
+GBox primBox(const float *verts, const uint32_t *tris, const uint32_t *tbase, const uint32_t *vbase,
+		uint32_t nMeshes, uint32_t i) {
+	float p[3][3];
+	loadTri(verts, tris, vbase, meshOf(tbase, nMeshes, i), i, p);
+	return boxOf(p);
+}
+
+// nearest neighbour of cluster i among places [i - r, i + r]: the smallest
+// merged area, equal areas by the pair's (lower, upper) place, so the pair
+// with the smallest such key of all is mutual and every round merges
+uint32_t plocNearest(const GBox *c, uint32_t nc, uint32_t i, uint32_t r) {
+	const uint32_t lo = i > r ? i - r : 0u;
+	const uint32_t hi = (nc - 1u - i > r) ? i + r : nc - 1u;
+	float best = INFINITY;
+	uint32_t arg = i;
+	for (uint32_t j = lo; j <= hi; ++j) {
+		if (j == i) continue;
+		const float a = mergedArea(c[i], c[j]);
+		bool better = arg == i || a < best;
+		if (arg != i && a == best) {
+			const uint32_t p0 = i < j ? i : j, q0 = i < j ? j : i;
+			const uint32_t p1 = i < arg ? i : arg, q1 = i < arg ? arg : i;
+			better = p0 < p1 || (p0 == p1 && q0 < q1);
+		}
+		if (better) {
+			best = a;
+			arg = j;
+		}
+	}
+	return arg;
+}
+
+uint32_t countOf(uint32_t c, const uint32_t *first, const uint32_t *last) {
+	return (c & kLeafBit) ? 1u : last[c] - first[c] + 1u;
+}
+
+// a child that becomes a leaf of the wide tree: a triangle, or a node the
+// cost chose as a leaf
+bool leafChild(uint32_t c, const uint32_t *leafOK) { return (c & kLeafBit) || leafOK[c]; }
+
+// 4a. the children of internal node b (Morton order): its two, then the
+// largest-area child that is not a leaf split until there are `width` (4 or
+// 8); returns how many of them become inner nodes
+uint32_t expandNode(uint32_t b, const uint32_t *left, const uint32_t *right, const uint32_t *leafOK,
+		const GBox *nodeBox, int width, uint32_t kids[kMaxWide]) {
+	uint32_t ch[kMaxWide] = {left[b], right[b], kNone, kNone, kNone, kNone, kNone, kNone};
+	int nch = 2;
+	while (nch < width) {
+		int pick = -1;
+		float best = -1.f;
+		for (int k = 0; k < nch; ++k) {
+			if (leafChild(ch[k], leafOK)) continue;
+			const float a = areaOf(nodeBox[ch[k]]);
+			if (a > best) {
+				best = a;
+				pick = k;
+			}
+		}
+		if (pick < 0) break;
+		const uint32_t c = ch[pick];
+		for (int k = nch; k > pick + 1; --k) ch[k] = ch[k - 1];
+		ch[pick] = left[c];
+		ch[pick + 1] = right[c];
+		++nch;
+	}
+	uint32_t inner = 0;
+	for (int k = 0; k < kMaxWide; ++k) {
+		kids[k] = ch[k];
+		if (ch[k] != kNone && !leafChild(ch[k], leafOK)) ++inner;
+	}
+	return inner;
+}
+
+// 4b. the wide node of a frontier entry: leaf children reference their key
+// range, inner children the slots innerOff, innerOff+1, ... after the level
+// (their binary ids go to next[slot])
+void emitNode(const uint32_t kids[kMaxWide], uint32_t innerOff, const uint32_t *first,
+		const uint32_t *last, const uint32_t *leafOK, const GBox *leafBox, const GBox *nodeBox, uint32_t childBase,
+		uint32_t layout, void *nodes, uint32_t nodeIndex, uint32_t *next) {
+	GBox cb[kMaxWide];
+	uint32_t ref[kMaxWide];
+	for (int k = 0; k < kMaxWide; ++k) ref[k] = LRH_CHILD_EMPTY;
+	int n = 0;
+	uint32_t slot = innerOff;
+	for (int k = 0; k < kMaxWide; ++k) {
+		const uint32_t c = kids[k];
+		if (c == kNone) continue;
+		cb[n] = (c & kLeafBit) ? leafBox[c & ~kLeafBit] : nodeBox[c];
+		if (leafChild(c, leafOK)) {
+			const uint32_t start = (c & kLeafBit) ? (c & ~kLeafBit) : first[c];
+			ref[n] = leafRef(start, countOf(c, first, last));
+		} else {
+			ref[n] = childBase + slot;
+			next[slot] = c;
+			++slot;
+		}
+		++n;
+	}
+	if (layout == 0)
+		lrhdev::quantizeNode(cb, n, ref, reinterpret_cast<lrh_node4q *>(nodes) + nodeIndex);
+	else if (layout == 2)
+		lrhdev::quantizeNode8(cb, n, ref, reinterpret_cast<lrh_node8q *>(nodes) + nodeIndex);
+	else
+		lrhdev::floatNode(cb, n, ref, reinterpret_cast<lrh_node4f *>(nodes) + nodeIndex);
+}
+
 template <class T>
 void put(const std::string &path, const std::vector<T> &v) {
 	std::ofstream f(path, std::ios::binary);
