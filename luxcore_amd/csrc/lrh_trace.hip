@@ -9,12 +9,13 @@
  *
  * Traversal is ordered (children sorted by entry distance) over 4-wide or
  * 8-wide nodes, with a per-lane stack whose top `ldsDepth` entries live in LDS and
- * deeper entries spill to a global scratch array; popped entries whose entry
- * distance is not below the current hit are dropped without a fetch.  The
- * reference walks a skip-pointer array in memory order instead
- * (bvh.cl:136-217, src/luxrays/accelerators/bvhaccel.cpp:184-257); both visit
- * a superset of the boxes containing the closest hit, so the closest hit is
- * the same up to ties at equal t.
+ * deeper entries spill to a global scratch array (lrh_stack.h); popped entries
+ * whose entry distance is above the current hit's, widened, are dropped
+ * without a fetch.  The reference walks a skip-pointer array in memory order
+ * instead (bvh.cl:136-217, src/luxrays/accelerators/bvhaccel.cpp:184-257); both
+ * visit a superset of the boxes containing the closest hit, so the closest hit
+ * is the same up to ties at equal t.  Which of two hits at equal t a ray
+ * reports is fixed by the scene and the ray: every kernel here visits alike.
  *
  * The triangle test is Triangle::Intersect
  * (include/luxrays/core/geometry/triangle.h:55-89) with every operation
